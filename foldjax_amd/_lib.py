@@ -26,7 +26,7 @@ FJX_ERR_WORKSPACE = 3
 FJX_ERR_HIP = 4
 
 ABI_VERSION = 6
-NOALLOC_SCRATCH_BYTES = 256 << 20
+NOALLOC_SCRATCH_BYTES = 3 * 591 * 640 * 256
 
 _vp = ctypes.c_void_p
 _i64 = ctypes.c_int64

@@ -176,12 +176,18 @@ dim3 grid_for(int64_t total) {
 }
 
 // --------------------------------------------------------------- layouts
+// a, b and o of the tri-mul have rows `pitch` elements apart: N rounded up to
+// 64, so that at any N every row is whole cache lines (the LDS-DMA
+// contraction, 16-byte stores and loads), or N itself (tight) where a fixed
+// scratch does not hold that.
 struct TriMulWs {
   size_t a, b, o, total;
+  int64_t pitch;
 };
-TriMulWs trimul_ws(int64_t batch, int64_t n, int32_t dtype) {
-  const size_t per = align_up((size_t)batch * n * n * 128 * esize(dtype));
+TriMulWs trimul_ws(int64_t batch, int64_t n, int32_t dtype, bool tight = false) {
   TriMulWs w;
+  w.pitch = tight ? n : round64(n);
+  const size_t per = align_up((size_t)batch * n * w.pitch * 128 * esize(dtype));
   w.a = 0;
   w.b = per;
   w.o = 2 * per;
@@ -227,8 +233,8 @@ T* at(void* base, size_t off) {
 
 // ----------------------------------------------------------- tri-mul body
 template <typename T>
-int trimul_run(const fjx_trimul_args* a, hipStream_t st) {
-  const TriMulWs ws = trimul_ws(a->batch, a->n, a->dtype);
+int trimul_run(const fjx_trimul_args* a, bool tight, hipStream_t st) {
+  const TriMulWs ws = trimul_ws(a->batch, a->n, a->dtype, tight);
   T* abuf = at<T>(a->workspace, ws.a);
   T* bbuf = at<T>(a->workspace, ws.b);
   T* obuf = at<T>(a->workspace, ws.o);
@@ -245,6 +251,7 @@ int trimul_run(const fjx_trimul_args* a, hipStream_t st) {
   pp.a_cm = abuf;
   pp.b_cm = bbuf;
   pp.n = a->n;
+  pp.pitch = ws.pitch;
   pp.eps = a->eps;
   pp.transpose = a->direction == FJX_INCOMING;
   pp.cw = cw;
@@ -254,15 +261,15 @@ int trimul_run(const fjx_trimul_args* a, hipStream_t st) {
   bool o_blocked = false;  // the LDS-DMA contraction writes o tile-blocked for the epilogue
   rc = timed(K_TRIMUL_CONTRACT, st, "trimul_contract", [&] {
     if constexpr (std::is_same<T, bf16>::value) {
-      o_blocked = launch_contract(abuf, bbuf, obuf, a->n, a->batch * 128, st, true);
+      o_blocked = launch_contract(abuf, bbuf, obuf, a->n, ws.pitch, a->batch * 128, st, true);
     } else {
       GemmParams<T, T> cp = {};
       cp.a = abuf;
       cp.b = bbuf;
       cp.c = obuf;
-      cp.m = cp.n = cp.k = a->n;
-      cp.lda = cp.ldb = cp.ldc = a->n;
-      cp.sa = cp.sb = cp.sc = a->n * a->n;
+      cp.m = cp.n = a->n;
+      cp.k = cp.lda = cp.ldb = cp.ldc = ws.pitch;  // zeros past n
+      cp.sa = cp.sb = cp.sc = a->n * ws.pitch;
       cp.batches = a->batch * 128;
       launch_gemm<T, T>(cp, st);
     }
@@ -271,6 +278,7 @@ int trimul_run(const fjx_trimul_args* a, hipStream_t st) {
 
   TriMulEpilogueParams<T> ep = {};
   ep.o = obuf;
+  ep.pitch = ws.pitch;
   ep.o_blocked = o_blocked;
   ep.x = static_cast<const T*>(a->x);
   ep.ln_in_w = pp.ln_w;
@@ -573,7 +581,7 @@ int trimul_generic_run(const fjx_trimul_args* a, hipStream_t st) {
 
   rc = timed(K_TRIMUL_CONTRACT, st, "trimul_contract", [&] {
     if constexpr (std::is_same<T, bf16>::value) {
-      launch_contract(acm, bcm, ocm, n, B * ch, st);
+      launch_contract(acm, bcm, ocm, n, n, B * ch, st);
     } else {
       GemmParams<T, T> cp = {};
       cp.a = acm;
@@ -995,10 +1003,10 @@ int trimul_check(const fjx_trimul_args* a, const char* fn) {
   return FJX_OK;
 }
 
-int trimul_dispatch(const fjx_trimul_args* a, hipStream_t st) {
+int trimul_dispatch(const fjx_trimul_args* a, bool tight, hipStream_t st) {
   if (!fused_trimul(a->c_z, a->c_h))
     return a->dtype == FJX_DTYPE_BF16 ? trimul_generic_run<bf16>(a, st) : trimul_generic_run<float>(a, st);
-  return a->dtype == FJX_DTYPE_BF16 ? trimul_run<bf16>(a, st) : trimul_run<float>(a, st);
+  return a->dtype == FJX_DTYPE_BF16 ? trimul_run<bf16>(a, tight, st) : trimul_run<float>(a, tight, st);
 }
 
 }  // namespace
@@ -1021,7 +1029,7 @@ int fjx_trimul_fwd(const fjx_trimul_args* a, hipStream_t st) {
   if (!a->workspace || a->workspace_bytes < need)
     return fail(FJX_ERR_WORKSPACE, "fjx_trimul_fwd: workspace of %zu bytes needed, %zu given", need,
                 a->workspace_bytes);
-  return trimul_dispatch(a, st);
+  return trimul_dispatch(a, false, st);
 }
 
 
@@ -1272,17 +1280,22 @@ __attribute__((visibility("hidden"))) int trimul_fwd_on_scratch(const fjx_trimul
                                                                void* scratch, size_t scratch_bytes, const char* fn) {
   g_err.clear();
   if (int rc = trimul_check(a, fn)) return rc;
-  const size_t need = fjx_trimul_workspace_size(a->batch, a->n, a->c_z, a->c_h, a->dtype);
-  if (need > scratch_bytes)
+  // refused by the size of the tight layout (rows of exactly n elements),
+  // which is also what runs where the padded one does not fit
+  const bool fused = fused_trimul(a->c_z, a->c_h);
+  const size_t need = fused ? trimul_ws(a->batch, a->n, a->dtype, true).total
+                            : gen_trimul_ws(a->batch, a->n, a->c_z, a->c_h, a->dtype).total;
+  if (need > FJX_NOALLOC_MAX_BYTES)
     return fail(FJX_ERR_WORKSPACE,
                 "%s: this shape needs %zu bytes of scratch, the library's static scratch holds %zu "
                 "(use fjx_trimul_fwd with a workspace)",
-                fn, need, scratch_bytes);
+                fn, need, (size_t)FJX_NOALLOC_MAX_BYTES);
+  const bool tight = fused && trimul_ws(a->batch, a->n, a->dtype).total > scratch_bytes;
   fjx_trimul_args b = *a;
   b.workspace = scratch;
   b.workspace_bytes = scratch_bytes;
   g_no_events = true;
-  const int rc = trimul_dispatch(&b, st);
+  const int rc = trimul_dispatch(&b, tight, st);
   g_no_events = false;
   return rc;
 }

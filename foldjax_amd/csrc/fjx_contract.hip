@@ -23,7 +23,6 @@
 namespace fjx {
 
 constexpr int kNumXcd = 8;
-constexpr int64_t kOBlk = 256;  // positions per block of the tile-blocked output
 
 template <typename T> struct GemmCfg;
 template <> struct GemmCfg<bf16> { static constexpr int BK = 64; };
@@ -298,16 +297,24 @@ __global__ __launch_bounds__(512) void contract_kernel(const bf16* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// The same contraction for n a multiple of 256, fed by LDS DMA
-// (global_load_lds_dwordx4): the operands go global -> LDS without passing
-// through registers or LDS write instructions. DS stages of DK k each; the
-// configuration used (2 x 64, 128 KB) measured faster than deeper pipelines
-// of 32-wide stages (3 or 4 x 32), which pay a barrier per 32 k. Stage layout
-// per operand: 256 rows of 8 16-byte chunks (DK = 64), chunk c of row r in
-// slot 8r + (c ^ swz(r)) -- each wave's DMA instruction writes whole rows
+// The same contraction fed by LDS DMA (buffer_load_dwordx4 ... lds), for any n:
+// a and b have rows `pitch` elements apart, n rounded up to 64 with zeros past
+// n, so every row is whole 128-byte lines and the contracted length is whole
+// k-stages. The operands go global -> LDS without passing through registers or
+// LDS write instructions, in two stages of 64 k (deeper pipelines of 32-wide
+// stages measured slower: a barrier per 32 k).
+//
+// BT x BT output tile: 256 (512 threads, 2 x 4 waves of 128 x 64, one
+// workgroup per CU) or 128 (256 threads, 2 x 2 waves of 64 x 64, two per CU).
+//
+// Stage layout per operand: BT rows of 8 16-byte chunks, chunk c of row r in
+// slot 8 r + (c ^ swz(r)): each wave's DMA instruction writes whole rows
 // (1 KB, lane-ordered), and the swizzle, applied through the lanes' source
 // addresses, keeps the 16-byte fragment reads on 16 distinct bank groups:
 // with 128-byte rows the bank group of a chunk is 8 (r % 2) + (c ^ swz(r)).
+// Rows past n read as zero: they are past the end of the buffer resource
+// (whose range check covers the lane offset, not the scalar one; so rows are
+// in the former, k in the latter).
 //
 // Output columns: the B fragment of column tile j holds B rows in the
 // permuted order pcol(j, r) (the same permutation the flash attention uses
@@ -323,10 +330,26 @@ __global__ __launch_bounds__(512) void contract_kernel(const bf16* __restrict__ 
 // 16 (swz_a ^ swz_b)(r), which for the rows of DMA instruction j is
 // 32 (lane bit 5) XOR a constant.
 //
+// Persistent: the resident workgroups walk their XCD's contiguous share of the
+// tiles (workgroup w runs on XCD w % 8), so all tiles of a channel stay on
+// one XCD and reuse its L2. During the last k-step of a tile the first stage
+// of the next tile is already in flight, and the tile's output stores go out
+// after it: the next tile's first wait then covers that DMA only (vmcnt counts
+// loads and stores in issue order, so it waits for vmcnt(kStores); the stores
+// are buffer stores, issued also where no lane is in range, so that the count
+// is fixed), and the stores drain under the next k-loop.
+//
 // Synchronisation: each wave waits for its own DMA with an explicit vmcnt,
 // then a bare s_barrier (a fenced __syncthreads would wait for every DMA
 // still in flight).
 // ---------------------------------------------------------------------------
+// an SGPR value the compiler can not see through (the constraint letter means
+// something else to the host pass, which only parses this)
+__device__ __forceinline__ void opaque_sgpr(int& v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(v));
+#endif
+}
 __device__ __forceinline__ int swz_a(int r) { return (r >> 1) & 7; }
 __device__ __forceinline__ int swz_b(int r) { return ((r >> 1) & 1) | (((r >> 3) & 3) << 1); }
 __device__ __forceinline__ int slot_a(int r, int c) { return 8 * r + (c ^ swz_a(r)); }
@@ -335,33 +358,30 @@ __device__ __forceinline__ int slot_b(int r, int c) { return 8 * r + (c ^ swz_b(
 __device__ __forceinline__ int pcol(int j, int r) { return 32 * (j >> 1) + 8 * (r >> 2) + 4 * (j & 1) + (r & 3); }
 // a lane's 8 consecutive output columns 32s + 8 (lane / 16) .. +7 of row tile
 // i: accumulator rows 4 (lane / 16) .. +3 of column tiles 2s and 2s + 1
-__device__ __forceinline__ bf16x8 cols8(const f32x4 (&acc)[4][8], int i, int s) {
+template <int MI>
+__device__ __forceinline__ u32x4 cols8(const f32x4 (&acc)[4][MI], int i, int s) {
   const float v[8] = {acc[2 * s][i][0],     acc[2 * s][i][1],     acc[2 * s][i][2],     acc[2 * s][i][3],
                       acc[2 * s + 1][i][0], acc[2 * s + 1][i][1], acc[2 * s + 1][i][2], acc[2 * s + 1][i][3]};
-  return pack8<bf16>(v);
+  return __builtin_bit_cast(u32x4, pack8<bf16>(v));
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t crsrc(const void* base, int64_t bytes) {
+  const int64_t b = bytes > 0x7FFFFFFF ? 0x7FFFFFFF : bytes;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)b, 0x00020000);
 }
 
-// Persistent: one workgroup per CU walks its XCD's contiguous share of the
-// tiles (workgroup w runs on XCD w % 8), so all tiles of a channel stay on
-// one XCD and reuse its L2. During the last k-step of a tile the first stage
-// of the next tile is already in flight (its LDS buffer is free), and the
-// tile's output stores go out after it: the next tile's first wait then
-// covers that DMA only (vmcnt counts loads and stores in issue order, so it
-// waits for vmcnt(kStores)), and the stores drain under the next k-loop
-// instead of holding the workgroup at its exit.
-template <int DS, int DK>
-__global__ __launch_bounds__(512) void contract_dma_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
-                                                           bf16* __restrict__ O, int64_t n, int64_t batches,
-                                                           bool blocked) {
-  static_assert(DS == 2, "the persistent hand-over assumes two stages");
-  static_assert(DK == 64, "the swizzle is built for 8 chunks per row");
-  constexpr int CH = DK / 8;       // 16-byte chunks per row
-  constexpr int RPI = 64 / CH;     // rows per DMA instruction (1 KB)
-  constexpr int NI = CH / 2;       // DMA instructions per wave per operand per stage
-  constexpr int kStores = 16;      // output stores per lane per tile (8 rows x 2 of 8 elements)
-  __shared__ __attribute__((aligned(16))) bf16 S[DS][2][kCT * DK];  // [stage][A, B][256 rows x DK]
+// blocked: o as [item][row][64-column block][128 channels][64]
+// (TriMulEpilogueParams::o_blocked), else [batch][row][pitch]
+template <int BT>
+__device__ __forceinline__ void contract_dma_body(const bf16* __restrict__ A, const bf16* __restrict__ B,
+                                                  bf16* __restrict__ O, int n, int pitch, int64_t batches,
+                                                  bool blocked) {
+  constexpr int DK = 64;               // k per stage
+  constexpr int MI = BT / 32;          // 16-row tiles per wave
+  constexpr int WN = BT / 64;          // waves along the columns (2 along the rows)
+  constexpr int kStores = 2 * MI;      // output stores per lane per tile
+  __shared__ __attribute__((aligned(16))) bf16 S[2][2][BT * DK];  // [stage][A, B][BT rows x 64]
 
-  const int64_t tpd = n / kCT;
+  const int tpd = (n + BT - 1) / BT;
   const int64_t total = batches * tpd * tpd;
   const int64_t per_xcd = gridDim.x / kNumXcd;  // workgroups per XCD (the grid is a multiple of 8)
   const int64_t xcd = blockIdx.x % kNumXcd;
@@ -372,70 +392,74 @@ __global__ __launch_bounds__(512) void contract_dma_kernel(const bf16* __restric
   const int lane = t & 63;
   const int li = lane & 15;
   const int lg = lane >> 4;
-  const int wm = (wave >> 2) * 128;
-  const int wn = (wave & 3) * 64;
+  const int wm = (wave / WN) * 16 * MI;
+  const int wn = (wave % WN) * 64;
 
-  // DMA sources: a uniform base per operand plus a 32-bit per-lane byte
-  // offset that is the same for both operands (row r of the tile, swizzled
-  // chunk c); 64-bit per-lane pointers would cost 32 VGPRs at a point where
-  // the accumulators leave none to spare
-  uint32_t voff[NI];
+  // DMA sources: row r = 32 wave + 8 j + lane / 8 of the tile, swizzled chunk
+  uint32_t voff[4];
+  const int pb = 2 * pitch;  // bytes per row, a multiple of 128
 #pragma unroll
-  for (int j = 0; j < NI; ++j) {
-    const int r = 32 * wave + RPI * j + lane / CH;
-    const int c = (lane % CH) ^ swz_a(r);
-    voff[j] = (uint32_t)(r * n * 2 + 16 * c);
+  for (int j = 0; j < 4; ++j) {
+    const int r = 32 * wave + 8 * j + lane / 8;
+    voff[j] = (uint32_t)(r * pb + 16 * ((lane % 8) ^ swz_a(r)));
   }
-  // B's offsets: voff[j] ^ xb ^ kBx[j] (r * n * 2 is a multiple of 512, so
-  // the XOR touches only the chunk bits)
-  static_assert(NI == 4, "kBx lists the four DMA instructions of a stage");
+  // B's offsets: voff[j] ^ xb ^ kBx[j] (the XOR touches only the chunk bits)
   constexpr uint32_t kBx[4] = {0u, 32u | 64u, 64u, 32u};  // 16 (2 (j % 2) + 4 ((j ^ (j >> 1)) % 2))
   const uint32_t xb = (uint32_t)(32 * ((lane >> 5) & 1));
   struct Tile {
-    int64_t bat, m0, n0;
-    const char* base[2];
+    int64_t bat;
+    int m0, n0;
+    __amdgpu_buffer_rsrc_t ra, rb;
   };
   // tile (bat, ti, tj) = lid as bat * tpd^2 + ti * tpd + tj; a workgroup's
   // tiles are lid, lid + per_xcd, ..., so the next one's coordinates come
   // from fixed carries instead of 64-bit divisions in the tile loop (whose
   // reciprocal estimates the compiler keeps in spilled registers, with a
   // vmcnt(0) reload that would wait for the previous tile's stores)
-  auto tile_at = [&](int64_t bat, int64_t ti, int64_t tj) {
+  auto tile_at = [&](int64_t bat, int ti, int tj) {
     Tile tl;
     tl.bat = bat;
-    tl.m0 = ti * kCT;
-    tl.n0 = tj * kCT;
-    tl.base[0] = reinterpret_cast<const char*>(A + (tl.bat * n + tl.m0) * n);
-    tl.base[1] = reinterpret_cast<const char*>(B + (tl.bat * n + tl.n0) * n);
+    tl.m0 = ti * BT;
+    tl.n0 = tj * BT;
+    tl.ra = crsrc(A + (bat * n + tl.m0) * pitch, (int64_t)(n - tl.m0) * pb);
+    tl.rb = crsrc(B + (bat * n + tl.n0) * pitch, (int64_t)(n - tl.n0) * pb);
     return tl;
   };
-  const int64_t tt = tpd * tpd;
-  const int64_t step_b = per_xcd / tt, step_i = (per_xcd % tt) / tpd, step_j = per_xcd % tpd;
-  // k-tile kt goes to stage kt % DS; the stage is always a compile-time
+  const int64_t tt = (int64_t)tpd * tpd;
+  const int64_t step_b = per_xcd / tt;
+  const int step_i = (int)((per_xcd % tt) / tpd), step_j = (int)(per_xcd % tpd);
+  // k-tile kt goes to stage kt % 2; the stage is always a compile-time
   // constant (a run-time stage index makes the compiler wait for every DMA in
   // flight before each LDS read)
-  auto issue = [&](const Tile& tl, int64_t kt, int st) {
-    const int64_t k0 = kt * DK;
+  auto issue = [&](const Tile& tl, int kt, int st) {
+    // opaque per call: keeps B's offsets from being hoisted into four more
+    // loop-invariant registers, which the accumulators leave no room for
 #pragma unroll
-    for (int op = 0; op < 2; ++op)
+    for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(voff[j]));
 #pragma unroll
-      for (int j = 0; j < NI; ++j)
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(tl.base[op] + 2 * k0 +
-                                                                       (op ? voff[j] ^ (xb ^ kBx[j]) : voff[j])),
-                                         reinterpret_cast<void*>(&S[st][op][(32 * wave + RPI * j) * DK]), 16, 0, 0);
+    for (int j = 0; j < 4; ++j) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          tl.ra, (__attribute__((address_space(3))) void*)(&S[st][0][(32 * wave + 8 * j) * DK]), 16, voff[j],
+          (uint32_t)(2 * DK * kt), 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          tl.rb, (__attribute__((address_space(3))) void*)(&S[st][1][(32 * wave + 8 * j) * DK]), 16,
+          voff[j] ^ (xb ^ kBx[j]), (uint32_t)(2 * DK * kt), 0, 0);
+    }
   };
 
-  const int64_t ktiles = n / DK;  // a multiple of DS (checked by the launcher)
+  const int ktiles = pitch / DK;
   int64_t lid = xcd * total / kNumXcd + blockIdx.x / kNumXcd;
   if (lid >= hi) return;
-  int64_t cb = lid / tt, ci = (lid % tt) / tpd, cj = lid % tpd;
+  int64_t cb = lid / tt;
+  int ci = (int)((lid % tt) / tpd), cj = (int)(lid % tpd);
   Tile cur = tile_at(cb, ci, cj);
   issue(cur, 0, 0);
-  bool first = true;
+  int pend = 0;  // the previous tile's stores may be in flight (opaque: or the compiler peels a k-step per case)
   for (;;) {
     const int64_t next_lid = lid + per_xcd;
     const bool has_next = next_lid < hi;
-    int64_t nb = cb + step_b, ni = ci + step_i, nj = cj + step_j;
+    int64_t nb = cb + step_b;
+    int ni = ci + step_i, nj = cj + step_j;
     if (nj >= tpd) {
       nj -= tpd;
       ++ni;
@@ -446,34 +470,34 @@ __global__ __launch_bounds__(512) void contract_dma_kernel(const bf16* __restric
     }
     const Tile nxt = has_next ? tile_at(nb, ni, nj) : cur;
 
-    f32x4 acc[4][8];
+    f32x4 acc[4][MI];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < MI; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    for (int64_t kb = 0; kb < ktiles; kb += DS) {
+    for (int kb = 0; kb < ktiles; kb += 2) {
 #pragma unroll
-      for (int st = 0; st < DS; ++st) {
-        const int64_t kt = kb + st;
-        // opaque per iteration: keeps the compiler from hoisting base + voff
-        // into eight loop-invariant 64-bit pointers (it then spills them)
-#pragma unroll
-        for (int j = 0; j < NI; ++j) asm volatile("" : "+v"(voff[j]));
+      for (int st = 0; st < 2; ++st) {
+        const int kt = kb + st;
+        if (st == 1 && kt >= ktiles) break;  // an odd number of k-tiles ends in stage 0
         // this wave's DMA of stage st is complete; on a tile's first k-step
         // the previous tile's stores, issued after that DMA, may still run
-        if (st == 0 && kt == 0 && !first) __builtin_amdgcn_s_waitcnt(0x0F70 | ((kStores >> 4) << 14) | (kStores & 15));
+        if (st == 0 && pend) __builtin_amdgcn_s_waitcnt(0x0F70 | ((kStores >> 4) << 14) | (kStores & 15));
         else __builtin_amdgcn_s_waitcnt(0xF70);
+        pend = 0;
+        opaque_sgpr(pend);
         __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");  // no LDS read moves above the barrier
         if (kt + 1 < ktiles) issue(cur, kt + 1, st ^ 1);
-        else if (has_next) issue(nxt, 0, st ^ 1);  // stage 0 of the next tile (ktiles is even: buffer 0)
+        else if (has_next && st == 1) issue(nxt, 0, 0);  // stage 0 of the next tile
         const bf16* As_ = &S[st][0][0];
         const bf16* Bs_ = &S[st][1][0];
 #pragma unroll
         for (int ks = 0; ks < DK / 32; ++ks) {
-          bf16x8 af[8], bfr[4];
+          bf16x8 af[MI], bfr[4];
 #pragma unroll
-          for (int i = 0; i < 8; ++i)
+          for (int i = 0; i < MI; ++i)
             af[i] = *reinterpret_cast<const bf16x8*>(As_ + 8 * slot_a(wm + 16 * i + li, 4 * ks + lg));
 #pragma unroll
           for (int j = 0; j < 4; ++j)
@@ -481,38 +505,36 @@ __global__ __launch_bounds__(512) void contract_dma_kernel(const bf16* __restric
 #pragma unroll
           for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) mma(acc[j][i], bfr[j], af[i]);
+            for (int i = 0; i < MI; ++i) mma(acc[j][i], bfr[j], af[i]);
         }
       }
     }
+    if (ktiles & 1) {
+      // an odd number of k-tiles: the last one is in stage 0, where the next
+      // tile's first stage goes once every wave is past its reads
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (has_next) issue(nxt, 0, 0);
+    }
 
-    // the lane's row and column offsets, opaque here: the store addresses are
-    // then formed after the k-loop instead of being hoisted above it (eight
-    // 64-bit addresses the accumulators leave no room for: spilled, and the
-    // reload's vmcnt(0) would wait for the next tile's DMA)
+    // the lane's row and column offsets, opaque here: the store offsets are
+    // then formed after the k-loop instead of being hoisted above it
     int lrow = li, lcol = 8 * lg;
     asm volatile("" : "+v"(lrow), "+v"(lcol));
-    if (blocked) {
-      // [item][position / 64][channel][position % 64]; cur.bat = item * 128 + channel
-      // the tile's 256 columns are one 256-position block of each row (n and
-      // n0 are multiples of 256): block row * n/256 + n0/256
-      bf16* Ob = O + ((cur.bat >> 7) * (n * n) * tile::kC) + (cur.bat & 127) * kOBlk +
-                 (cur.n0 / kOBlk) * (tile::kC * kOBlk) + wn + lcol;
-      const int64_t bpr = (n / kOBlk) * (tile::kC * kOBlk);  // elements per row of blocks
+    // this wave's 64 columns start at c0, all of them within the pitch or none
+    const int c0 = cur.n0 + wn;
+    const int rstride = blocked ? pitch * tile::kC : pitch;  // elements per output row
+    const bf16* Ob = blocked ? O + ((cur.bat >> 7) * n + cur.m0) * (int64_t)rstride + (int64_t)c0 * tile::kC +
+                                   (cur.bat & 127) * 64
+                             : O + (cur.bat * n + cur.m0) * (int64_t)rstride + c0;
+    const __amdgpu_buffer_rsrc_t ro = crsrc(Ob, c0 < pitch ? ((int64_t)(n - cur.m0 - 1) * rstride + 64) * 2 : 0);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        bf16* dst = Ob + (cur.m0 + wm + 16 * i + lrow) * bpr;
+    for (int i = 0; i < MI; ++i) {
+      const int r = wm + 16 * i + lrow;
+      const uint32_t off = (uint32_t)(r * rstride + lcol) * 2;
 #pragma unroll
-        for (int s = 0; s < 2; ++s) store8(dst + 32 * s, cols8(acc, i, s));
-      }
-    } else {
-      bf16* Ob = O + cur.bat * n * n + cur.n0 + wn + lcol;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        bf16* dst = Ob + (cur.m0 + wm + 16 * i + lrow) * n;
-#pragma unroll
-        for (int s = 0; s < 2; ++s) store8(dst + 32 * s, cols8(acc, i, s));
-      }
+      for (int s = 0; s < 2; ++s)
+        __builtin_amdgcn_raw_buffer_store_b128(cols8<MI>(acc, i, s), ro, off, 64 * s, 0);
     }
     if (!has_next) break;
     lid = next_lid;
@@ -520,25 +542,54 @@ __global__ __launch_bounds__(512) void contract_dma_kernel(const bf16* __restric
     ci = ni;
     cj = nj;
     cur = nxt;
-    first = false;
+    pend = 1;
+    opaque_sgpr(pend);
   }
 }
 
-bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t batches, hipStream_t st,
+__global__ __launch_bounds__(512) void contract_dma_kernel_256(const bf16* __restrict__ A, const bf16* __restrict__ B,
+                                                               bf16* __restrict__ O, int n, int pitch,
+                                                               int64_t batches, bool blocked) {
+  contract_dma_body<256>(A, B, O, n, pitch, batches, blocked);
+}
+__global__ __launch_bounds__(256) void contract_dma_kernel_128(const bf16* __restrict__ A, const bf16* __restrict__ B,
+                                                               bf16* __restrict__ O, int n, int pitch,
+                                                               int64_t batches, bool blocked) {
+  contract_dma_body<128>(A, B, O, n, pitch, batches, blocked);
+}
+
+template <int BT>
+static void launch_contract_dma(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t pitch, int64_t batches,
+                                hipStream_t st, bool blocked) {
+  // persistent: the device's resident capacity, a multiple of the 8 XCDs,
+  // and no more workgroups than tiles need (rounded up to 8)
+  const int64_t tpd = (n + BT - 1) / BT;
+  const int64_t total = batches * tpd * tpd;
+  const auto kern = BT == 256 ? contract_dma_kernel_256 : contract_dma_kernel_128;
+  const void* k = reinterpret_cast<const void*>(kern);
+  const int64_t cap = std::max<int64_t>(kNumXcd, tile::resident_blocks(k, 2 * BT) / kNumXcd * kNumXcd);
+  const int64_t grid = std::min<int64_t>(cap, (total + kNumXcd - 1) / kNumXcd * kNumXcd);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(2 * BT), 0, st, a, b, o, (int)n, (int)pitch,
+                     batches, blocked);
+}
+
+bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t pitch, int64_t batches, hipStream_t st,
                      bool blocked) {
-  const int64_t tpd = (n + kCT - 1) / kCT;
-  if (n % kCT == 0) {
+  if (pitch % 64 == 0) {
     blocked = blocked && batches % tile::kC == 0;
-    // persistent: the device's resident capacity, a multiple of the 8 XCDs,
-    // and no more workgroups than tiles need (rounded up to 8)
-    const void* k = reinterpret_cast<const void*>(&contract_dma_kernel<2, 64>);
-    const int64_t total = batches * tpd * tpd;
-    const int64_t cap = std::max<int64_t>(kNumXcd, tile::resident_blocks(k, 512) / kNumXcd * kNumXcd);
-    const int64_t grid = std::min<int64_t>(cap, (total + kNumXcd - 1) / kNumXcd * kNumXcd);
-    hipLaunchKernelGGL((contract_dma_kernel<2, 64>), dim3((unsigned)grid), dim3(512), 0, st, a, b, o, n, batches,
-                       blocked);
+    // 128-wide tiles where 256-wide ones would leave CUs without a tile or
+    // compute a quarter more padding: whole tri-mul, 128 against 256: 51.8 / 54.5
+    // us at n = 256 and 73.5 / 83.3 at 300; 256 elsewhere, its operands being
+    // read half as often: 748.7 / 677.5 us at n = 1024, 342 / 335 at 700
+    const int64_t t256 = (n + 255) / 256, t128 = (n + 127) / 128;
+    if (batches * t256 * t256 < 256 || 5 * t128 * t128 <= 16 * t256 * t256)
+      launch_contract_dma<128>(a, b, o, n, pitch, batches, st, blocked);
+    else
+      launch_contract_dma<256>(a, b, o, n, pitch, batches, st, blocked);
     return blocked;
   }
+  // rows not padded (a fixed scratch that does not hold the padding)
+  const int64_t tpd = (n + kCT - 1) / kCT;
   hipLaunchKernelGGL(contract_kernel, dim3((unsigned)(batches * tpd * tpd)), dim3(512), 0, st, a, b, o, n, batches);
   return false;
 }

@@ -15,9 +15,10 @@ struct TriMulPrologueParams {
   const T* ln_b;
   const T* w_p;     // [256][128]: rows 0..127 -> a, 128..255 -> b
   const T* w_g;     // [256][128]
-  T* a_cm;          // [B][128][N*N] virtual grid
+  T* a_cm;          // [B][128][N][pitch] virtual grid; columns N .. pitch-1 are written as zeros
   T* b_cm;
   int64_t n;
+  int64_t pitch;    // elements per row of a and b: N rounded up to 8, or N (tight)
   float eps;
   int transpose;    // 1 for the incoming direction
   int cw;           // channels of x (and rows of w_p/w_g) when below 128 (a multiple of 32); 0: 128
@@ -49,7 +50,7 @@ struct TriAttnPrologueParams {
 
 template <typename T>
 struct TriMulEpilogueParams {
-  const T* o;         // contraction output, channel-major [B][128][N*N], or tile-blocked (o_blocked)
+  const T* o;         // contraction output, channel-major [B][128][N][pitch], or tile-blocked (o_blocked)
   const T* x;         // the op's input [B][N][N][128] (for the output gate)
   const T* ln_in_w;   // LN_in, recomputed for the gate
   const T* ln_in_b;
@@ -62,9 +63,10 @@ struct TriMulEpilogueParams {
   T* out;
   int64_t n;
   float eps;
-  // o tile-blocked: [B][N*N/256][128][256], the 128 channels of 256
-  // consecutive positions in one 64 KB block (the LDS-DMA contraction's
-  // blocked output)
+  int64_t pitch;      // elements per row of o: N rounded up to 8, or N (tight)
+  // o tile-blocked (the LDS-DMA contraction's output): a row's columns in
+  // blocks of 64, [B][N rows][pitch / 64 blocks][128 channels][64], the last
+  // block of a row pitch % 64 columns wide when that is not 0
   bool o_blocked;
   int cw;             // channels of x / out (k of w_gout, rows of both weights) when below 128; 0: 128
 };
@@ -194,11 +196,13 @@ void launch_gemm(const GemmParams<T, TO>& p, hipStream_t st);
 bool launch_gemm_dma(const GemmParams<bf16, bf16>& p, hipStream_t st);
 // whether launch_gemm_dma takes p (shape, alignment and size)
 bool gemm_dma_ok(const GemmParams<bf16, bf16>& p);
-// triangle contraction, bf16: o[c] = a[c] b[c]^T for c < batches, each n x n
-// blocked: write o tile-blocked, [batches / 128][N*N/256][128][256] (needs
-// batches a multiple of 128 and n a multiple of 256), else [batches][N*N];
-// returns whether it wrote the blocked layout
-bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t batches, hipStream_t st,
+// triangle contraction, bf16: o[c] = a[c] b[c]^T for c < batches, each n rows
+// of n elements, rows `pitch` apart in a, b and o. A pitch that is a multiple
+// of 8 (with zeros past n in a and b) runs the LDS-DMA kernel; pitch == n any n.
+// blocked: write o tile-blocked (TriMulEpilogueParams::o_blocked; needs
+// batches a multiple of 128), else [batches][n][pitch]; returns whether it
+// wrote the blocked layout
+bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t pitch, int64_t batches, hipStream_t st,
                      bool blocked = false);
 template <typename T>
 void launch_transition(const TransitionParams<T>& p, int c, hipStream_t st);

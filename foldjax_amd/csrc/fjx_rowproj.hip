@@ -51,9 +51,11 @@ namespace {
 // Triangle multiplication prologue, 512 threads: waves 0-3 produce a, waves 4-7
 // produce b, each wave 32 channels, holding the p_in and g_in slabs of those
 // channels for the whole launch.
-//   a_cm/b_cm: [B][128][N*N] channel-major in the virtual grid (contraction
-//   operands with the contracted axis contiguous), each
-//   mask * sigmoid(x_ln g_in^T) * (x_ln p_in^T).
+//   a_cm/b_cm: [B][128][N][pitch] channel-major in the virtual grid
+//   (contraction operands with the contracted axis contiguous), each
+//   mask * sigmoid(x_ln g_in^T) * (x_ln p_in^T), zero past column N.
+// A pitch that is a multiple of 8 makes every store 16 bytes whatever N is
+// (rows N apart: 2-byte stores when N is odd, 568 against 213 us at N = 1003).
 // kNarrow: x has P.cw < 128 channels (a multiple of 32); the tile's channels
 // past cw are held at zero (zero LayerNorm affine, zero weight columns). NB:
 // the 32-channel blocks of x worked on (cw / 32 when it is known at compile
@@ -79,8 +81,9 @@ __global__ __launch_bounds__(512) void trimul_prologue_kernel(TriMulProloguePara
   const int half = wave >> 2;
   const int col0 = 32 * (wave & 3);
   const int p = t >> 2;  // LayerNorm position of this thread
-  const bool vec4 = (n % 4) == 0;
-  const bool vec8 = (n % 8) == 0;
+  const int64_t pitch = P.pitch, plane = n * pitch;
+  const bool vec4 = (pitch % 4) == 0;
+  const bool vec8 = (pitch % 8) == 0;
   const int cw = kNarrow ? P.cw : kC;
 
   WSlab<T> wp, wg;
@@ -130,8 +133,9 @@ __global__ __launch_bounds__(512) void trimul_prologue_kernel(TriMulProloguePara
   __syncthreads();
   for (int cur = 0; tile < ntiles; tile += gridDim.x, cur ^= 1) {
     const TileRS tl = tile_at(tile, ntx, n);
-    const int nvalid = (int)min<int64_t>(kTP, n - tl.s0);
-    T* dst = (half == 0 ? P.a_cm : P.b_cm) + (int64_t)tl.b * kC * nn + (int64_t)tl.r * n + tl.s0;
+    // columns stored: up to the pitch, the ones past n zero (mrow is 0 there)
+    const int nstore = (int)min<int64_t>(kTP, pitch - tl.s0);
+    T* dst = (half == 0 ? P.a_cm : P.b_cm) + (int64_t)tl.b * kC * plane + (int64_t)tl.r * pitch + tl.s0;
     auto pair = [&](int j) {
       f32x4 ap[2][2], ag[2][2];
 #pragma unroll
@@ -148,7 +152,7 @@ __global__ __launch_bounds__(512) void trimul_prologue_kernel(TriMulProloguePara
           v[q] = m0[q] * sigmoid_nl2e(ag[0][ct][q]) * ap[0][ct][q];
           v[4 + q] = m1[q] * sigmoid_nl2e(ag[1][ct][q]) * ap[1][ct][q];
         }
-        store8_masked<T>(dst + (int64_t)(col0 + 16 * ct + (lane & 15)) * nn + p0, v, nvalid - p0, vec8, vec4);
+        store8_masked<T>(dst + (int64_t)(col0 + 16 * ct + (lane & 15)) * plane + p0, v, nstore - p0, vec8, vec4);
       }
     };
     pair(0);
@@ -368,7 +372,8 @@ __global__ __launch_bounds__(256) void trimul_epilogue_kernel(TriMulEpiloguePara
   const int col0 = 32 * wave;
   const int p = t >> 2;  // LayerNorm position of this thread
   constexpr bool res_x = kResX;
-  const bool vec8 = (n % 8) == 0;
+  const int64_t pitch = P.pitch;
+  const bool vec8 = (pitch % 8) == 0;
   const int cw = kNarrow ? P.cw : kC;
   const bool active = !kNarrow || col0 < cw;
 
@@ -403,17 +408,17 @@ __global__ __launch_bounds__(256) void trimul_epilogue_kernel(TriMulEpiloguePara
     const int64_t pos0 = (int64_t)tl.b * nn + (int64_t)tl.r * n + tl.s0;
     if constexpr (kNarrow) load_row_part_w<T, NB>(p < nvalid ? P.x + (pos0 + p) * cw : nullptr, xr, cw);
     else load_row_part<T>(p < nvalid ? P.x + (pos0 + p) * kC : nullptr, xr);
-    // channel-major: channel ch of the tile at src + ch * nn; tile-blocked:
-    // the whole tile is one contiguous [128][64] block
-    const int64_t cstride = P.o_blocked ? 256 : nn;
-    const int64_t ipos = (int64_t)tl.r * n + tl.s0;  // within the batch item
-    const T* src = P.o_blocked ? P.o + ((int64_t)tl.b * nn + (ipos & ~(int64_t)255)) * kC + (ipos & 255)
-                               : P.o + (int64_t)tl.b * kC * nn + ipos;
+    // channel-major: channel ch of the tile at src + ch * n * pitch;
+    // tile-blocked: the whole tile is one contiguous [128][ncols] block
+    const int ncols = (int)min<int64_t>(kTE, pitch - tl.s0);  // columns of o that exist
+    const int64_t cstride = P.o_blocked ? ncols : n * pitch;
+    const T* src = P.o_blocked ? P.o + (((int64_t)tl.b * n + tl.r) * pitch + tl.s0) * kC
+                               : P.o + ((int64_t)tl.b * kC * n + tl.r) * pitch + tl.s0;
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       int ch, p0;
       o_chunk(it, ch, p0);
-      if (vec8 && p0 + 8 <= nvalid) {
+      if (vec8 && p0 + 8 <= ncols) {
         ot[it] = load8(src + (int64_t)ch * cstride + p0);
       } else {
 #pragma unroll

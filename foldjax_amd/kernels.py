@@ -438,8 +438,7 @@ def trimul(
 
     ``no_alloc``: run ``fjx_trimul_fwd_noalloc`` instead, whose workspace is
     the library's static per-GPU scratch (shapes up to
-    ``_lib.NOALLOC_SCRATCH_BYTES`` of workspace; calls on one GPU must not
-    overlap). Only the output is allocated here, unless ``out`` is given:
+    256 MiB of unpadded workspace; calls on one GPU must not overlap). Only the output is allocated here, unless ``out`` is given:
     the result then goes into that tensor (x's shape, dtype and device,
     contiguous), which may be ``x`` and/or ``residual`` (in place)."""
     if direction not in ("outgoing", "incoming"):
