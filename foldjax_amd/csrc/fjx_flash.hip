@@ -1,4 +1,5 @@
-// Flash triangle attention on MFMA.
+// Flash triangle attention on MFMA with a softmax offset: the fp32 kernel, and
+// the bf16 fallback of the pipelined offset-free pass (fjx_flash_pipe.hip).
 //
 // One wave owns one attention row i of the pair grid and 64 or 128 queries of
 // one head; the ROWS waves of a workgroup own ROWS consecutive rows with the same
@@ -92,9 +93,9 @@ template <> __device__ __forceinline__ f32x8 ones8<float>(bool on) {
 // accumulator whose A operand is 1 only in rows 4(qt%4) .. +3, so lane group
 // g holds the sums of tile 4(qt/4) + g -- padded queries have zero scores,
 // so the zero-weighted rows add nothing)
-// vb: the workgroup's index in the launch grid of `total` workgroups (its
-// fallback flag and, through xcd_remap_f, its tile)
-template <typename T, int ROWS, int NQT, bool FAST = false>
+// vb: the workgroup's index in the launch grid of `total` workgroups (through
+// xcd_remap_f, its tile)
+template <typename T, int ROWS, int NQT>
 __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t vb, int64_t total) {
   typedef typename Frag<T>::type FragT;
   constexpr int QTL = 16 * NQT;
@@ -104,15 +105,10 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   __shared__ __attribute__((aligned(16))) FragT q_s[kQLds ? ROWS : 1][4][64];  // [wave][qt][lane]: B fragments of Q
   __shared__ __attribute__((aligned(16))) float mb_s[2][ROWS][kKB];  // each row's mask bias, one key block
 
-  // the offset path after a FAST launch: only the workgroups it flagged
-  if constexpr (!FAST) {
-    if (P.fallback && P.fallback[vb] == 0u) return;
-  }
-
   const int64_t n = P.n;
   const int64_t np = P.np;
   const int64_t H = P.heads;
-  const int64_t QT = np / QTL;
+  const int64_t QT = (np + QTL - 1) / QTL;
   const int64_t RG = (P.rows + ROWS - 1) / ROWS;
   int64_t lid = xcd_remap_f(vb, total);
   const int64_t qtile = lid % QT;
@@ -141,23 +137,6 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
 
   const int64_t nblk = np / kKB;
 
-  // offset-free pass: a row with every key masked (no mask bias above -1e8)
-  // would sum to 0. Its softmax is that of the unmasked scores (the mask is
-  // the same constant on every key and cancels), so such a row drops the
-  // masked keys' bias and keeps only the -inf of the padded keys.
-  bool full_row = false;
-  if constexpr (FAST) {
-    // 16-byte loads over the whole padded row (np is a multiple of 128; the
-    // padded keys hold -inf), four in flight per lane
-    bool any_valid = false;
-#pragma unroll 4
-    for (int64_t k0 = 4 * lane; k0 < np; k0 += 256) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(MB + k0);
-      any_valid |= (v[0] > -1.0e8f) | (v[1] > -1.0e8f) | (v[2] > -1.0e8f) | (v[3] > -1.0e8f);
-    }
-    full_row = __builtin_amdgcn_ballot_w64(any_valid) == 0;
-  }
-
   // Q stays in LDS (in fragment order: conflict-free 16-byte reads) and is
   // re-read per key block, which leaves registers for a second V buffer
   FragT qreg[kQLds ? 1 : NQT];
@@ -166,7 +145,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
     for (int qt = 0; qt < 4; ++qt) q_s[wave][qt][lane] = load8(Q + (q0 + 16 * qt + li) * kD + 8 * lg);
   } else {
 #pragma unroll
-    for (int qt = 0; qt < NQT; ++qt) qreg[qt] = load8(Q + (q0 + 16 * qt + li) * kD + 8 * lg);
+    for (int qt = 0; qt < NQT; ++qt) qreg[qt] = load8(Q + min<int64_t>(q0 + 16 * qt + li, np - 1) * kD + 8 * lg);
   }
 
   float m[NQT];
@@ -188,7 +167,10 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   static_assert(PASSES * RPP == QTL, "bias tile fill");
   const int br = t >> 3;
   const int bc = 8 * (t & 7);
-  const T* bsrc = BIAS + (q0 + br) * np + bc;
+  // a 128-query tile may end past np (by 64): its missing queries repeat the
+  // last row (of q too, above) and are not stored
+  const T* bsrc = BIAS + bc;
+  auto brow = [&](int c) { return min<int64_t>(q0 + br + RPP * c, np - 1) * np; };
   // the next key block's bias tile and mask bias travel in registers and are
   // written to the other LDS buffer at the end of the current block; the
   // mask flag (any non-zero mask bias in this row's block) is wave-uniform
@@ -196,7 +178,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   float mbn;
   auto fetch_tile = [&](int64_t k0) {
 #pragma unroll
-    for (int c = 0; c < PASSES; ++c) breg[c] = load8(bsrc + (int64_t)RPP * c * np + k0);
+    for (int c = 0; c < PASSES; ++c) breg[c] = load8(bsrc + brow(c) + k0);
     mbn = MB[k0 + lane];
   };
   auto put_tile = [&](int buf) {
@@ -257,12 +239,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
       if (masked_blk) {
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
-          f32x4 mv = *reinterpret_cast<const f32x4*>(&mb_s[buf][wave][col_of(kt, lg)]);
-          if (FAST && full_row) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) mv[r] = mv[r] < -1.0e30f ? mv[r] : 0.f;
-          }
-          s[kt] += mv;
+          s[kt] += *reinterpret_cast<const f32x4*>(&mb_s[buf][wave][col_of(kt, lg)]);
         }
       }
 #pragma unroll
@@ -273,14 +250,6 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
         for (int kt = 0; kt < 4; ++kt) kf[kt] = load8(K + (kn + key_of(kt, li)) * kD + 8 * lg);
       }
       float pv[4][4];
-      if constexpr (FAST) {
-        // no offset: exp2 of the raw log2-unit score; overflow or underflow
-        // of a whole row is caught after the last block
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) pv[kt][r] = __builtin_amdgcn_exp2f(s[kt][r]);
-      } else {
       // this lane's 16 scores: a max3 tree (5 + 2 + 1)
       const float t0 = fmaxf(fmaxf(s[0][0], s[0][1]), s[0][2]);
       const float t1 = fmaxf(fmaxf(s[0][3], s[1][0]), s[1][1]);
@@ -309,7 +278,6 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
       for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) pv[kt][r] = __builtin_amdgcn_exp2f(s[kt][r] - mnew);
-      }
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         const float f[8] = {pv[2 * c][0], pv[2 * c][1], pv[2 * c][2], pv[2 * c][3],
@@ -334,28 +302,6 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   }
 
   if (!row_ok) return;
-  if constexpr (FAST) {
-    // every softmax sum in [2^-100, inf) and every output finite, checked on
-    // the bit patterns (this file is compiled without NaN semantics);
-    // otherwise the workgroup is left to the offset path
-    bool bad = false;
-#pragma unroll
-    for (int qt = 0; qt < NQT; ++qt) {
-      float ls;
-      if constexpr (kQLds) ls = lsum[qt][0];
-      else ls = __shfl(lsum[qt >> 2][0], 16 * (qt & 3) + li, 64);
-      const unsigned u = __float_as_uint(ls);
-      bad |= !(u >= 0x0D800000u && u < 0x7F800000u);
-#pragma unroll
-      for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) bad |= (__float_as_uint(o[dt][qt][r]) & 0x7F800000u) == 0x7F800000u;
-    }
-    if (__builtin_amdgcn_ballot_w64(bad) != 0) {
-      if (lane == 0) P.fallback[vb] = 1u;
-      return;
-    }
-  }
   T* OUT = P.out + b * P.o_stride_b + i * P.o_stride_row + h * P.o_stride_head;
 #pragma unroll
   for (int qt = 0; qt < NQT; ++qt) {
@@ -378,22 +324,15 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
 
 constexpr int kRows = 4;
 
-// 128 queries per wave (bf16, np a multiple of 128): 256 VGPRs, 2 waves per
-// SIMD, 72 KB of LDS (two workgroups per CU); measured a few percent faster
-// than 64 queries at 3 waves per SIMD, as each K and V load serves twice the
-// queries
-__global__ __launch_bounds__(64 * kRows) __attribute__((amdgpu_waves_per_eu(2, 2))) void flash_tri8_kernel_bf16(FlashParams<bf16> P) {
-  flash_tri_body<bf16, kRows, 8>(P, blockIdx.x, gridDim.x);
-}
-
-// The same kernel as the fallback of the pipelined pass, over that pass's
-// grid of `total` workgroups: workgroup w reads the flags of `per`
-// consecutive ones (64 a load) and recomputes the flagged ones. Launched with
-// no more workgroups than the GPU holds at once, it costs few short
-// workgroups when nothing is flagged and, when everything is, as many rounds
-// of resident workgroups as the full grid would.
-__global__ __launch_bounds__(64 * kRows) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void flash_tri8_redo_kernel_bf16(FlashParams<bf16> P, int64_t total, int64_t per) {
+// The bf16 fallback of the pipelined offset-free pass (fjx_flash_pipe.hip),
+// over that pass's grid of `total` workgroups of 16 NQT queries: workgroup w
+// reads the flags of `per` consecutive ones (64 a load) and recomputes the
+// flagged ones with a softmax offset. Launched with no more workgroups than
+// the GPU holds at once, it costs few short workgroups when nothing is flagged
+// and, when everything is, as many rounds of resident workgroups as the full
+// grid would.
+template <int NQT>
+__device__ __forceinline__ void flash_redo_body(const FlashParams<bf16>& P, int64_t total, int64_t per) {
   const int64_t base = (int64_t)blockIdx.x * per;
   const int lane = threadIdx.x & 63;
   for (int64_t c0 = 0; c0 < per; c0 += 64) {
@@ -403,83 +342,53 @@ void flash_tri8_redo_kernel_bf16(FlashParams<bf16> P, int64_t total, int64_t per
     while (m != 0) {
       const int k = __builtin_ctzll(m);
       m &= m - 1;
-      flash_tri_body<bf16, kRows, 8>(P, base + c0 + k, total);
+      flash_tri_body<bf16, kRows, NQT>(P, base + c0 + k, total);
       __syncthreads();  // LDS is reused by the next flagged workgroup
     }
   }
 }
-
-// The same 128-query kernel without a softmax offset: p = exp2(s) straight
-// from the log2-unit scores, so no running max, no subtraction and no rescale
-// branch per query tile. Softmax is invariant to the offset, and exp2 of any
-// score in [-126, 127] is a normal float whose bf16 rounding is the same
-// relative error as with an offset; a row whose scores leave that range (or a
-// row with every key masked, whose sums underflow to 0) shows up as a sum
-// below 2^-100 or a non-finite value after its last block, and its workgroup
-// is then recomputed by the offset kernel above.
-__global__ __launch_bounds__(64 * kRows) __attribute__((amdgpu_waves_per_eu(2, 2))) void flash_tri8_fast_kernel_bf16(FlashParams<bf16> P) {
-  flash_tri_body<bf16, kRows, 8, true>(P, blockIdx.x, gridDim.x);
+// 128 queries per wave: 256 VGPRs, 2 waves per SIMD, 72 KB of LDS
+__global__ __launch_bounds__(64 * kRows) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void flash_tri8_redo_kernel_bf16(FlashParams<bf16> P, int64_t total, int64_t per) {
+  flash_redo_body<8>(P, total, per);
 }
-
-__global__ void zero_flags_kernel(unsigned* __restrict__ f, int64_t count) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
-    f[i] = 0u;
-}
-
-// bf16: 3 waves per SIMD (168 VGPRs) measured faster than 2 without spills;
-// the fp32 variant would spill heavily under that cap and keeps 2.
+// 64 queries: 3 waves per SIMD (168 VGPRs) measured faster than 2 without spills
 __global__ __launch_bounds__(64 * kRows) __attribute__((amdgpu_waves_per_eu(3, 3)))
-void flash_tri_kernel_bf16(FlashParams<bf16> P) {
-  flash_tri_body<bf16, kRows, 4>(P, blockIdx.x, gridDim.x);
+void flash_tri4_redo_kernel_bf16(FlashParams<bf16> P, int64_t total, int64_t per) {
+  flash_redo_body<4>(P, total, per);
 }
-// its offset-free pass (as flash_tri8_fast_kernel_bf16)
-__global__ __launch_bounds__(64 * kRows) __attribute__((amdgpu_waves_per_eu(3, 3)))
-void flash_tri_fast_kernel_bf16(FlashParams<bf16> P) {
-  flash_tri_body<bf16, kRows, 4, true>(P, blockIdx.x, gridDim.x);
-}
+
 __global__ __launch_bounds__(64 * kRows) void flash_tri_kernel_f32(FlashParams<float> P) {
   flash_tri_body<float, kRows, 4>(P, blockIdx.x, gridDim.x);
 }
 
 template <typename T>
-void launch_flash(const FlashParams<T>& p_in, int64_t batch, hipStream_t st) {
-  const int64_t rg = (p_in.rows + kRows - 1) / kRows;
-  const dim3 grid((unsigned)(batch * p_in.heads * rg * (p_in.np / kQT)));
+void launch_flash(const FlashParams<T>& p, int64_t batch, hipStream_t st) {
   // one row (the single-track attention, a bias per head): the keys are split
   // over the waves of a workgroup instead (fjx_single_flash.hip)
-  if (p_in.rows == 1) {
-    launch_flash_single<T>(p_in, batch, st);
+  if (p.rows == 1) {
+    launch_flash_single<T>(p, batch, st);
     return;
   }
-  // the offset kernels skip unflagged workgroups whenever `fallback` is set,
-  // so it stays set only where an offset-free pass fills the flags first
-  FlashParams<T> plain = p_in;
-  plain.fallback = nullptr;
+  const int64_t groups = batch * p.heads * ((p.rows + kRows - 1) / kRows);
   if constexpr (std::is_same<T, bf16>::value) {
-    const FlashParams<T>& p = p_in;
-    const bool q128 = p.np % 128 == 0;
-    const dim3 g = q128 ? dim3((unsigned)(batch * p.heads * rg * (p.np / 128))) : grid;
-    if (p.fallback) {
-      // the pipelined pass writes every flag in the 128-query grid of the
-      // offset kernel; the offset kernel then redoes the flagged workgroups
-      if (q128 && launch_flash_pipe(p, batch, st)) {
-        const int64_t total = g.x;
-        const int64_t cap = tile::resident_blocks(reinterpret_cast<const void*>(&flash_tri8_redo_kernel_bf16), 64 * kRows);
-        const int64_t per = (total + cap - 1) / cap;
-        hipLaunchKernelGGL(flash_tri8_redo_kernel_bf16, dim3((unsigned)((total + per - 1) / per)), dim3(64 * kRows), 0,
-                           st, p, total, per);
-        return;
-      }
-      // offset-free pass, then the offset kernel for the workgroups it flagged
-      const int64_t nb = ((int64_t)g.x + 255) / 256;
-      hipLaunchKernelGGL(zero_flags_kernel, dim3((unsigned)(nb < 4096 ? nb : 4096)), dim3(256), 0, st, p.fallback,
-                         (int64_t)g.x);
-      hipLaunchKernelGGL(q128 ? flash_tri8_fast_kernel_bf16 : flash_tri_fast_kernel_bf16, g, dim3(64 * kRows), 0, st,
-                         p);
-    }
-    hipLaunchKernelGGL(q128 ? flash_tri8_kernel_bf16 : flash_tri_kernel_bf16, g, dim3(64 * kRows), 0, st, p);
-  } else
-    hipLaunchKernelGGL(flash_tri_kernel_f32, grid, dim3(64 * kRows), 0, st, plain);
+    // the pipelined pass writes every flag of its grid; the offset kernel then
+    // redoes the flagged workgroups
+    // 128 queries a workgroup (each K and V load serves twice the queries)
+    // unless that leaves the GPU mostly without workgroups: whole tri-attn,
+    // 64 against 128 queries: 36.2 / 38.0 us at n = 77, 49.8 / 54.3 at 150 (304
+    // workgroups of 128), 55.3 / 55.3 at 180 (360), 64.8 / 62.8 at 200, 267.7 /
+    // 237.7 at 499
+    const int queries = groups * ((p.np + 127) / 128) < 320 ? 64 : 128;
+    const int64_t total = groups * ((p.np + queries - 1) / queries);
+    launch_flash_pipe(p, groups, queries, st);
+    const auto redo = queries == 128 ? flash_tri8_redo_kernel_bf16 : flash_tri4_redo_kernel_bf16;
+    const int64_t cap = tile::resident_blocks(reinterpret_cast<const void*>(redo), 64 * kRows);
+    const int64_t per = (total + cap - 1) / cap;
+    hipLaunchKernelGGL(redo, dim3((unsigned)((total + per - 1) / per)), dim3(64 * kRows), 0, st, p, total, per);
+  } else {
+    hipLaunchKernelGGL(flash_tri_kernel_f32, dim3((unsigned)(groups * (p.np / kQT))), dim3(64 * kRows), 0, st, p);
+  }
 }
 
 template void launch_flash<bf16>(const FlashParams<bf16>&, int64_t, hipStream_t);

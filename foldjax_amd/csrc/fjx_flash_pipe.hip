@@ -7,11 +7,11 @@
 // from the log2-unit score. A workgroup whose sums or outputs leave the safe
 // range is flagged for the offset kernel of fjx_flash.hip, which recomputes
 // it (flash_tri8_redo_kernel_bf16 walks the flags); the flags are indexed in
-// that kernel's grid, which this kernel runs exactly (4 rows x 128 queries of
-// one head per workgroup).
+// that kernel's grid, which this kernel runs exactly (4 rows x 128 or 64
+// queries of one head per workgroup).
 //
 // Layout: 4 waves per workgroup, each owning one row of the group and its
-// 128 queries (NQT = 8 tiles of 16); two workgroups per CU, so two waves per
+// 128 queries (NQT = 8 tiles of 16; 64 in small calls); two workgroups per CU, so two waves per
 // SIMD (a wave cannot overlap its own exponentials with its own MFMAs; the
 // other wave of the SIMD fills in, also while one workgroup waits at its
 // per-block barrier).
@@ -42,10 +42,7 @@ namespace {
 constexpr int kPKB = 64;    // keys per block
 constexpr int kPD = 32;     // head dim
 constexpr int kPRows = 4;   // rows per workgroup
-constexpr int kPHalves = 1; // query groups per row (waves per row)
-constexpr int kPNqt = 8;    // query tiles of 16 per wave
-constexpr int kPQwg = 16 * kPNqt * kPHalves;  // queries per workgroup: 128, the fallback kernel's tile
-constexpr int kPWaves = kPRows * kPHalves;
+constexpr int kPWaves = kPRows;
 static_assert(kPWaves <= 4, "one byte of a workgroup's 32-bit fallback flag per wave");
 constexpr int kPXcd = 8;
 
@@ -77,16 +74,19 @@ __device__ __forceinline__ bf16x8 buf_load8(__amdgpu_buffer_rsrc_t r, uint32_t v
 
 }  // namespace
 
-__global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void flash_pipe_kernel_bf16(FlashParams<bf16> P) {
-  constexpr int NQT = kPNqt;
+// NQT query tiles of 16 per wave: 8 (128 queries a workgroup) or 4 (64). ODD:
+// an odd number of key blocks (a kernel of its own: one body with both tails
+// spilled 74 registers)
+template <int NQT, bool ODD>
+__device__ __forceinline__ void flash_pipe_body(const FlashParams<bf16>& P) {
+  constexpr int kPQwg = 16 * NQT;  // queries per workgroup, the fallback kernel's tile
   constexpr int NDMA = kPQwg / kPWaves / 8;  // DMA instructions per wave per block (8 bias rows of 128 B each)
   __shared__ __attribute__((aligned(16))) u32x4 bias_s[2][kPQwg * 8];
 
   const int64_t n = P.n;
   const int64_t np = P.np;
   const int64_t H = P.heads;
-  const int64_t QT = np / kPQwg;
+  const int64_t QT = (np + kPQwg - 1) / kPQwg;
   const int64_t RG = (P.rows + kPRows - 1) / kPRows;
   int64_t lid = pipe_remap(blockIdx.x, (int64_t)gridDim.x);
   const int64_t qtile = lid % QT;
@@ -103,12 +103,10 @@ void flash_pipe_kernel_bf16(FlashParams<bf16> P) {
   const int lane = t & 63;
   const int li = lane & 15;
   const int lg = lane >> 4;
-  const int half = wave / kPRows;
-  const int64_t row = rg * kPRows + wave % kPRows;
+  const int64_t row = rg * kPRows + wave;
   const bool row_ok = row < P.rows;
   const int64_t i = row_ok ? row : P.rows - 1;
   const int64_t q0 = qtile * kPQwg;
-  const int qw = 16 * NQT * half;  // this wave's first query in the workgroup's tile
 
   const int64_t head_off = ((b * P.rows + i) * H + h) * np;  // in rows of kPD
   const bf16* Q = P.q + head_off * kPD;
@@ -119,8 +117,14 @@ void flash_pipe_kernel_bf16(FlashParams<bf16> P) {
   const __amdgpu_buffer_rsrc_t rk = buf_rsrc(K, (uint32_t)(np * kPD * 2));
   const __amdgpu_buffer_rsrc_t rv = buf_rsrc(VT, (uint32_t)(kPD * np * 2));
   const __amdgpu_buffer_rsrc_t rm = buf_rsrc(MB, (uint32_t)(np * 4));
-  const __amdgpu_buffer_rsrc_t rb = buf_rsrc(BIAS, (uint32_t)(kPQwg * np * 2));
-  const int64_t nblk = np / kPKB;  // even: np is a multiple of 128
+  // the last 128-query tile of an np that is an odd multiple of 64 ends half
+  // way: its missing queries read zeros (q from past its resource's end, the
+  // bias rows of whole waves from an empty resource; the DMA's row offset is
+  // partly scalar, which the range check leaves out) and are not stored
+  const int qvalid = (int)min<int64_t>(kPQwg, np - q0);  // a multiple of 64
+  const __amdgpu_buffer_rsrc_t rb =
+      buf_rsrc(BIAS, kPQwg / kPWaves * wave < qvalid ? (uint32_t)(kPQwg * np * 2) : 0u);
+  const int64_t nblk = np / kPKB;
 
   // a row with every key masked would sum to 0; its softmax is that of the
   // unmasked scores (the mask is one constant on every key), so such a row
@@ -166,11 +170,11 @@ void flash_pipe_kernel_bf16(FlashParams<bf16> P) {
   // offsets, so that no 64-bit query index is formed here and kept (spilled
   // to scratch, whose stores and reloads reached HBM) until the output
   // stores after the key loop
-  const __amdgpu_buffer_rsrc_t rq = buf_rsrc(Q + q0 * kPD, (uint32_t)(kPQwg * kPD * 2));
+  const __amdgpu_buffer_rsrc_t rq = buf_rsrc(Q + q0 * kPD, (uint32_t)(qvalid * kPD * 2));
   bf16x8 qreg[NQT];
 #pragma unroll
   for (int qt = 0; qt < NQT; ++qt)
-    qreg[qt] = buf_load8(rq, (uint32_t)((qw + 16 * qt + li) * kPD * 2 + 16 * lg), 0);
+    qreg[qt] = buf_load8(rq, (uint32_t)((16 * qt + li) * kPD * 2 + 16 * lg), 0);
 
   bf16x8 kf[2][4];     // K of two blocks
   bf16x8 vf[2][2][2];  // V^T of two blocks: [set][dt][32-key chunk]
@@ -208,14 +212,15 @@ void flash_pipe_kernel_bf16(FlashParams<bf16> P) {
   for (int u = 0; u < NQT / 4; ++u) lsum[u] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // prologue: blocks 0 and 1 staged, their K, V and mask bias
+  const int64_t blk1 = ODD && nblk == 1 ? 0 : 1;
   dma_bias(0, IC<0>());
-  dma_bias(1, IC<1>());
+  dma_bias(blk1, IC<1>());
   load_k(0, IC<0>());
-  load_k(1, IC<1>());
+  load_k(blk1, IC<1>());
   load_v(0, IC<0>());
-  load_v(1, IC<1>());
+  load_v(blk1, IC<1>());
   load_mb(0, IC<0>());
-  load_mb(1, IC<1>());
+  load_mb(blk1, IC<1>());
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
 
@@ -240,7 +245,7 @@ void flash_pipe_kernel_bf16(FlashParams<bf16> P) {
   // 4 + lg key tiles 2 and 3; bf16 -> fp32 is the 16-bit word moved to the
   // high half
   auto read_bias = [&](f32x4 (&s)[4], auto buf, int qt) {
-    const int r = qw + 16 * qt + li;
+    const int r = 16 * qt + li;
 #pragma unroll
     for (int h2 = 0; h2 < 2; ++h2) {
       const u32x4 w = bias_s[decltype(buf)::value][8 * r + ((4 * h2 + lg) ^ ((r >> 1) & 7))];
@@ -377,9 +382,14 @@ void flash_pipe_kernel_bf16(FlashParams<bf16> P) {
     run_block(blk, IC<0>(), IC<1>());
     run_block(blk + 1, IC<1>(), IC<1>());
   }
-  run_block(nblk - 2, IC<0>(), IC<1>());
-  run_block(nblk - 1, IC<1>(), IC<0>());
-  accumulate(Pp, IC<1>(), NQT - 1);  // nblk is even: the last block used set 1
+  if constexpr (ODD) {
+    run_block(nblk - 1, IC<0>(), IC<0>());
+    accumulate(Pp, IC<0>(), NQT - 1);
+  } else {
+    run_block(nblk - 2, IC<0>(), IC<1>());
+    run_block(nblk - 1, IC<1>(), IC<0>());
+    accumulate(Pp, IC<1>(), NQT - 1);
+  }
   // the clamped prefetches may still be writing LDS: drain before leaving
   __builtin_amdgcn_s_waitcnt(0);
 
@@ -415,7 +425,7 @@ void flash_pipe_kernel_bf16(FlashParams<bf16> P) {
   for (int qt = 0; qt < NQT; ++qt) {
     const float ls = __shfl(lsum[qt >> 2][0], 16 * (qt & 3) + li, 64);
     const float inv = 1.0f / ls;
-    const int ql = qw + 16 * qt + li;  // query q0 + ql
+    const int ql = 16 * qt + li;  // query q0 + ql
     uint32_t a[2], c[2];  // a: dims 4g .., c: dims 16 + 4g ..
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
@@ -435,16 +445,23 @@ void flash_pipe_kernel_bf16(FlashParams<bf16> P) {
   }
 }
 
-bool launch_flash_pipe(const FlashParams<bf16>& p, int64_t batch, hipStream_t st) {
-  // needs the fallback flags (the offset kernel recomputes what this pass
-  // flags; every flag is written, none needs clearing first) and a padded
-  // length that is a multiple of 128; launches the grid of the fallback
-  // kernel
-  if (!p.fallback || p.rows < 2 || p.np % kPQwg != 0) return false;
-  const int64_t rg = (p.rows + kPRows - 1) / kPRows;
-  const dim3 grid((unsigned)(batch * p.heads * rg * (p.np / kPQwg)));
-  hipLaunchKernelGGL(flash_pipe_kernel_bf16, grid, dim3(64 * kPWaves), 0, st, p);
-  return true;
+#define FJX_PIPE(name, NQT, ODD)                                                                      \
+  __global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void name( \
+      FlashParams<bf16> P) {                                                                          \
+    flash_pipe_body<NQT, ODD>(P);                                                                     \
+  }
+FJX_PIPE(flash_pipe_kernel_bf16, 8, false)
+FJX_PIPE(flash_pipe_odd_kernel_bf16, 8, true)
+FJX_PIPE(flash_pipe64_kernel_bf16, 4, false)
+FJX_PIPE(flash_pipe64_odd_kernel_bf16, 4, true)
+#undef FJX_PIPE
+
+void launch_flash_pipe(const FlashParams<bf16>& p, int64_t groups, int queries, hipStream_t st) {
+  const dim3 grid((unsigned)(groups * ((p.np + queries - 1) / queries)));
+  const bool odd = (p.np / kPKB) & 1;
+  hipLaunchKernelGGL(queries == 128 ? (odd ? flash_pipe_odd_kernel_bf16 : flash_pipe_kernel_bf16)
+                                    : (odd ? flash_pipe64_odd_kernel_bf16 : flash_pipe64_kernel_bf16),
+                     grid, dim3(64 * kPWaves), 0, st, p);
 }
 
 }  // namespace fjx

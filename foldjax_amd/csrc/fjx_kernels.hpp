@@ -176,8 +176,8 @@ struct FlashParams {
   int64_t o_stride_head;
   int64_t o_stride_q;
   int64_t bias_stride_b;  // 0 when one bias is shared by all batches
-  // the bf16 pair-track path without a softmax offset (see fjx_flash.hip):
-  // one flag per workgroup of that launch, or null for the offset path only
+  // bf16, rows > 1: a flag per workgroup of the offset-free pass, written by
+  // it (fjx_flash_pipe.hip) and read by the offset kernel (fjx_flash.hip)
   unsigned* fallback;
 };
 
@@ -236,9 +236,10 @@ void launch_flash(const FlashParams<T>& p, int64_t batch, hipStream_t st);
 // (fjx_single_flash.hip); launch_flash routes such calls here
 template <typename T>
 void launch_flash_single(const FlashParams<T>& p, int64_t batch, hipStream_t st);
-// the pipelined offset-free pass (fjx_flash_pipe.hip); false when the shape
-// or the parameters do not suit it (then nothing is launched)
-bool launch_flash_pipe(const FlashParams<bf16>& p, int64_t batch, hipStream_t st);
+// the pipelined offset-free pass (fjx_flash_pipe.hip): `groups` (batch x heads
+// x row groups of 4) times np / queries workgroups (64 or 128 queries each),
+// each writing its fallback flag
+void launch_flash_pipe(const FlashParams<bf16>& p, int64_t groups, int queries, hipStream_t st);
 // the flash tile's instruction mix alone (fjx_probe.hip): kernel ms, or -1 on a HIP error
 int probe_issue_mix(int mix, int waves_per_simd, int iters, float* ms, hipStream_t st);
 int probe_hbm_stream(int mode, int wgs_per_cu, int64_t bytes, float* ms, hipStream_t st);

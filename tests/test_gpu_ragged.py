@@ -1,4 +1,4 @@
-"""Pair lengths that are no multiple of any tile, bf16 tri-mul.
+"""Pair lengths that are no multiple of any tile, bf16 tri-mul and tri-attn.
 
 The padding rule gives an exact check: a tail of masked tokens contributes
 zeros to the contraction, every position's own arithmetic is unchanged, and
@@ -6,7 +6,10 @@ both contraction tile sizes accumulate in the same order, so the n x n corner
 of an N x N call whose last N - n tokens are masked is bit-identical to the
 n x n call. The lengths sit around the edges of the 64-column rows, the
 128- and 256-wide tiles and the rule that picks between those. The padded
-side is checked against the oracle in test_gpu_triangle.py.
+side is checked against the oracle in test_gpu_triangle.py. The same holds
+for tri-attn (masked keys have probability zero, key blocks accumulate in one
+order), around the edges of the 64-key blocks, of the 64- and 128-query tiles
+and of the rule between those.
 """
 
 from __future__ import annotations
@@ -61,3 +64,48 @@ def test_trimul_without_row_padding():
     got = kernels.trimul(z, None, w, "incoming", no_alloc=True)
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n,padded", [(2, 64), (37, 64), (64, 128), (65, 192), (129, 192), (150, 256), (170, 256),
+                                      (191, 384), (257, 320), (300, 512), (449, 577)])
+@pytest.mark.parametrize("starting", [True, False])
+def test_triattn_corner_of_a_masked_call(n, padded, starting):
+    say(f"ragged triattn n={n} in {padded} starting={starting}")
+    w = P.pack_triattn_protenix(P.triattn_to_protenix(syn.triattn_weights(seed=6)), torch.bfloat16, "cuda")
+    z = _pair(padded, torch.bfloat16)
+    tok = (torch.arange(padded, device="cuda") < n).to(torch.bfloat16)
+    want = kernels.triattn(z, torch.outer(tok, tok)[None], w, starting=starting, residual=z)[:, :n, :n]
+    zn = z[:, :n, :n].contiguous()
+    got = kernels.triattn(zn, None, w, starting=starting, residual=zn)
+    torch.cuda.synchronize()
+    assert torch.isfinite(got.float()).all()
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows,n", [(5, 40), (3, 100), (9, 150), (81, 300), (81, 330)])
+def test_triattn_core_redone_at_every_tile(rows, n):
+    """Scores of hundreds in log2 units send workgroups of both query tiles,
+    of odd and even block counts and of the half-empty last tile to the offset
+    kernel. The reference is float32 torch on the same bf16 values; the
+    kernel's bf16 probabilities and output leave at most 2^-8 of the largest
+    value each (2^-9 per rounding, sums of positive terms), 2e-2 as for every
+    bf16 check."""
+    say(f"triattn core redo rows={rows} n={n}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    q, k, v = (torch.randn(1, rows, 4, n, 32, generator=g, device="cuda").bfloat16() for _ in range(3))
+    q = (q.float() * 40.0).bfloat16()
+    tb = torch.randn(1, 1, 4, n, n, generator=g, device="cuda").bfloat16()
+    keep = torch.rand(1, rows, n, generator=g, device="cuda") > 0.2
+    keep[..., 0] = True
+    mb = torch.where(keep, 0.0, -1e9)[:, :, None, None, :]
+    got = kernels.triattn_core(q, k, v, tb, mb, scale=32 ** -0.5)
+    # the kernels take scale * log2(e) into q in bf16
+    log2e = 1.4426950408889634
+    qs = (q.float() * (32 ** -0.5 * log2e)).bfloat16().float()
+    s = (qs @ k.float().transpose(-1, -2).contiguous()) / log2e + tb.float() + mb
+    want = torch.softmax(s, -1) @ v.float()
+    torch.cuda.synchronize()
+    assert torch.isfinite(got.float()).all()
+    err = (got.float() - want).norm() / want.norm()
+    assert err <= 2e-2, float(err)
