@@ -116,7 +116,8 @@ int timed(int id, hipStream_t st, const char* what, F&& launch) {
 }
 
 // --------------------------------------------------- attention-core prep
-// q/k: [B][R][H][n][32] -> [B][R][H][np][32] (q times qscale), zero padded keys
+// q/k: [B][R][H][n][32] -> [B][R][H][np][32] (q times qscale), zero padded
+// keys; for one attention row (the single-track flash kernel) only
 template <typename T>
 __global__ void pad_qk_kernel(const T* __restrict__ src, T* __restrict__ dst, int64_t n, int64_t np,
                               int64_t heads_rows, float mul) {
@@ -129,43 +130,76 @@ __global__ void pad_qk_kernel(const T* __restrict__ src, T* __restrict__ dst, in
     dst[idx] = s < n ? from_f32<T>(to_f32(src[(hr * n + s) * 32 + d]) * mul) : from_f32<T>(0.f);
   }
 }
-// v: [B][R][H][n][32] -> vt [B][R][H*32][np]
+
+// The other operands of the attention core, in one launch of three block
+// ranges of 256 threads:
+//   v: [heads_rows][n][32] -> vt [heads_rows][32][np] (zero past n), a 128-key
+//      piece per block through LDS, 16-byte accesses on both sides;
+//   bias: [planes][n][n] -> [planes][np][np] times log2 e (zero past n), a
+//      row per wave;
+//   mask bias: [mrows][n] fp32 -> [mrows][np] times log2 e, -inf past n (all
+//      zero without one), a row per wave.
+// q and k are read by the flash pass as they are. At 499 rows and keys, 4
+// heads: 270 us in five element-wise launches (q and k copied too) -> 28 us.
+constexpr int kPrepKeys = 128;
 template <typename T>
-__global__ void transpose_v_kernel(const T* __restrict__ src, T* __restrict__ dst, int64_t n, int64_t np,
-                                   int64_t heads_rows) {
-  const int64_t total = heads_rows * 32 * np;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t s = idx % np;
-    const int64_t d = (idx / np) % 32;
-    const int64_t hr = idx / (32 * np);
-    dst[idx] = s < n ? src[(hr * n + s) * 32 + d] : from_f32<T>(0.f);
+__global__ __launch_bounds__(256) void core_prep_kernel(const T* __restrict__ v, T* __restrict__ vt,
+                                                        const T* __restrict__ bias, T* __restrict__ bias_p,
+                                                        const float* __restrict__ mask, float* __restrict__ mask_p,
+                                                        int64_t n, int64_t np, int64_t vblocks, int64_t bblocks,
+                                                        int64_t planes, int64_t mrows) {
+  typedef typename Frag<T>::type Frag8;
+  const int t = threadIdx.x;
+  if (blockIdx.x < vblocks) {
+    // rows of 128 keys plus a 16-byte pad: a thread holds 8 dims of a pair of
+    // keys and writes them as pairs, 8 rows apart
+    __shared__ __attribute__((aligned(16))) T tile[32][kPrepKeys + 8];
+    const int64_t pieces = (np + kPrepKeys - 1) / kPrepKeys;
+    const int64_t hr = blockIdx.x / pieces;
+    const int64_t k0 = (blockIdx.x - hr * pieces) * kPrepKeys;
+    const int pair = t >> 2, d0 = 8 * (t & 3);
+    Frag8 r[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int64_t key = k0 + 2 * pair + u;
+      if (key < n) {
+        r[u] = load8(v + (hr * n + key) * 32 + d0);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r[u][e] = from_f32<T>(0.f);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      typedef T T2 __attribute__((ext_vector_type(2)));
+      *reinterpret_cast<T2*>(&tile[d0 + e][2 * pair]) = T2{r[0][e], r[1][e]};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int d = (t >> 4) + 16 * u, c = 8 * (t & 15);  // 16 lanes: one dim's 128 keys
+      if (k0 + c < np) store8(vt + (hr * 32 + d) * np + k0 + c, load8(&tile[d][c]));
+    }
+    return;
   }
-}
-// bias [B][H][n][n] -> [B][H][np][np] times log2 e, zeros outside
-template <typename T>
-__global__ void pad_bias_kernel(const T* __restrict__ src, T* __restrict__ dst, int64_t n, int64_t np,
-                                int64_t planes) {
-  const int64_t total = planes * np * np;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t k = idx % np;
-    const int64_t q = (idx / np) % np;
-    const int64_t pl = idx / (np * np);
-    const float v = (q < n && k < n) ? to_f32(src[(pl * n + q) * n + k]) * kLog2e : 0.f;
-    dst[idx] = from_f32<T>(v);
+  const int lane = t & 63;
+  int64_t row = (blockIdx.x - vblocks) * 4 + (t >> 6);
+  if (blockIdx.x < vblocks + bblocks) {
+    if (row >= planes * np) return;
+    const int64_t pl = row / np, q = row - pl * np;
+    const T* src = bias + (pl * n + q) * n;
+    for (int64_t k = 8 * lane; k < np; k += 512) {
+      float f[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = q < n && k + e < n ? to_f32(src[k + e]) * kLog2e : 0.f;
+      store8(bias_p + row * np + k, pack8<T>(f));
+    }
+    return;
   }
-}
-// mask bias [B][R][n] fp32 -> [B][R][np] times log2 e, -inf for padded keys
-__global__ void pad_mb_kernel(const float* __restrict__ src, float* __restrict__ dst, int64_t n, int64_t np,
-                              int64_t rows) {
-  const int64_t total = rows * np;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t k = idx % np;
-    const int64_t r = idx / np;
-    dst[idx] = k < n ? (src ? src[r * n + k] * kLog2e : 0.f) : -INFINITY;
-  }
+  row -= 4 * bblocks;
+  if (row >= mrows) return;
+  for (int64_t k = lane; k < np; k += 64)
+    mask_p[row * np + k] = k < n ? (mask ? mask[row * n + k] * kLog2e : 0.f) : -INFINITY;
 }
 
 dim3 grid_for(int64_t total) {
@@ -202,16 +236,17 @@ struct TriAttnWs {
 size_t flash_flags_bytes(int64_t batch, int64_t rows, int64_t heads, int64_t np) {
   return align_up((size_t)batch * heads * ((rows + 3) / 4) * ((np + 63) / 64) * sizeof(unsigned));
 }
-TriAttnWs triattn_ws(int64_t batch, int64_t rows, int64_t n, int64_t heads, int32_t dtype, bool with_o) {
+TriAttnWs triattn_ws(int64_t batch, int64_t rows, int64_t n, int64_t heads, int32_t dtype, bool with_o,
+                     bool with_qk = true) {
   const int64_t np = round64(n);
   const size_t es = esize(dtype);
   const size_t qk = align_up((size_t)batch * rows * heads * np * 32 * es);
   TriAttnWs w;
   size_t off = 0;
   w.q = off;
-  off += qk;
+  if (with_qk) off += qk;
   w.k = off;
-  off += qk;
+  if (with_qk) off += qk;
   w.vt = off;
   off += qk;
   w.bias = off;
@@ -332,6 +367,8 @@ int triattn_run(const fjx_triattn_args* a, hipStream_t st) {
   FlashParams<T> fp = {};
   fp.q = pp.q;
   fp.k = pp.k;
+  fp.qk_rows = np;
+  fp.q_mul = 1.f;
   fp.vt = pp.vt;
   fp.bias = pp.bias;
   fp.mb = pp.mb;
@@ -369,35 +406,44 @@ int triattn_run(const fjx_triattn_args* a, hipStream_t st) {
   return timed(K_TRIATTN_EPILOGUE, st, "triattn_epilogue", [&] { launch_triattn_epilogue<T>(ep, a->batch, st); });
 }
 
+// q and k are copied (padded) only for one attention row
+TriAttnWs core_ws(const int64_t batch, int64_t rows, int64_t n, int64_t heads, int32_t dtype) {
+  return triattn_ws(batch, rows, n, heads, dtype, false, rows == 1);
+}
+
 template <typename T>
 int core_run(const fjx_triattn_core_args* a, hipStream_t st) {
   const int64_t n = a->n;
   const int64_t np = round64(n);
   const int64_t hr = a->batch * a->rows * a->heads;
-  const TriAttnWs ws = triattn_ws(a->batch, a->rows, n, a->heads, a->dtype, false);
+  const TriAttnWs ws = core_ws(a->batch, a->rows, n, a->heads, a->dtype);
   void* W = a->workspace;
-  T* q = at<T>(W, ws.q);
-  T* k = at<T>(W, ws.k);
+  const bool one_row = a->rows == 1;
+  const T* q = one_row ? at<T>(W, ws.q) : static_cast<const T*>(a->q);
+  const T* k = one_row ? at<T>(W, ws.k) : static_cast<const T*>(a->k);
   T* vt = at<T>(W, ws.vt);
   T* bias = at<T>(W, ws.bias);
   float* mb = at<float>(W, ws.mb);
   int rc = timed(K_TRIATTN_CORE_PREP, st, "triattn_core_prep", [&] {
-    hipLaunchKernelGGL(pad_qk_kernel<T>, grid_for(hr * np * 32), dim3(256), 0, st,
-                       static_cast<const T*>(a->q), q, n, np, hr, a->scale * kLog2e);
-    hipLaunchKernelGGL(pad_qk_kernel<T>, grid_for(hr * np * 32), dim3(256), 0, st,
-                       static_cast<const T*>(a->k), k, n, np, hr, 1.0f);
-    hipLaunchKernelGGL(transpose_v_kernel<T>, grid_for(hr * np * 32), dim3(256), 0, st,
-                       static_cast<const T*>(a->v), vt, n, np, hr);
-    hipLaunchKernelGGL(pad_bias_kernel<T>, grid_for(a->batch * a->heads * np * np), dim3(256), 0, st,
-                       static_cast<const T*>(a->tri_bias), bias, n, np, a->batch * a->heads);
-    hipLaunchKernelGGL(pad_mb_kernel, grid_for(a->batch * a->rows * np), dim3(256), 0, st, a->mask_bias, mb, n,
-                       np, a->batch * a->rows);
+    if (one_row) {
+      hipLaunchKernelGGL(pad_qk_kernel<T>, grid_for(hr * np * 32), dim3(256), 0, st, static_cast<const T*>(a->q),
+                         at<T>(W, ws.q), n, np, hr, a->scale * kLog2e);
+      hipLaunchKernelGGL(pad_qk_kernel<T>, grid_for(hr * np * 32), dim3(256), 0, st, static_cast<const T*>(a->k),
+                         at<T>(W, ws.k), n, np, hr, 1.0f);
+    }
+    const int64_t planes = a->batch * a->heads, mrows = a->batch * a->rows;
+    const int64_t vblocks = hr * ((np + kPrepKeys - 1) / kPrepKeys), bblocks = (planes * np + 3) / 4;
+    hipLaunchKernelGGL(core_prep_kernel<T>, dim3((unsigned)(vblocks + bblocks + (mrows + 3) / 4)), dim3(256), 0, st,
+                       static_cast<const T*>(a->v), vt, static_cast<const T*>(a->tri_bias), bias, a->mask_bias, mb, n,
+                       np, vblocks, bblocks, planes, mrows);
   });
   if (rc) return rc;
 
   FlashParams<T> fp = {};
   fp.q = q;
   fp.k = k;
+  fp.qk_rows = one_row ? np : n;
+  fp.q_mul = one_row ? 1.f : a->scale * kLog2e;
   fp.vt = vt;
   fp.bias = bias;
   fp.mb = mb;
@@ -708,6 +754,8 @@ int triattn_generic_run(const fjx_triattn_args* a, hipStream_t st) {
   FlashParams<T> fp = {};
   fp.q = at<T>(W, ws.q);
   fp.k = at<T>(W, ws.k);
+  fp.qk_rows = np;
+  fp.q_mul = 1.f;
   fp.vt = at<T>(W, ws.vt);
   fp.bias = at<T>(W, ws.bias);
   fp.mb = at<float>(W, ws.mb);
@@ -935,6 +983,8 @@ int single_run(const fjx_single_attention_args* a, hipStream_t st) {
   FlashParams<T> fp = {};
   fp.q = at<T>(W, ws.q);
   fp.k = at<T>(W, ws.k);
+  fp.qk_rows = np;
+  fp.q_mul = 1.f;
   fp.vt = at<T>(W, ws.vt);
   fp.bias = a->pair_bias && !a->extra_bias ? static_cast<const T*>(a->pair_bias) : at<T>(W, ws.bias);
   fp.mb = at<float>(W, ws.mb);
@@ -1071,7 +1121,7 @@ size_t fjx_triattn_core_workspace_size(int64_t batch, int64_t rows, int64_t head
                                        int32_t dtype) {
   (void)head_dim;
   if (batch < 1 || rows < 1 || heads < 1 || n < 1 || !dtype_ok(dtype)) return 0;
-  return triattn_ws(batch, rows, n, heads, dtype, false).total;
+  return core_ws(batch, rows, n, heads, dtype).total;
 }
 
 int fjx_triattn_core(const fjx_triattn_core_args* a, hipStream_t st) {
@@ -1087,7 +1137,7 @@ int fjx_triattn_core(const fjx_triattn_core_args* a, hipStream_t st) {
     return fail(FJX_ERR_INVALID, "fjx_triattn_core: a required pointer is NULL");
   if (!aligned16({a->q, a->k, a->v, a->tri_bias, a->out}))
     return fail(FJX_ERR_INVALID, "fjx_triattn_core: tensors must be 16-byte aligned");
-  const size_t need = triattn_ws(a->batch, a->rows, a->n, a->heads, a->dtype, false).total;
+  const size_t need = core_ws(a->batch, a->rows, a->n, a->heads, a->dtype).total;
   if (!a->workspace || a->workspace_bytes < need)
     return fail(FJX_ERR_WORKSPACE, "fjx_triattn_core: workspace of %zu bytes needed, %zu given", need,
                 a->workspace_bytes);

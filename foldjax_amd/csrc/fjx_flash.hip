@@ -128,7 +128,8 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   const int64_t i = row_ok ? row : P.rows - 1;
   const int64_t q0 = qtile * QTL;
 
-  const int64_t head_off = ((b * P.rows + i) * H + h) * np;  // in rows of length kD
+  const int64_t head_off = ((b * P.rows + i) * H + h) * P.qk_rows;  // in rows of length kD
+  const int64_t last = P.qk_rows - 1;  // rows past it (padded queries and keys) repeat it
   const T* Q = P.q + head_off * kD;
   const T* K = P.k + head_off * kD;
   const T* VT = P.vt + ((b * P.rows + i) * H * kD + h * kD) * np;
@@ -140,12 +141,15 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   // Q stays in LDS (in fragment order: conflict-free 16-byte reads) and is
   // re-read per key block, which leaves registers for a second V buffer
   FragT qreg[kQLds ? 1 : NQT];
-  if constexpr (kQLds) {
 #pragma unroll
-    for (int qt = 0; qt < 4; ++qt) q_s[wave][qt][lane] = load8(Q + (q0 + 16 * qt + li) * kD + 8 * lg);
-  } else {
+  for (int qt = 0; qt < NQT; ++qt) {
+    FragT f = load8(Q + min<int64_t>(q0 + 16 * qt + li, last) * kD + 8 * lg);
+    if (P.q_mul != 1.f) {
 #pragma unroll
-    for (int qt = 0; qt < NQT; ++qt) qreg[qt] = load8(Q + min<int64_t>(q0 + 16 * qt + li, np - 1) * kD + 8 * lg);
+      for (int e = 0; e < 8; ++e) f[e] = from_f32<T>(to_f32(f[e]) * P.q_mul);
+    }
+    if constexpr (kQLds) q_s[wave][qt][lane] = f;
+    else qreg[qt] = f;
   }
 
   float m[NQT];
@@ -197,7 +201,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
 
   FragT kf[4];
 #pragma unroll
-  for (int kt = 0; kt < 4; ++kt) kf[kt] = load8(K + key_of(kt, li) * kD + 8 * lg);
+  for (int kt = 0; kt < 4; ++kt) kf[kt] = load8(K + min<int64_t>(key_of(kt, li), last) * kD + 8 * lg);
   // V of the current block in vf, the next block's arriving in vn
   FragT vf[2][2], vn[2][2];  // [dt][c]
   auto load_v = [&](FragT (&v)[2][2], int64_t k0) {
@@ -247,7 +251,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
       if (qt == NQT - 1) {
         // K of this block is consumed: fetch the next block's into the same registers
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) kf[kt] = load8(K + (kn + key_of(kt, li)) * kD + 8 * lg);
+        for (int kt = 0; kt < 4; ++kt) kf[kt] = load8(K + min<int64_t>(kn + key_of(kt, li), last) * kD + 8 * lg);
       }
       float pv[4][4];
       // this lane's 16 scores: a max3 tree (5 + 2 + 1)

@@ -108,13 +108,13 @@ __device__ __forceinline__ void flash_pipe_body(const FlashParams<bf16>& P) {
   const int64_t i = row_ok ? row : P.rows - 1;
   const int64_t q0 = qtile * kPQwg;
 
-  const int64_t head_off = ((b * P.rows + i) * H + h) * np;  // in rows of kPD
+  const int64_t head_off = ((b * P.rows + i) * H + h) * P.qk_rows;  // in rows of kPD
   const bf16* Q = P.q + head_off * kPD;
   const bf16* K = P.k + head_off * kPD;
   const bf16* VT = P.vt + ((b * P.rows + i) * H * kPD + h * kPD) * np;
   const float* MB = P.mb + (b * P.rows + i) * np;
   const bf16* BIAS = P.bias + b * P.bias_stride_b + (h * np + q0) * np;
-  const __amdgpu_buffer_rsrc_t rk = buf_rsrc(K, (uint32_t)(np * kPD * 2));
+  const __amdgpu_buffer_rsrc_t rk = buf_rsrc(K, (uint32_t)(P.qk_rows * kPD * 2));  // keys past it read as zero
   const __amdgpu_buffer_rsrc_t rv = buf_rsrc(VT, (uint32_t)(kPD * np * 2));
   const __amdgpu_buffer_rsrc_t rm = buf_rsrc(MB, (uint32_t)(np * 4));
   // the last 128-query tile of an np that is an odd multiple of 64 ends half
@@ -170,11 +170,17 @@ __device__ __forceinline__ void flash_pipe_body(const FlashParams<bf16>& P) {
   // offsets, so that no 64-bit query index is formed here and kept (spilled
   // to scratch, whose stores and reloads reached HBM) until the output
   // stores after the key loop
-  const __amdgpu_buffer_rsrc_t rq = buf_rsrc(Q + q0 * kPD, (uint32_t)(qvalid * kPD * 2));
+  const __amdgpu_buffer_rsrc_t rq = buf_rsrc(Q + q0 * kPD, (uint32_t)(max<int64_t>(0, min<int64_t>(kPQwg, P.qk_rows - q0)) * kPD * 2));
   bf16x8 qreg[NQT];
 #pragma unroll
   for (int qt = 0; qt < NQT; ++qt)
     qreg[qt] = buf_load8(rq, (uint32_t)((16 * qt + li) * kPD * 2 + 16 * lg), 0);
+  if (P.q_mul != 1.f) {
+#pragma unroll
+    for (int qt = 0; qt < NQT; ++qt)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qreg[qt][e] = from_f32<bf16>(to_f32(qreg[qt][e]) * P.q_mul);
+  }
 
   bf16x8 kf[2][4];     // K of two blocks
   bf16x8 vf[2][2][2];  // V^T of two blocks: [set][dt][32-key chunk]
@@ -182,10 +188,12 @@ __device__ __forceinline__ void flash_pipe_body(const FlashParams<bf16>& P) {
   // 8 (li/4) + li%4 plus 32 (kt/2) + 4 (kt%2), the latter a constant offset
   const uint32_t koff = (uint32_t)((8 * (li >> 2) + (li & 3)) * kPD * 2 + 16 * lg);
   auto load_k = [&](int64_t blk, auto set) {
+    // the block in the lane offset: the range check leaves the scalar one out
+    const uint32_t kblk = koff + (uint32_t)(blk * kPKB * kPD * 2);
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
       kf[decltype(set)::value][kt] =
-          buf_load8(rk, koff + (uint32_t)((32 * (kt >> 1) + 4 * (kt & 1)) * kPD * 2), (uint32_t)(blk * kPKB * kPD * 2));
+          buf_load8(rk, kblk + (uint32_t)((32 * (kt >> 1) + 4 * (kt & 1)) * kPD * 2), 0);
   };
   const uint32_t voff = (uint32_t)(li * np * 2 + 16 * lg);  // V^T row li, keys 8 lg .. +7
   auto load_v = [&](int64_t blk, auto set) {

@@ -161,8 +161,8 @@ struct TransitionParams {
 
 template <typename T>
 struct FlashParams {
-  const T* q;        // [B][N][H][Np][32], pre-scaled by scale*log2 e
-  const T* k;        // [B][N][H][Np][32]
+  const T* q;        // [B][N][H][qk_rows][32], times q_mul on load: scale*log2 e (or 1, pre-scaled)
+  const T* k;        // [B][N][H][qk_rows][32]
   const T* vt;       // [B][N][H*32][Np]
   const T* bias;     // [B][H][Np][Np], already times log2 e
   const float* mb;   // [B][N][Np], already times log2 e; -inf for padded keys
@@ -171,6 +171,8 @@ struct FlashParams {
   int64_t np;
   int64_t heads;
   int64_t rows;      // number of attention rows i (== n for the fused module)
+  int64_t qk_rows;   // q and k rows per head: np, zeros past n; or n (rows > 1 only), nothing read past them
+  float q_mul;
   int64_t o_stride_b;
   int64_t o_stride_row;
   int64_t o_stride_head;

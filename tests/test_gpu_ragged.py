@@ -82,19 +82,20 @@ def test_triattn_corner_of_a_masked_call(n, padded, starting):
     assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("rows,n", [(5, 40), (3, 100), (9, 150), (81, 300), (81, 330)])
-def test_triattn_core_redone_at_every_tile(rows, n):
-    """Scores of hundreds in log2 units send workgroups of both query tiles,
-    of odd and even block counts and of the half-empty last tile to the offset
-    kernel. The reference is float32 torch on the same bf16 values; the
+@pytest.mark.parametrize("mul", [1.0, 40.0])
+@pytest.mark.parametrize("rows,n", [(1, 100), (5, 1), (5, 40), (3, 100), (9, 150), (81, 300), (81, 330)])
+def test_triattn_core_at_every_tile(rows, n, mul):
+    """The core reads q and k unpadded. At mul = 40, scores of hundreds in
+    log2 units send workgroups of both query tiles, of odd and even block
+    counts and of the half-empty last tile to the offset kernel. The reference is float32 torch on the same bf16 values; the
     kernel's bf16 probabilities and output leave at most 2^-8 of the largest
     value each (2^-9 per rounding, sums of positive terms), 2e-2 as for every
     bf16 check."""
-    say(f"triattn core redo rows={rows} n={n}")
+    say(f"triattn core rows={rows} n={n} mul={mul}")
     g = torch.Generator(device="cuda")
     g.manual_seed(n)
     q, k, v = (torch.randn(1, rows, 4, n, 32, generator=g, device="cuda").bfloat16() for _ in range(3))
-    q = (q.float() * 40.0).bfloat16()
+    q = (q.float() * mul).bfloat16()
     tb = torch.randn(1, 1, 4, n, n, generator=g, device="cuda").bfloat16()
     keep = torch.rand(1, rows, n, generator=g, device="cuda") > 0.2
     keep[..., 0] = True
