@@ -897,7 +897,7 @@ int transition_generic_run(const fjx_transition_args* a, hipStream_t st) {
 
 // ------------------------------------------------ single-track attention
 struct SingleWs {
-  size_t s_ln, qkvg, q, k, vt, bias, mb, o, go, total;
+  size_t s_ln, qkvg, q, k, vt, bias, mb, go, total;
 };
 SingleWs single_ws(int64_t batch, int64_t n, int64_t c_s, int64_t heads, int32_t dtype) {
   const int64_t np = round64(n);
@@ -916,7 +916,6 @@ SingleWs single_ws(int64_t batch, int64_t n, int64_t c_s, int64_t heads, int32_t
   w.vt = take((size_t)batch * heads * np * 32 * es);
   w.bias = take((size_t)batch * heads * np * np * es);
   w.mb = take((size_t)batch * np * sizeof(float));
-  w.o = take((size_t)batch * n * heads * 32 * es);
   w.go = take((size_t)batch * n * c_s * es);
   w.total = off;
   return w;
@@ -962,8 +961,8 @@ int single_run(const fjx_single_attention_args* a, hipStream_t st) {
       launch_gemm<T, T>(g, st);
     }
     launch_split_heads<T>(qkvg, 4 * cs, B, n, np, (int)H, dh, (1.0f / sqrtf((float)dh)) * kLog2e,
-                          at<T>(W, ws.q), at<T>(W, ws.k), at<T>(W, ws.vt), st);
-    launch_key_mask<T>(static_cast<const T*>(a->mask), at<float>(W, ws.mb), B, n, np, a->inf, st);
+                          at<T>(W, ws.q), at<T>(W, ws.k), at<T>(W, ws.vt), static_cast<const T*>(a->mask),
+                          at<float>(W, ws.mb), a->inf, st);
   });
   if (rc) return rc;
   if (!a->pair_bias || a->extra_bias) {
@@ -988,24 +987,21 @@ int single_run(const fjx_single_attention_args* a, hipStream_t st) {
   fp.vt = at<T>(W, ws.vt);
   fp.bias = a->pair_bias && !a->extra_bias ? static_cast<const T*>(a->pair_bias) : at<T>(W, ws.bias);
   fp.mb = at<float>(W, ws.mb);
-  fp.out = at<T>(W, ws.o);
+  fp.out = at<T>(W, ws.go);
   fp.n = n;
   fp.np = np;
   fp.heads = H;
   fp.rows = 1;
-  fp.o_stride_b = n * H * 32;
-  fp.o_stride_row = 0;
-  fp.o_stride_head = 32;
-  fp.o_stride_q = H * 32;
+  fp.gate = qkvg + 3 * cs;
+  fp.gate_ld = 4 * cs;
+  fp.gate_dh = dh;
   fp.bias_stride_b = H * np * np;
   rc = timed(K_SINGLE_FLASH, st, "single_flash", [&] { launch_flash<T>(fp, B, st); });
   if (rc) return rc;
 
   return timed(K_SINGLE_OUT, st, "single_out", [&] {
-    T* go = at<T>(W, ws.go);
-    launch_gate_unpad<T>(fp.out, qkvg + 3 * cs, 4 * cs, go, B * n, (int)H, dh, st);
     GemmParams<T, T> g = {};
-    g.a = go;
+    g.a = fp.out;
     g.b = static_cast<const T*>(a->o_weight);
     g.c = static_cast<T*>(a->out);
     g.m = B * n;

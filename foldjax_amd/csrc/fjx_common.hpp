@@ -144,6 +144,18 @@ __device__ __forceinline__ float quad_sum(float v) {
   return v;
 }
 
+// the sum over the 4 lanes {l % 16 + 16 g} of an MFMA fragment's row, on lane
+// swaps instead of ds_bpermute round trips; the same value in all 4
+__device__ __forceinline__ float group_sum(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const uint32_t a0 = a[0], a1 = a[1];
+  const uint32_t v = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, a0) + __builtin_bit_cast(float, a1));
+  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  const uint32_t b0 = b[0], b1 = b[1];
+  return __builtin_bit_cast(float, b0) + __builtin_bit_cast(float, b1);
+}
+
 // LayerNorm of one row of c <= 512 channels by one wave, lane l holding
 // channels 8 l .. 8 l + 7
 template <typename T>

@@ -181,6 +181,11 @@ struct FlashParams {
   // bf16, rows > 1: a flag per workgroup of the offset-free pass, written by
   // it (fjx_flash_pipe.hip) and read by the offset kernel (fjx_flash.hip)
   unsigned* fallback;
+  // rows == 1 only: out is [B][n][heads * gate_dh], the first gate_dh (<= 32)
+  // dims of each head times gate[B n][ld]'s same columns; null: o_stride_*
+  const T* gate;
+  int64_t gate_ld;
+  int gate_dh;
 };
 
 template <typename T>
@@ -214,7 +219,7 @@ template <typename T>
 void launch_layernorm_rows(const T* x, const T* w, const T* b, T* y, int64_t rows, int c, float eps, hipStream_t st);
 template <typename T>
 void launch_split_heads(const T* qkv, int64_t ld, int64_t batch, int64_t n, int64_t np, int heads, int dh,
-                        float q_mul, T* q, T* k, T* vt, hipStream_t st);
+                        float q_mul, T* q, T* k, T* vt, const T* mask, float* mb, float inf, hipStream_t st);
 // z (and its norm and weight) in TZ, the bias in T: the Boltz-2 single track
 // runs in fp32 over a bf16 pair tensor
 template <typename TZ, typename T>
@@ -227,11 +232,6 @@ void launch_add_extra_bias(const T* src, T* bias, const T* extra, int64_t sb, in
                            int64_t n, int64_t np, hipStream_t st);
 template <typename T>
 void launch_pair_bias_border(T* bias, int64_t planes, int64_t n, int64_t np, hipStream_t st);
-template <typename T>
-void launch_key_mask(const T* mask, float* mb, int64_t batch, int64_t n, int64_t np, float inf, hipStream_t st);
-template <typename T>
-void launch_gate_unpad(const T* o, const T* g, int64_t ldg, T* out, int64_t rows, int heads, int dh,
-                       hipStream_t st);
 template <typename T>
 void launch_flash(const FlashParams<T>& p, int64_t batch, hipStream_t st);
 // rows == 1, a bias per head: keys split over the waves of a workgroup

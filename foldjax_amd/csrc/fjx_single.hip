@@ -1,7 +1,7 @@
 // Single-track helpers for the attention with pair bias of a Pairformer block
 // (Boltz-2 attention_pair_bias_forward): row LayerNorm, head split into the
-// padded flash layout, the pair-bias projection LN(z) W_z^T, the key mask
-// bias and the gate-and-unpad step before the output projection.
+// padded flash layout with the key mask bias, and the pair-bias projection
+// LN(z) W_z^T.
 #include "fjx_common.hpp"
 #include "fjx_kernels.hpp"
 #include "fjx_tile.hpp"
@@ -58,10 +58,11 @@ __global__ __launch_bounds__(256) void layernorm_rows8_kernel(const T* __restric
 
 // qkv rows [B*N][ld] holding q | k | v (each heads*dh wide) ->
 //   q, k: [B][H][Np][32] (q times q_mul), vt: [B][H*32][Np]; zero padding in d and keys
+// and the key mask mb[b][k] = log2(e) * (1 - mask[b,k]) * (-inf_const), -inf for padded keys
 template <typename T>
 __global__ void split_heads_kernel(const T* __restrict__ qkv, int64_t ld, int64_t batch, int64_t n, int64_t np,
                                    int heads, int dh, float q_mul, T* __restrict__ q, T* __restrict__ k,
-                                   T* __restrict__ vt) {
+                                   T* __restrict__ vt, const T* __restrict__ mask, float* __restrict__ mb, float inf) {
   const int64_t total = batch * heads * np * 32;
   const int64_t hd = (int64_t)heads * dh;
   for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
@@ -80,37 +81,42 @@ __global__ void split_heads_kernel(const T* __restrict__ qkv, int64_t ld, int64_
     q[idx] = from_f32<T>(qv);
     k[idx] = from_f32<T>(kv);
     vt[((b * heads + h) * 32 + d) * np + s] = from_f32<T>(vv);
+    if (idx < batch * np) {
+      const int64_t mk = idx % np, bm = idx / np;
+      mb[idx] = mk < n ? (mask ? (1.0f - to_f32(mask[bm * n + mk])) * (-inf) * kLog2e : 0.f) : -INFINITY;
+    }
   }
 }
 
 // bias[b][h][q][k] = log2(e) * LN(z[b,q,k,:]) . w[h,:] over the padded
 // [np, np] grid, zeros outside [n, n] (the attention never reads
-// uninitialised memory next to a -inf key mask). Persistent 512-thread
-// workgroups over tiles of 128 keys of one query row: the LayerNormed tile
-// goes to LDS, wave w multiplies row tile w (16 keys) by the [heads][128]
-// weight, 16 heads per MFMA column tile, and each lane stores 4 consecutive
-// keys of one head. The next tile's z rows are loaded before the current one
-// is multiplied; the weight is held in registers when heads <= 16.
+// uninitialised memory next to a -inf key mask).
+//
+// Waves work alone, each walking 16-key tiles of a query row: the 4 lanes of a
+// key (16 apart) load its 128 channels as the MFMA fragments they are needed
+// as, LayerNorm them in registers and multiply by the [heads][128] weight, 16
+// heads per MFMA column tile; a lane stores 4 consecutive keys of one head.
+// No tile goes through LDS and no wave waits for another; the next tile's rows
+// are in flight meanwhile. Bound by HBM: 257 MB of z read and 67 MB of fp32
+// bias written at n = 1003 take 116 us with the tile LayerNormed into LDS by
+// the workgroup (two barriers a tile), 75 us so
+// (three waves per SIMD where z is bf16; two, 79 us).
 // z may be narrower than the bias (TZ = bf16, T = float: the fp32 single
 // track of Boltz-2 over a bf16 pair tensor); the LayerNorm runs in fp32 and
-// its output is stored in T, so the projection then runs at T's precision.
+// its output is rounded to T, so the projection then runs at T's precision.
 template <typename TZ, typename T>
-__global__ __launch_bounds__(512) void pair_bias_kernel(const TZ* __restrict__ z, const T* __restrict__ ln_w,
+__global__ __launch_bounds__(256, (sizeof(TZ) == 2 ? 3 : 2)) void pair_bias_kernel(const TZ* __restrict__ z, const T* __restrict__ ln_w,
                                                         const T* __restrict__ ln_b, const T* __restrict__ w,
                                                         T* __restrict__ bias, int64_t n, int64_t np, int heads,
                                                         float eps, int64_t ntiles) {
   using namespace tile;
-  __shared__ __attribute__((aligned(16))) T xs[kTP][kLd];
   __shared__ __attribute__((aligned(16))) LnAffine ln;
 
-  const int64_t ntx = (np + kTP - 1) / kTP;
-  const int t = threadIdx.x;
-  const int wave = t >> 6;
-  const int lane = t & 63;
+  const int lane = threadIdx.x & 63;
   const int li = lane & 15;
   const int lg = lane >> 4;
-  const int p = t >> 2;
   const int nht = (heads + 15) / 16;
+  stage_ln<T>(ln_w, ln_b, ln);
 
   auto load_heads = [&](int ht, typename Frag<T>::type (&wf)[4]) {
     const float zero[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -120,49 +126,65 @@ __global__ __launch_bounds__(512) void pair_bias_kernel(const TZ* __restrict__ z
   };
   typename Frag<T>::type w0[4];
   load_heads(0, w0);
-  stage_ln<T>(ln_w, ln_b, ln);
 
-  RowPart<TZ> xr;
-  auto fetch = [&](int64_t tile) {
-    const TileRS tl = tile_at(tile, ntx, np);
-    const int64_t kk = tl.s0 + p;
-    const bool valid = tl.r < n && kk < n;
-    load_row_part<TZ>(valid ? z + (((int64_t)tl.b * n + tl.r) * n + kk) * kC : nullptr, xr);
+  // tile -> (batch, query row, key tile), advanced by fixed carries
+  const int64_t kt_row = np / 16;
+  const int64_t nw = (int64_t)gridDim.x * 4;
+  int64_t tile = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  struct At {
+    int64_t b, r, k;
   };
-
-  int64_t tile = blockIdx.x;
-  if (tile < ntiles) fetch(tile);
-  __syncthreads();
-  for (; tile < ntiles; tile += gridDim.x) {
-    const TileRS tl = tile_at(tile, ntx, np);
-    const int nstore = (int)min<int64_t>(kTP, np - tl.s0);  // a multiple of 64
-    const int nreal = tl.r < n ? (int)max<int64_t>(0, min<int64_t>(kTP, n - tl.s0)) : 0;
-    ln_quad<TZ>(xr, ln, eps, &xs[p][0]);
-    __syncthreads();
-    if (tile + gridDim.x < ntiles) fetch(tile + gridDim.x);
-
-    const int p0 = 16 * wave + 4 * lg;  // this lane's 4 keys within the tile
-#pragma unroll 1
+  const At step = {nw / kt_row / np, nw / kt_row % np, nw % kt_row};
+  At cur = {tile / kt_row / np, tile / kt_row % np, tile % kt_row};
+  auto next = [&](const At& a) {
+    At o = {a.b + step.b, a.r + step.r, a.k + step.k};
+    if (o.k >= kt_row) {
+      o.k -= kt_row;
+      ++o.r;
+    }
+    if (o.r >= np) {
+      o.r -= np;
+      ++o.b;
+    }
+    return o;
+  };
+  RowPart<TZ> xr;
+  auto fetch = [&](const At& a) {
+    const int64_t kk = 16 * a.k + li;
+    const bool valid = a.r < n && kk < n;
+    load_row_part<TZ, true>(valid ? z + ((a.b * n + a.r) * n + kk) * kC : nullptr, xr);
+  };
+  if (tile < ntiles) fetch(cur);
+  __syncthreads();  // LayerNorm affine staged
+  for (; tile < ntiles; tile += nw) {
+    const bool some = cur.r < n && 16 * cur.k < n;  // wave-uniform
+    typename Frag<T>::type xf[4];
+    ln_frag<TZ, T>(xr, ln, eps, xf);
+    const At nxt = next(cur);
+    if (tile + nw < ntiles) fetch(nxt);
+    const int64_t p0 = 16 * cur.k + 4 * lg;  // this lane's 4 keys
+    T* dst = bias + ((cur.b * heads + li) * np + cur.r) * np + p0;
     for (int ht = 0; ht < nht; ++ht) {
-      typename Frag<T>::type wf[4];
-      if (ht == 0) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) wf[ks] = w0[ks];
-      } else {
-        load_heads(ht, wf);
-      }
       f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (some) {
+        typename Frag<T>::type wf[4];
+        if (ht == 0) {
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) mma(acc, load8(&xs[16 * wave + li][32 * ks + 8 * lg]), wf[ks]);
-      const int h = 16 * ht + li;
-      if (h < heads && p0 < nstore) {
+          for (int ks = 0; ks < 4; ++ks) wf[ks] = w0[ks];
+        } else {
+          load_heads(ht, wf);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) mma(acc, xf[ks], wf[ks]);
+      }
+      if (16 * ht + li < heads) {
         float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = p0 + q < nreal ? acc[q] * kLog2e : 0.f;
-        store4f(bias + (((int64_t)tl.b * heads + h) * np + tl.r) * np + tl.s0 + p0, v);
+        for (int q = 0; q < 4; ++q) v[q] = cur.r < n && p0 + q < n ? acc[q] * kLog2e : 0.f;
+        store4f(dst + 16 * ht * np * np, v);
       }
     }
-    __syncthreads();  // xs is free for the next tile
+    cur = nxt;
   }
 }
 
@@ -211,37 +233,6 @@ __global__ void add_extra_bias_kernel(const T* __restrict__ src, T* __restrict__
   }
 }
 
-// mb[b][k] = log2(e) * (1 - mask[b,k]) * (-inf_const), -inf for padded keys
-template <typename T>
-__global__ void key_mask_kernel(const T* __restrict__ mask, float* __restrict__ mb, int64_t batch, int64_t n,
-                                int64_t np, float inf) {
-  const int64_t total = batch * np;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t k = idx % np;
-    const int64_t b = idx / np;
-    float v = -INFINITY;
-    if (k < n) v = mask ? (1.0f - to_f32(mask[b * n + k])) * (-inf) * kLog2e : 0.f;
-    mb[idx] = v;
-  }
-}
-
-// out[r][h*dh + d] = g[r*ldg + h*dh + d] * o[r][h][d] (o rows padded to 32 per head)
-template <typename T>
-__global__ void gate_unpad_kernel(const T* __restrict__ o, const T* __restrict__ g, int64_t ldg, T* __restrict__ out,
-                                  int64_t rows, int heads, int dh) {
-  const int64_t hd = (int64_t)heads * dh;
-  const int64_t total = rows * hd;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = idx / hd;
-    const int64_t c = idx % hd;
-    const int64_t h = c / dh;
-    const int64_t d = c % dh;
-    out[idx] = from_f32<T>(to_f32(g[r * ldg + c]) * to_f32(o[(r * heads + h) * 32 + d]));
-  }
-}
-
 dim3 grid_stride(int64_t total) {
   int64_t blocks = (total + 255) / 256;
   if (blocks > 65536) blocks = 65536;
@@ -263,17 +254,17 @@ void launch_layernorm_rows(const T* x, const T* w, const T* b, T* y, int64_t row
 }
 template <typename T>
 void launch_split_heads(const T* qkv, int64_t ld, int64_t batch, int64_t n, int64_t np, int heads, int dh,
-                        float q_mul, T* q, T* k, T* vt, hipStream_t st) {
+                        float q_mul, T* q, T* k, T* vt, const T* mask, float* mb, float inf, hipStream_t st) {
   hipLaunchKernelGGL(split_heads_kernel<T>, grid_stride(batch * heads * np * 32), dim3(256), 0, st, qkv, ld, batch, n,
-                     np, heads, dh, q_mul, q, k, vt);
+                     np, heads, dh, q_mul, q, k, vt, mask, mb, inf);
 }
 template <typename TZ, typename T>
 void launch_pair_bias(const TZ* z, const T* ln_w, const T* ln_b, const T* w, T* bias, int64_t batch, int64_t n,
                       int64_t np, int heads, float eps, hipStream_t st) {
-  const int64_t ntiles = (np + tile::kTP - 1) / tile::kTP * np * batch;
+  const int64_t ntiles = np / 16 * np * batch;
   const unsigned grid =
-      tile::persistent_grid(reinterpret_cast<const void*>(&pair_bias_kernel<TZ, T>), 512, ntiles);
-  hipLaunchKernelGGL((pair_bias_kernel<TZ, T>), dim3(grid), dim3(512), 0, st, z, ln_w, ln_b, w, bias, n, np, heads,
+      tile::persistent_grid(reinterpret_cast<const void*>(&pair_bias_kernel<TZ, T>), 256, (ntiles + 3) / 4);
+  hipLaunchKernelGGL((pair_bias_kernel<TZ, T>), dim3(grid), dim3(256), 0, st, z, ln_w, ln_b, w, bias, n, np, heads,
                      eps, ntiles);
 }
 template <typename T>
@@ -288,28 +279,15 @@ void launch_pair_bias_border(T* bias, int64_t planes, int64_t n, int64_t np, hip
   hipLaunchKernelGGL(pair_bias_border_kernel<T>, grid_stride(planes * (n * (np - n) + (np - n) * np)), dim3(256), 0,
                      st, bias, planes, n, np);
 }
-template <typename T>
-void launch_key_mask(const T* mask, float* mb, int64_t batch, int64_t n, int64_t np, float inf, hipStream_t st) {
-  hipLaunchKernelGGL(key_mask_kernel<T>, grid_stride(batch * np), dim3(256), 0, st, mask, mb, batch, n, np, inf);
-}
-template <typename T>
-void launch_gate_unpad(const T* o, const T* g, int64_t ldg, T* out, int64_t rows, int heads, int dh,
-                       hipStream_t st) {
-  hipLaunchKernelGGL(gate_unpad_kernel<T>, grid_stride(rows * heads * dh), dim3(256), 0, st, o, g, ldg, out, rows,
-                     heads, dh);
-}
-
 #define FJX_INST(T)                                                                                              \
   template void launch_layernorm_rows<T>(const T*, const T*, const T*, T*, int64_t, int, float, hipStream_t);   \
   template void launch_split_heads<T>(const T*, int64_t, int64_t, int64_t, int64_t, int, int, float, T*, T*, T*, \
-                                      hipStream_t);                                                              \
+                                      const T*, float*, float, hipStream_t);                                     \
   template void launch_pair_bias<T, T>(const T*, const T*, const T*, const T*, T*, int64_t, int64_t, int64_t, int, \
                                        float, hipStream_t);                                                      \
   template void launch_add_extra_bias<T>(const T*, T*, const T*, int64_t, int64_t, int64_t, int, int64_t, int64_t,  \
                                          hipStream_t);                                                           \
-  template void launch_pair_bias_border<T>(T*, int64_t, int64_t, int64_t, hipStream_t);                        \
-  template void launch_key_mask<T>(const T*, float*, int64_t, int64_t, int64_t, float, hipStream_t);             \
-  template void launch_gate_unpad<T>(const T*, const T*, int64_t, T*, int64_t, int, int, hipStream_t);
+  template void launch_pair_bias_border<T>(T*, int64_t, int64_t, int64_t, hipStream_t);
 FJX_INST(bf16)
 FJX_INST(float)
 #undef FJX_INST

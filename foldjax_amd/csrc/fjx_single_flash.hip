@@ -177,6 +177,16 @@ __device__ __forceinline__ void flash_single_body(const FlashParams<T>& P) {
   float y[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) y[e] = O[e] * inv;
+  if (P.gate) {
+    // the attention's own output, rounded to T, times the gate
+    const int dh = P.gate_dh;
+    const T* g = P.gate + (b * P.n + q) * P.gate_ld + h * dh + d0;
+    T* dst = P.out + (b * P.n + q) * (H * dh) + h * dh + d0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (d0 + e < dh) dst[e] = from_f32<T>(to_f32(g[e]) * round_to<T>(y[e]));
+    return;
+  }
   store4f(P.out + b * P.o_stride_b + q * P.o_stride_q + h * P.o_stride_head + d0, y);
 }
 

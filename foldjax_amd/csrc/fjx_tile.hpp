@@ -78,13 +78,18 @@ struct RowPart {
 // The 4 threads of a position hold interleaved 8-channel chunks: part j has
 // chunks j, 4+j, 8+j, 12+j (f[q] = channels 32q + 8j .. +7), so each of the
 // four 16-byte loads of the quad reads 64 contiguous bytes of the row.
-__device__ __forceinline__ int row_chunk(int q) { return 32 * q + 8 * (threadIdx.x & 3); }
+// kFrag: the 4 threads are the lanes l % 16 + 16 j of a wave instead, whose
+// chunks are the row's MFMA fragments.
+template <bool kFrag = false>
+__device__ __forceinline__ int row_chunk(int q) {
+  return 32 * q + 8 * (kFrag ? (threadIdx.x >> 4) & 3 : threadIdx.x & 3);
+}
 
-template <typename T>
+template <typename T, bool kFrag = false>
 __device__ __forceinline__ void load_row_part(const T* __restrict__ src, RowPart<T>& r) {
   if (src) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) r.f[q] = load8(src + row_chunk(q));
+    for (int q = 0; q < 4; ++q) r.f[q] = load8(src + row_chunk<kFrag>(q));
   } else {
     const float z[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -112,13 +117,18 @@ __device__ __forceinline__ void store_row_part(const RowPart<T>& r, T* __restric
 // cw < 128: the statistics are those of the first cw channels (the chunks
 // past cw hold zeros and are left out of the variance). kDot: bf16 rows
 // take their statistics on v_dot2_f32_bf16 (below) and the quad sums on
-// DPP; otherwise, and for fp32 rows, two passes over the unpacked values
-template <typename T, typename Put, int NB = 4, bool kDot = true>
+// DPP; otherwise, and for fp32 rows, two passes over the unpacked values.
+// kFrag as for row_chunk
+template <typename T, typename Put, int NB = 4, bool kDot = true, bool kFrag = false>
 __device__ __forceinline__ void ln_quad_put(const RowPart<T>& r, const LnAffine& l, float eps, Put put, int cw = kC) {
   float v[8 * NB];
 #pragma unroll
   for (int q = 0; q < NB; ++q) to_f32x8(r.f[q], v + 8 * q);
   const float inv_c = cw == kC ? 1.0f / kC : 1.0f / (float)cw;
+  auto sum4 = [](float x) {
+    if constexpr (kFrag) return group_sum(x);
+    else return quad_sum(x);
+  };
   float mean, var;
   if constexpr (kDot && std::is_same<T, bf16>::value) {
     // bf16 rows: the sum and the sum of squares straight from the packed
@@ -142,7 +152,7 @@ __device__ __forceinline__ void ln_quad_put(const RowPart<T>& r, const LnAffine&
         q2[e & 1] = __builtin_amdgcn_fdot2_f32_bf16(pr, pr, q2[e & 1], false);
       }
     }
-    const float st = quad_sum(s[0] + s[1]), qt = quad_sum(q2[0] + q2[1]);
+    const float st = sum4(s[0] + s[1]), qt = sum4(q2[0] + q2[1]);
     mean = st * inv_c;
     var = fmaxf(fmaf(-mean, mean, qt * inv_c), 0.f);
     // E[x^2] - mean^2 cancels when the mean dwarfs the spread; past a
@@ -155,13 +165,13 @@ __device__ __forceinline__ void ln_quad_put(const RowPart<T>& r, const LnAffine&
         const float d = v[e] - mean;
         if (cw == kC || 32 * (e / 8) < cw) q2b += d * d;
       }
-      var = quad_sum(q2b) * inv_c;
+      var = sum4(q2b) * inv_c;
     }
   } else {
     // the same sums whichever way the quad's lanes are combined (DPP or
     // ds_bpermute); the tri-mul prologue measured faster with the latter
-    auto qsum = [](float x) {
-      if constexpr (kDot) return quad_sum(x);
+    auto qsum = [&](float x) {
+      if constexpr (kDot) return sum4(x);
       x += shfl_xor(x, 1);
       return x + shfl_xor(x, 2);
     };
@@ -184,7 +194,7 @@ __device__ __forceinline__ void ln_quad_put(const RowPart<T>& r, const LnAffine&
     // one 8-channel chunk at a time: keeps the scheduler from hoisting all 16
     // affine reads (64 VGPRs) ahead of the arithmetic
     __builtin_amdgcn_sched_barrier(0);
-    const int c = row_chunk(q);
+    const int c = row_chunk<kFrag>(q);
     const f32x4 w0 = *reinterpret_cast<const f32x4*>(&l.w[c]);
     const f32x4 w1 = *reinterpret_cast<const f32x4*>(&l.w[c + 4]);
     const f32x4 b0 = *reinterpret_cast<const f32x4*>(&l.b[c]);
@@ -205,6 +215,16 @@ __device__ __forceinline__ void ln_quad(const RowPart<T>& r, const LnAffine& l, 
                                         int cw = kC) {
   auto put = [&](int c, const float* o) { store8(dst_row + c, pack8<TO>(o)); };
   ln_quad_put<T, decltype(put), NB, kDot>(r, l, eps, put, cw);
+}
+
+// ... kept as the 16-row tile's MFMA operand fragments in TO (a row's 4 lanes
+// are its lane groups, row_chunk<true>)
+template <typename T, typename TO>
+__device__ __forceinline__ void ln_frag(const RowPart<T>& r, const LnAffine& l, float eps,
+                                        typename Frag<TO>::type (&xf)[4]) {
+  int q = 0;
+  auto put = [&](int, const float* o) { xf[q++] = pack8<TO>(o); };
+  ln_quad_put<T, decltype(put), 4, true, true>(r, l, eps, put);
 }
 
 // One wave's 32 output channels col0..col0+31 of a [128][128] weight as MFMA

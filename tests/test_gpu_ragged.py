@@ -110,3 +110,36 @@ def test_triattn_core_at_every_tile(rows, n, mul):
     assert torch.isfinite(got.float()).all()
     err = (got.float() - want).norm() / want.norm()
     assert err <= 2e-2, float(err)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,heads,c_s", [(1, 16, 384), (17, 3, 24), (65, 16, 384), (130, 20, 320), (200, 32, 160)])
+def test_single_attention_head_widths(n, heads, c_s, dtype):
+    """The pair bias past one 16-head tile and at lengths that are no multiple
+    of 16, and the gated output of head widths 8, 24 and 5 and 16, against
+    float64 torch on the same values."""
+    say(f"single attention n={n} heads={heads} c_s={c_s} {dtype}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    lin = lambda o, i: (rnd(o, i) / i ** 0.5).to(dtype)  # noqa: E731
+    w = kernels.SingleAttentionWeights(
+        pre_norm_weight=(1 + 0.1 * rnd(c_s)).to(dtype), pre_norm_bias=(0.1 * rnd(c_s)).to(dtype),
+        z_norm_weight=(1 + 0.1 * rnd(128)).to(dtype), z_norm_bias=(0.1 * rnd(128)).to(dtype), z_weight=lin(heads, 128),
+        q_weight=lin(c_s, c_s), q_bias=(0.1 * rnd(c_s)).to(dtype), k_weight=lin(c_s, c_s), v_weight=lin(c_s, c_s),
+        g_weight=lin(c_s, c_s), o_weight=lin(c_s, c_s)).to(dtype, "cuda")
+    s, z = rnd(1, n, c_s).to(dtype), rnd(1, n, n, 128).bfloat16()
+    mask = (torch.arange(n, device="cuda") < max(1, n - 3)).to(dtype)[None]
+    got = kernels.single_attention(s, z, mask, w)
+    ln = lambda x, a, b: torch.nn.functional.layer_norm(x.double(), x.shape[-1:], a.double(), b.double())  # noqa: E731
+    mm = lambda x, m: x @ m.double().t().contiguous()  # noqa: E731
+    x = ln(s[0], w.pre_norm_weight, w.pre_norm_bias)
+    split = lambda t: t.reshape(n, heads, -1).permute(1, 0, 2).contiguous()  # noqa: E731
+    q, k, v = split(mm(x, w.q_weight) + w.q_bias.double()), split(mm(x, w.k_weight)), split(mm(x, w.v_weight))
+    sc = q @ k.transpose(1, 2).contiguous() * (c_s // heads) ** -0.5
+    sc = sc + mm(ln(z[0], w.z_norm_weight, w.z_norm_bias), w.z_weight).permute(2, 0, 1) + 1e6 * (mask[0].double() - 1)
+    o = (torch.softmax(sc, -1) @ v).permute(1, 0, 2).reshape(n, c_s)
+    want = mm(o * torch.sigmoid(mm(x, w.g_weight)), w.o_weight)
+    torch.cuda.synchronize()
+    err = float((got[0].double() - want).norm() / want.norm())
+    assert err <= (2e-5 if dtype == torch.float32 else 2e-2), err
