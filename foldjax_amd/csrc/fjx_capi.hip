@@ -213,19 +213,24 @@ dim3 grid_for(int64_t total) {
 // a, b and o of the tri-mul have rows `pitch` elements apart: N rounded up to
 // 64, so that at any N every row is whole cache lines (the LDS-DMA
 // contraction, 16-byte stores and loads), or N itself (tight) where a fixed
-// scratch does not hold that.
+// scratch does not hold that. split: fp32 a and b as three bf16 planes each,
+// `plane` elements apart (the fp32 path on the bf16 matrix cores).
 struct TriMulWs {
   size_t a, b, o, total;
-  int64_t pitch;
+  int64_t pitch, plane;
+  bool split;
 };
-TriMulWs trimul_ws(int64_t batch, int64_t n, int32_t dtype, bool tight = false) {
+TriMulWs trimul_ws(int64_t batch, int64_t n, int64_t c_z, int32_t dtype, bool tight = false) {
   TriMulWs w;
   w.pitch = tight ? n : round64(n);
-  const size_t per = align_up((size_t)batch * n * w.pitch * 128 * esize(dtype));
+  w.plane = batch * n * w.pitch * 128;
+  w.split = dtype == FJX_DTYPE_F32 && c_z == 128 && !tight;
+  const size_t per_o = align_up((size_t)w.plane * esize(dtype));
+  const size_t per_ab = w.split ? align_up((size_t)w.plane * 3 * sizeof(bf16)) : per_o;
   w.a = 0;
-  w.b = per;
-  w.o = 2 * per;
-  w.total = 3 * per;
+  w.b = per_ab;
+  w.o = 2 * per_ab;
+  w.total = w.o + per_o;
   return w;
 }
 
@@ -269,7 +274,7 @@ T* at(void* base, size_t off) {
 // ----------------------------------------------------------- tri-mul body
 template <typename T>
 int trimul_run(const fjx_trimul_args* a, bool tight, hipStream_t st) {
-  const TriMulWs ws = trimul_ws(a->batch, a->n, a->dtype, tight);
+  const TriMulWs ws = trimul_ws(a->batch, a->n, a->c_z, a->dtype, tight);
   T* abuf = at<T>(a->workspace, ws.a);
   T* bbuf = at<T>(a->workspace, ws.b);
   T* obuf = at<T>(a->workspace, ws.o);
@@ -290,13 +295,23 @@ int trimul_run(const fjx_trimul_args* a, bool tight, hipStream_t st) {
   pp.eps = a->eps;
   pp.transpose = a->direction == FJX_INCOMING;
   pp.cw = cw;
-  int rc = timed(K_TRIMUL_PROLOGUE, st, "trimul_prologue", [&] { launch_trimul_prologue<T>(pp, a->batch, st); });
+  int rc = timed(K_TRIMUL_PROLOGUE, st, "trimul_prologue", [&] {
+    if constexpr (std::is_same<T, float>::value) {
+      if (ws.split)
+        return launch_trimul_prologue_split(pp, at<bf16>(a->workspace, ws.a), at<bf16>(a->workspace, ws.b), ws.plane,
+                                            a->batch, st);
+    }
+    launch_trimul_prologue<T>(pp, a->batch, st);
+  });
   if (rc) return rc;
 
   bool o_blocked = false;  // the LDS-DMA contraction writes o tile-blocked for the epilogue
   rc = timed(K_TRIMUL_CONTRACT, st, "trimul_contract", [&] {
     if constexpr (std::is_same<T, bf16>::value) {
       o_blocked = launch_contract(abuf, bbuf, obuf, a->n, ws.pitch, a->batch * 128, st, true);
+    } else if (ws.split) {
+      launch_contract_split(at<bf16>(a->workspace, ws.a), at<bf16>(a->workspace, ws.b), obuf, a->n, ws.pitch, ws.plane,
+                            a->batch * 128, st);
     } else {
       GemmParams<T, T> cp = {};
       cp.a = abuf;
@@ -328,7 +343,12 @@ int trimul_run(const fjx_trimul_args* a, bool tight, hipStream_t st) {
   ep.n = a->n;
   ep.eps = a->eps;
   ep.cw = cw;
-  return timed(K_TRIMUL_EPILOGUE, st, "trimul_epilogue", [&] { launch_trimul_epilogue<T>(ep, a->batch, st); });
+  return timed(K_TRIMUL_EPILOGUE, st, "trimul_epilogue", [&] {
+    if constexpr (std::is_same<T, float>::value) {
+      if (ws.split) return launch_trimul_epilogue_split(ep, a->batch, st);
+    }
+    launch_trimul_epilogue<T>(ep, a->batch, st);
+  });
 }
 
 // ---------------------------------------------------------- tri-attn body
@@ -361,7 +381,12 @@ int triattn_run(const fjx_triattn_args* a, hipStream_t st) {
   pp.q_scale = (1.0f / sqrtf((float)a->head_dim)) * kLog2e;
   pp.transpose = a->starting ? 0 : 1;
   pp.cw = cw;
-  int rc = timed(K_TRIATTN_PROLOGUE, st, "triattn_prologue", [&] { launch_triattn_prologue<T>(pp, a->batch, st); });
+  int rc = timed(K_TRIATTN_PROLOGUE, st, "triattn_prologue", [&] {
+    if constexpr (std::is_same<T, float>::value) {
+      if (!cw) return launch_triattn_prologue_split(pp, a->batch, st);
+    }
+    launch_triattn_prologue<T>(pp, a->batch, st);
+  });
   if (rc) return rc;
 
   FlashParams<T> fp = {};
@@ -403,7 +428,12 @@ int triattn_run(const fjx_triattn_args* a, hipStream_t st) {
   ep.eps = a->eps;
   ep.transpose = pp.transpose;
   ep.cw = cw;
-  return timed(K_TRIATTN_EPILOGUE, st, "triattn_epilogue", [&] { launch_triattn_epilogue<T>(ep, a->batch, st); });
+  return timed(K_TRIATTN_EPILOGUE, st, "triattn_epilogue", [&] {
+    if constexpr (std::is_same<T, float>::value) {
+      if (!cw && ep.w_g) return launch_triattn_epilogue_split(ep, a->batch, st);
+    }
+    launch_triattn_epilogue<T>(ep, a->batch, st);
+  });
 }
 
 // q and k are copied (padded) only for one attention row
@@ -502,6 +532,9 @@ int transition_run(const fjx_transition_args* a, bool pb_fused, hipStream_t st) 
       launch_pair_bias_border<float>(p.pbf_out, planes, a->pb_n, p.pb_np, st);
     else if (pb_fused)
       launch_pair_bias_border<T>(p.pb_out, planes, a->pb_n, p.pb_np, st);
+    if constexpr (std::is_same<T, float>::value) {
+      if (a->c == 128) return launch_transition_split(p, st);
+    }
     launch_transition<T>(p, (int)a->c, st);
   });
 }
@@ -1064,7 +1097,7 @@ int fjx_abi_version(void) { return FJX_ABI_VERSION; }
 
 size_t fjx_trimul_workspace_size(int64_t batch, int64_t n, int64_t c_z, int64_t c_h, int32_t dtype) {
   if (batch < 1 || n < 1 || c_z < 1 || c_h < 1 || !dtype_ok(dtype)) return 0;
-  return fused_trimul(c_z, c_h) ? trimul_ws(batch, n, dtype).total : gen_trimul_ws(batch, n, c_z, c_h, dtype).total;
+  return fused_trimul(c_z, c_h) ? trimul_ws(batch, n, c_z, dtype).total : gen_trimul_ws(batch, n, c_z, c_h, dtype).total;
 }
 
 
@@ -1329,14 +1362,14 @@ __attribute__((visibility("hidden"))) int trimul_fwd_on_scratch(const fjx_trimul
   // refused by the size of the tight layout (rows of exactly n elements),
   // which is also what runs where the padded one does not fit
   const bool fused = fused_trimul(a->c_z, a->c_h);
-  const size_t need = fused ? trimul_ws(a->batch, a->n, a->dtype, true).total
+  const size_t need = fused ? trimul_ws(a->batch, a->n, a->c_z, a->dtype, true).total
                             : gen_trimul_ws(a->batch, a->n, a->c_z, a->c_h, a->dtype).total;
   if (need > FJX_NOALLOC_MAX_BYTES)
     return fail(FJX_ERR_WORKSPACE,
                 "%s: this shape needs %zu bytes of scratch, the library's static scratch holds %zu "
                 "(use fjx_trimul_fwd with a workspace)",
                 fn, need, (size_t)FJX_NOALLOC_MAX_BYTES);
-  const bool tight = fused && trimul_ws(a->batch, a->n, a->dtype).total > scratch_bytes;
+  const bool tight = fused && trimul_ws(a->batch, a->n, a->c_z, a->dtype).total > scratch_bytes;
   fjx_trimul_args b = *a;
   b.workspace = scratch;
   b.workspace_bytes = scratch_bytes;

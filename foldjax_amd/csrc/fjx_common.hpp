@@ -43,6 +43,42 @@ __device__ __forceinline__ void mma(f32x4& acc, const f32x8& a, const f32x8& b) 
   for (int e = 0; e < 8; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
 }
 
+// fp32 products on the bf16 matrix cores: x = h + m + l with h = bf16(x),
+// m = bf16(x - h), l = bf16(x - h - m), which leaves less than 2^-26 |x|, and
+//   x y = h h' + (h m' + m h') + (h l' + l h' + m m')
+// whose dropped terms are below 2^-25 |x y|: products as good as fp32's, six
+// 16-cycle v_mfma_f32_16x16x32_bf16 in place of eight 32-cycle
+// v_mfma_f32_16x16x4_f32 per 32 k. kInf: an infinite value keeps m = l = 0 (its
+// remainder is NaN); without it, an infinity gives NaN products, for operands
+// that are finite unless the result is lost anyway (LayerNormed activations,
+// weights).
+struct Split8 {
+  bf16x8 p[3];
+};
+template <bool kInf = false>
+__device__ __forceinline__ Split8 split8(const f32x8& x) {
+  constexpr float kBig = 3.3e38f;  // below the largest bf16
+  Split8 s;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    s.p[0][e] = static_cast<bf16>(x[e]);
+    const float h = static_cast<float>(s.p[0][e]);
+    const float r = kInf ? __builtin_amdgcn_fmed3f(x[e], -kBig, kBig) - __builtin_amdgcn_fmed3f(h, -kBig, kBig)
+                         : x[e] - h;
+    s.p[1][e] = static_cast<bf16>(r);
+    s.p[2][e] = static_cast<bf16>(r - static_cast<float>(s.p[1][e]));
+  }
+  return s;
+}
+__device__ __forceinline__ void mma(f32x4& acc, const Split8& a, const Split8& b) {
+  mma(acc, a.p[2], b.p[0]);
+  mma(acc, a.p[0], b.p[2]);
+  mma(acc, a.p[1], b.p[1]);
+  mma(acc, a.p[1], b.p[0]);
+  mma(acc, a.p[0], b.p[1]);
+  mma(acc, a.p[0], b.p[0]);
+}
+
 __device__ __forceinline__ float to_f32(float x) { return x; }
 __device__ __forceinline__ float to_f32(bf16 x) { return static_cast<float>(x); }
 

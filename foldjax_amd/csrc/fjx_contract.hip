@@ -573,6 +573,165 @@ static void launch_contract_dma(const bf16* a, const bf16* b, bf16* o, int64_t n
                      batches, blocked);
 }
 
+// ---------------------------------------------------------------------------
+// The contraction in fp32 on the bf16 matrix cores: a and b arrive as three
+// bf16 planes each (Split8, written so by the prologue: no conversion here),
+// `plane` elements apart, rows `pitch` apart as above; o is fp32. 128 x 128
+// output tiles, 512 threads (2 x 4 waves of 64 x 32), two stages of 32 k with
+// the six planes of the operands in 96 KB; six MFMAs per tile and 32 k.
+// Rows of 64 bytes: chunk c of row r in slot 4 r + (c ^ ((r / 4) % 4)), which
+// puts the 16 rows of a fragment on 16 bank groups. Wave w's DMA copies rows
+// 16 w .. 16 w + 15 of every plane: one lane offset serves all six. Walk,
+// tile hand-over and synchronisation as contract_dma_kernel.
+// 128 contractions of 245 x 245 x 245: 94 us on fp32 MFMAs (gemm_nt_kernel), 32
+// so.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(512) void contract_split_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
+                                                             float* __restrict__ O, int n, int pitch, int64_t plane,
+                                                             int64_t batches, bool blocked) {
+  constexpr int BT = 128, DK = 32;
+  constexpr int MI = 4, NJ = 2;  // 16-row and 16-column tiles per wave
+  constexpr int kStores = MI * NJ;
+  __shared__ __attribute__((aligned(16))) bf16 S[2][2][3][BT * DK];  // [stage][A, B][plane][128 rows x 32]
+
+  const int tpd = (n + BT - 1) / BT;
+  const int64_t total = batches * tpd * tpd;
+  const int64_t per_xcd = gridDim.x / kNumXcd;
+  const int64_t xcd = blockIdx.x % kNumXcd;
+  const int64_t hi = (xcd + 1) * total / kNumXcd;
+
+  const int t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int lane = t & 63;
+  const int li = lane & 15;
+  const int lg = lane >> 4;
+  const int wm = (wave >> 2) * 64;
+  const int wn = (wave & 3) * 32;
+  const int pb = 2 * pitch;
+
+  uint32_t voff = (uint32_t)((16 * wave + lane / 4) * pb + 16 * ((lane % 4) ^ ((lane / 16) & 3)));
+  struct Tile {
+    int64_t bat;
+    int m0, n0;
+  };
+  auto issue = [&](const Tile& tl, int kt, int st) {
+    asm volatile("" : "+v"(voff));
+    const bf16* base[2] = {A + (tl.bat * n + tl.m0) * pitch, B + (tl.bat * n + tl.n0) * pitch};
+    const int64_t bytes[2] = {(int64_t)(n - tl.m0) * pb, (int64_t)(n - tl.n0) * pb};
+#pragma unroll
+    for (int op = 0; op < 2; ++op)
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            crsrc(base[op] + u * plane, bytes[op]),
+            (__attribute__((address_space(3))) void*)(&S[st][op][u][16 * wave * DK]), 16, voff,
+            (uint32_t)(2 * DK * kt), 0, 0);
+  };
+  const int64_t tt = (int64_t)tpd * tpd;
+  const int64_t step_b = per_xcd / tt;
+  const int step_i = (int)((per_xcd % tt) / tpd), step_j = (int)(per_xcd % tpd);
+
+  const int ktiles = pitch / DK;  // even: the pitch is a multiple of 64
+  int64_t lid = xcd * total / kNumXcd + blockIdx.x / kNumXcd;
+  if (lid >= hi) return;
+  int64_t cb = lid / tt;
+  int ci = (int)((lid % tt) / tpd), cj = (int)(lid % tpd);
+  Tile cur = {cb, ci * BT, cj * BT};
+  issue(cur, 0, 0);
+  int pend = 0;  // the previous tile's stores may be in flight
+  for (;;) {
+    const int64_t next_lid = lid + per_xcd;
+    const bool has_next = next_lid < hi;
+    int64_t nb = cb + step_b;
+    int ni = ci + step_i, nj = cj + step_j;
+    if (nj >= tpd) {
+      nj -= tpd;
+      ++ni;
+    }
+    if (ni >= tpd) {
+      ni -= tpd;
+      ++nb;
+    }
+    const Tile nxt = {nb, ni * BT, nj * BT};
+
+    f32x4 acc[NJ][MI];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int i = 0; i < MI; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    for (int kb = 0; kb < ktiles; kb += 2) {
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        const int kt = kb + st;
+        if (st == 0 && pend) __builtin_amdgcn_s_waitcnt(0x0F70 | ((kStores >> 4) << 14) | (kStores & 15));
+        else __builtin_amdgcn_s_waitcnt(0xF70);
+        pend = 0;
+        opaque_sgpr(pend);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");  // no LDS read moves above the barrier
+        if (kt + 1 < ktiles) issue(cur, kt + 1, st ^ 1);
+        else if (has_next) issue(nxt, 0, 0);  // ktiles is even: st is 1 here
+        Split8 af[MI], bfr[NJ];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+#pragma unroll
+          for (int i = 0; i < MI; ++i) {
+            const int r = wm + 16 * i + li;
+            af[i].p[u] = load8(&S[st][0][u][8 * (4 * r + (lg ^ ((r >> 2) & 3)))]);
+          }
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) {
+            const int r = wn + 16 * j + li;
+            bfr[j].p[u] = load8(&S[st][1][u][8 * (4 * r + (lg ^ ((r >> 2) & 3)))]);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int i = 0; i < MI; ++i) mma(acc[j][i], bfr[j], af[i]);
+      }
+    }
+
+    int lrow = li, lcol = 4 * lg;
+    asm volatile("" : "+v"(lrow), "+v"(lcol));
+    // transposed accumulators: a lane holds 4 consecutive columns of a row;
+    // the wave's 32 columns are all within the pitch or none
+    const int c0 = cur.n0 + wn;
+    const int rstride = blocked ? pitch * tile::kC : pitch;
+    const float* Ob = blocked ? O + ((cur.bat >> 7) * n + cur.m0) * (int64_t)rstride + (int64_t)(c0 & ~63) * tile::kC +
+                                    (cur.bat & 127) * 64 + (c0 & 63)
+                              : O + (cur.bat * n + cur.m0) * (int64_t)rstride + c0;
+    const __amdgpu_buffer_rsrc_t ro = crsrc(Ob, c0 < pitch ? ((int64_t)(n - cur.m0 - 1) * rstride + 32) * 4 : 0);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const uint32_t off = (uint32_t)((wm + 16 * i + lrow) * rstride + lcol) * 4;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[j][i]), ro, off, 64 * j, 0);
+    }
+    if (!has_next) break;
+    lid = next_lid;
+    cb = nb;
+    ci = ni;
+    cj = nj;
+    cur = nxt;
+    pend = 1;
+    opaque_sgpr(pend);
+  }
+}
+
+void launch_contract_split(const bf16* a, const bf16* b, float* o, int64_t n, int64_t pitch, int64_t plane,
+                           int64_t batches, hipStream_t st) {
+  const int64_t tpd = (n + 127) / 128;
+  const int64_t total = batches * tpd * tpd;
+  const void* k = reinterpret_cast<const void*>(contract_split_kernel);
+  const int64_t cap = std::max<int64_t>(kNumXcd, tile::resident_blocks(k, 512) / kNumXcd * kNumXcd);
+  const int64_t grid = std::min<int64_t>(cap, (total + kNumXcd - 1) / kNumXcd * kNumXcd);
+  hipLaunchKernelGGL(contract_split_kernel, dim3((unsigned)grid), dim3(512), 0, st, a, b, o, (int)n, (int)pitch, plane,
+                     batches, true);
+}
+
 bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t pitch, int64_t batches, hipStream_t st,
                      bool blocked) {
   if (pitch % 64 == 0) {

@@ -211,8 +211,21 @@ bool gemm_dma_ok(const GemmParams<bf16, bf16>& p);
 // wrote the blocked layout
 bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t pitch, int64_t batches, hipStream_t st,
                      bool blocked = false);
+// the same in fp32 from bf16 planes (Split8) of a and b, `plane` elements
+// apart; pitch a multiple of 64, batches of 128, o tile-blocked
+void launch_contract_split(const bf16* a, const bf16* b, float* o, int64_t n, int64_t pitch, int64_t plane,
+                           int64_t batches, hipStream_t st);
 template <typename T>
 void launch_transition(const TransitionParams<T>& p, int c, hipStream_t st);
+// fp32 on the bf16 matrix cores (fjx_rowproj_f32.hip), c_z = 128: a and b of
+// the prologue as three bf16 planes `plane` elements apart, o tile-blocked
+void launch_trimul_prologue_split(const TriMulPrologueParams<float>& p, bf16* a, bf16* b, int64_t plane, int64_t batch,
+                                  hipStream_t st);
+void launch_trimul_epilogue_split(const TriMulEpilogueParams<float>& p, int64_t batch, hipStream_t st);
+void launch_triattn_prologue_split(const TriAttnPrologueParams<float>& p, int64_t batch, hipStream_t st);
+// gated only
+void launch_triattn_epilogue_split(const TriAttnEpilogueParams<float>& p, int64_t batch, hipStream_t st);
+void launch_transition_split(const TransitionParams<float>& p, hipStream_t st);
 
 // single-track helpers (fjx_single.hip)
 template <typename T>

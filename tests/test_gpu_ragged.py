@@ -143,3 +143,63 @@ def test_single_attention_head_widths(n, heads, c_s, dtype):
     torch.cuda.synchronize()
     err = float((got[0].double() - want).norm() / want.norm())
     assert err <= (2e-5 if dtype == torch.float32 else 2e-2), err
+
+
+@pytest.mark.parametrize("n,padded", [(1, 64), (63, 128), (65, 192), (127, 192), (129, 200)])
+@pytest.mark.parametrize("direction", ["outgoing", "incoming"])
+def test_trimul_fp32_corner_of_a_masked_call(n, padded, direction):
+    """As for bf16: the fp32 path's splits, its 64-position tiles and its
+    128-wide contraction tiles leave every valid position's arithmetic alone."""
+    say(f"ragged fp32 trimul n={n} in {padded} {direction}")
+    w = _weights(torch.float32)
+    z = _pair(padded, torch.float32)
+    tok = (torch.arange(padded, device="cuda") < n).float()
+    want = kernels.trimul(z, torch.outer(tok, tok)[None], w, direction, residual=z)[:, :n, :n]
+    zn = z[:, :n, :n].contiguous()
+    got = kernels.trimul(zn, None, w, direction, residual=zn)
+    torch.cuda.synchronize()
+    assert torch.isfinite(got).all()
+    assert torch.equal(got, want)
+
+
+def test_trimul_fp32_without_planes():
+    """The static scratch does not hold the split planes of 400 tokens: the
+    fp32 matrix instructions run instead, within the two paths' fp32 errors
+    (5e-7 of the result's norm each)."""
+    n = 400
+    say(f"trimul fp32 without planes n={n}")
+    w = _weights(torch.float32)
+    z = _pair(n, torch.float32)
+    want = kernels.trimul(z, None, w, "outgoing")
+    got = kernels.trimul(z, None, w, "outgoing", no_alloc=True)
+    torch.cuda.synchronize()
+    assert float((got - want).norm() / want.norm()) <= 2e-6
+
+
+@pytest.mark.parametrize("n", [1, 5, 8, 33])
+@pytest.mark.parametrize("heads", [1, 16])
+def test_transition_fp32_with_pair_bias(n, heads):
+    """The fp32 pair transition at row counts around its 64-row tile, with every
+    option and the pair bias, against float64 torch (fp32 products: 1e-5)."""
+    say(f"transition fp32 n={n} heads={heads}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    w = P.pack_transition_torch(P.transition_to_protenix(syn.transition_weights(seed=3)), torch.float32, "cuda")
+    aw = kernels.SingleAttentionWeights(
+        pre_norm_weight=None, pre_norm_bias=None, z_norm_weight=1 + 0.1 * rnd(128), z_norm_bias=0.1 * rnd(128),
+        z_weight=rnd(heads, 128), q_weight=rnd(32, 32), q_bias=None, k_weight=rnd(32, 32), v_weight=rnd(32, 32),
+        g_weight=rnd(32, 32), o_weight=rnd(32, 32))
+    x, res = rnd(2, n, n, 128), rnd(2, n, n, 128)
+    rm, om = (rnd(2, n, n) > 0).float() * 0.5, (rnd(2, n, n) > -1).float()
+    out, pb = kernels.transition(x, w, row_mask=rm, residual=res, out_mask=om, pair_bias_for=aw)
+    ln = lambda v, a, b: torch.nn.functional.layer_norm(v, (128,), a.double(), b.double())  # noqa: E731
+    mm = lambda v, m: v @ m.double().t().contiguous()  # noqa: E731
+    xn = ln(x.double(), w.norm_weight, w.norm_bias)
+    y = mm(torch.nn.functional.silu(mm(xn, w.w_a)) * mm(xn, w.w_b), w.w_o) * rm[..., None] + res
+    y = y * (om != 0)[..., None]
+    bias = mm(ln(out.double(), aw.z_norm_weight, aw.z_norm_bias), aw.z_weight).permute(0, 3, 1, 2) * 1.4426950408889634
+    torch.cuda.synchronize()
+    assert float((out.double() - y).norm() / y.norm()) <= 1e-5
+    assert float((pb[:, :, :n, :n].double() - bias).norm() / bias.norm()) <= 1e-5
+    assert not pb[:, :, n:].any() and not pb[..., n:].any()
