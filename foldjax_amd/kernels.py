@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass, fields
+from operator import attrgetter
 from typing import ClassVar
 
 import torch
@@ -40,7 +41,8 @@ def _dev(x: torch.Tensor) -> None:
 
 
 def _stream(x: torch.Tensor) -> int:
-    return torch.cuda.current_stream(x.device).cuda_stream
+    # torch.cuda.current_stream(x.device).cuda_stream without its Stream object
+    return torch._C._cuda_getCurrentRawStream(x.get_device())
 
 
 def _prep(t: torch.Tensor | None, dtype: torch.dtype, device) -> torch.Tensor | None:
@@ -59,15 +61,15 @@ def _same_device(x: torch.Tensor, **operands) -> None:
 
 
 def _need_shape(name: str, t: torch.Tensor | None, shape) -> None:
-    if t is not None and tuple(t.shape) != tuple(int(v) for v in shape):
+    if t is not None and t.shape != shape and tuple(t.shape) != tuple(int(v) for v in shape):
         raise ValueError(f"{name} must have shape {tuple(int(v) for v in shape)}, got {tuple(t.shape)}")
 
 
 def _rows_of(m: torch.Tensor | None, shape, dtype: torch.dtype, name: str) -> torch.Tensor | None:
     """A per-row (per-position) mask broadcast to ``shape`` in ``dtype``,
     contiguous, as the kernels index it."""
-    if m is None:
-        return None
+    if m is None or (m.shape == shape and m.dtype is dtype and m.is_contiguous()):
+        return m
     try:
         m = torch.broadcast_to(m, tuple(shape))
     except RuntimeError:
@@ -94,6 +96,11 @@ class TriMulWeights:
     def check(self, c_z: int) -> int:
         """Shapes against the pair width ``c_z``; returns ``c_h``."""
         c_h = int(self.norm_out_weight.shape[0])
+        in_, proj = (c_z,), (2 * c_h, c_z)
+        if (self.norm_in_weight.shape == in_ and self.norm_in_bias.shape == in_ and self.p_in_weight.shape == proj
+                and self.g_in_weight.shape == proj and self.norm_out_bias.shape == (c_h,)
+                and self.p_out_weight.shape == (c_z, c_h) and self.g_out_weight.shape == (c_z, c_z)):
+            return c_h
         for name, shape in (("norm_in_weight", (c_z,)), ("norm_in_bias", (c_z,)), ("p_in_weight", (2 * c_h, c_z)),
                             ("g_in_weight", (2 * c_h, c_z)), ("norm_out_bias", (c_h,)), ("p_out_weight", (c_z, c_h)),
                             ("g_out_weight", (c_z, c_z))):
@@ -126,6 +133,12 @@ class TriAttnWeights:
         hd = int(self.q_weight.shape[0])
         if hd % self.heads:
             raise ValueError(f"q projection width {hd} is not divisible by {self.heads} heads")
+        in_, proj = (c_z,), (hd, c_z)
+        if (self.norm_weight.shape == in_ and self.norm_bias.shape == in_
+                and self.bias_weight.shape == (self.heads, c_z) and self.q_weight.shape == proj
+                and self.k_weight.shape == proj and self.v_weight.shape == proj
+                and (self.g_weight is None or self.g_weight.shape == proj) and self.o_weight.shape == (c_z, hd)):
+            return hd
         for name, shape in (("norm_weight", (c_z,)), ("norm_bias", (c_z,)), ("bias_weight", (self.heads, c_z)),
                             ("q_weight", (hd, c_z)), ("k_weight", (hd, c_z)), ("v_weight", (hd, c_z)),
                             ("g_weight", (hd, c_z)), ("o_weight", (c_z, hd))):
@@ -151,6 +164,9 @@ class TransitionWeights:
     def check(self, c: int) -> int:
         """Shapes against the width ``c``; returns the hidden width."""
         hidden = int(self.w_a.shape[0])
+        if (self.norm_weight.shape == (c,) and self.norm_bias.shape == (c,) and self.w_a.shape == (hidden, c)
+                and self.w_b.shape == (hidden, c) and self.w_o.shape == (c, hidden)):
+            return hidden
         for name, shape in (("norm_weight", (c,)), ("norm_bias", (c,)), ("w_a", (hidden, c)), ("w_b", (hidden, c)),
                             ("w_o", (c, hidden))):
             _need_shape(f"transition weight {name}", getattr(self, name), shape)
@@ -196,13 +212,34 @@ class SingleAttentionWeights:
     def check(self, c_s: int, c_z: int | None) -> None:
         """Shapes against the single width ``c_s`` and (when z is read) the
         pair width ``c_z``."""
-        for name in ("q_weight", "k_weight", "v_weight", "g_weight", "o_weight"):
-            _need_shape(f"single attention weight {name}", getattr(self, name), (c_s, c_s))
+        sq = (c_s, c_s)
+        if not (self.q_weight.shape == sq and self.k_weight.shape == sq and self.v_weight.shape == sq
+                and self.g_weight.shape == sq and self.o_weight.shape == sq):
+            for name in ("q_weight", "k_weight", "v_weight", "g_weight", "o_weight"):
+                _need_shape(f"single attention weight {name}", getattr(self, name), sq)
         for name in ("q_bias", "pre_norm_weight", "pre_norm_bias"):
             _need_shape(f"single attention weight {name}", getattr(self, name), (c_s,))
         if c_z is not None:
             for name, shape in (("z_norm_weight", (c_z,)), ("z_norm_bias", (c_z,)), ("z_weight", (self.heads, c_z))):
                 _need_shape(f"single attention weight {name}", getattr(self, name), shape)
+
+
+# per packed weight class, a getter of every field as one tuple
+_TENSORS: dict = {}
+
+
+def _tensors(w) -> tuple:
+    get = _TENSORS.get(type(w))
+    if get is None:
+        get = _TENSORS[type(w)] = attrgetter(*(f.name for f in fields(w)))
+    return get(w)
+
+
+def _like(t: torch.Tensor | None, dtype: torch.dtype) -> torch.Tensor | None:
+    """``t`` in ``dtype`` and contiguous."""
+    if t is None or (t.dtype is dtype and t.is_contiguous()):
+        return t
+    return t.to(dtype=dtype).contiguous()
 
 
 def transition(
@@ -265,7 +302,7 @@ def transition(
         pb = torch.empty((rows // (pb_n * pb_n), pb_heads, np_, np_), dtype=pb_dtype, device=x.device)
     rm = _rows_of(row_mask, x.shape[:-1], x.dtype, "row_mask")
     om = _rows_of(out_mask, x.shape[:-1], x.dtype, "out_mask")
-    res = None if residual is None else residual.to(dtype=x.dtype).contiguous()
+    res = _like(residual, x.dtype)
     hidden = int(w.w_a.shape[0])
     ws_bytes = lib.fjx_transition_workspace_size(rows, c, hidden, _code(x.dtype))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
@@ -360,7 +397,7 @@ def single_attention(
     _dev(s)
     res = None
     if residual is not None:
-        res = (residual.unsqueeze(0) if squeeze else residual).to(dtype=s.dtype).contiguous()
+        res = _like(residual, s.dtype)
     lib = _lib.load()
     code = _code(s.dtype)
     if out is not None and out.data_ptr() == s.data_ptr() and (residual is None or residual.data_ptr() != s.data_ptr()):
@@ -392,18 +429,23 @@ def _out_buffer(out: torch.Tensor | None, x: torch.Tensor, flat: torch.Tensor) -
     the workgroup that writes a position reads it)."""
     if out is None:
         return torch.empty_like(flat)
-    if tuple(out.shape) != tuple(x.shape) or out.dtype != x.dtype or out.device != x.device:
+    if out.shape != x.shape or out.dtype != x.dtype or out.device != x.device:
         raise ValueError(f"out must be a {x.dtype} tensor of shape {tuple(x.shape)} on {x.device}, "
                          f"got {out.dtype} {tuple(out.shape)} on {out.device}")
     if not out.is_contiguous():
         raise ValueError("out must be contiguous")
-    return out.reshape(flat.shape)
+    return out if out.shape == flat.shape else out.reshape(flat.shape)
 
 
 def _flatten_pair(x: torch.Tensor, mask: torch.Tensor | None):
     if x.dim() < 3:
         raise ValueError(f"pair tensor must be [..., N, N, C], got shape {tuple(x.shape)}")
     _same_device(x, mask=mask)
+    if x.dim() == 4 and x.is_contiguous() and (mask is None or (mask.shape == x.shape[:3] and mask.dtype is x.dtype
+                                                                and mask.is_contiguous())):
+        batch, n, n2, c = x.shape
+        if n == n2:
+            return x, mask, (batch,), batch, n, c
     n, n2, c = x.shape[-3:]
     if n != n2:
         raise ValueError(f"pair tensor must be square in its two pair axes, got {tuple(x.shape)}")
@@ -453,7 +495,7 @@ def trimul(
     lib = _lib.load()
     code = _code(x.dtype)
     out = _out_buffer(out, x, xf)
-    res = None if residual is None else residual.to(dtype=x.dtype).contiguous().reshape(batch, n, n, c)
+    res = _like(residual, x.dtype)
     ws_bytes = 0 if no_alloc else lib.fjx_trimul_workspace_size(batch, n, c, c_h, code)
     ws = None if no_alloc else torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
     a = _lib.TriMulArgs(
@@ -471,7 +513,7 @@ def trimul(
     _check_weights(x, w)
     entry = lib.fjx_trimul_fwd_noalloc if no_alloc else lib.fjx_trimul_fwd
     _lib.check(entry(ctypes.byref(a), _stream(x)))
-    return out.reshape(tuple(lead) + (n, n, c))
+    return out if len(lead) == 1 else out.reshape(tuple(lead) + (n, n, c))
 
 
 def triattn(
@@ -499,7 +541,7 @@ def triattn(
     lib = _lib.load()
     code = _code(x.dtype)
     out = _out_buffer(out, x, xf)
-    res = None if residual is None else residual.to(dtype=x.dtype).contiguous().reshape(batch, n, n, c)
+    res = _like(residual, x.dtype)
     ws_bytes = lib.fjx_triattn_workspace_size(batch, n, c, heads, hd // heads, code)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
     a = _lib.TriAttnArgs(
@@ -514,7 +556,7 @@ def triattn(
     )
     _check_weights(x, w)
     _lib.check(lib.fjx_triattn_fwd(ctypes.byref(a), _stream(x)))
-    return out.reshape(tuple(lead) + (n, n, c))
+    return out if len(lead) == 1 else out.reshape(tuple(lead) + (n, n, c))
 
 
 def triattn_core(
@@ -577,12 +619,12 @@ def triattn_core(
 
 
 def _check_weights(x: torch.Tensor, w) -> None:
-    for f in fields(w):
-        t = getattr(w, f.name)
-        if t is None:
-            continue
-        if t.dtype != x.dtype or t.device != x.device or not t.is_contiguous():
+    """Every weight contiguous, in ``x``'s dtype and on its (cuda) device."""
+    dtype, dev = x.dtype, x.get_device()
+    for t in _tensors(w):
+        if t is not None and (t.dtype is not dtype or t.get_device() != dev or not t.is_contiguous()):
+            name = next(f.name for f in fields(w) if getattr(w, f.name) is t)
             raise ValueError(
-                f"weight {f.name} must be a contiguous {x.dtype} tensor on {x.device}; "
+                f"weight {name} must be a contiguous {x.dtype} tensor on {x.device}; "
                 "pack weights with .to(dtype, device) first"
             )

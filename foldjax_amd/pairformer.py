@@ -150,11 +150,13 @@ class PairformerLayerWeights:
         valid = None
         if pair_mask is not None:
             valid = torch.diagonal(pair_mask, dim1=-2, dim2=-1).ne(0)
+            if s is not None:
+                valid = valid.to(s.dtype)  # once for the attention's two masks and the transition's
         z = self.triangle.forward(z, pair_mask, out_mask=pair_mask, donate=donate)
         z, bias = self._pair_transition(z, s, out_mask=pair_mask)
         if self.attention is None:
             if s is not None and valid is not None:
-                s = s * valid.to(s.dtype)[..., None]
+                s = s * valid[..., None]
             return s, z
         if s is None:
             raise ValueError("PairformerBlock single path requires s")
