@@ -591,11 +591,14 @@ GemmParams<T, T> rows_gemm(const T* x, int64_t rows, int64_t k, const void* w, i
 }
 
 struct GenTriMulWs {
-  size_t xn, pg, acm, bcm, ocm, g2, wcat, total;
+  size_t xn, pg, acm, bcm, ocm, g2, total;
+  int64_t pitch;  // of the rows of a, b and o
 };
-GenTriMulWs gen_trimul_ws(int64_t batch, int64_t n, int64_t c_z, int64_t c_h, int32_t dtype) {
+GenTriMulWs gen_trimul_ws(int64_t batch, int64_t n, int64_t c_z, int64_t c_h, int32_t dtype, bool tight = false) {
   const size_t pos = (size_t)batch * n * n * esize(dtype);
   GenTriMulWs w;
+  w.pitch = tight ? n : round64(n);
+  const size_t planes = (size_t)batch * n * w.pitch * esize(dtype);
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
@@ -603,20 +606,25 @@ GenTriMulWs gen_trimul_ws(int64_t batch, int64_t n, int64_t c_z, int64_t c_h, in
     return at;
   };
   w.xn = take(pos * c_z);
-  w.pg = take(pos * 2 * c_h);  // G, then P = (x p_in^T) * G, then o position-major
-  w.acm = take(pos * c_h);     // a, then LN_out(o)
-  w.bcm = take(pos * c_h);
-  w.ocm = take(pos * c_h);
+  w.pg = take(pos * 2 * c_h);  // G, then P = (x p_in^T) * G where the planes do not come from the GEMM; LN_out(o)
+  w.acm = take(planes * c_h);
+  w.bcm = take(planes * c_h);
+  w.ocm = take(planes * c_h);
   w.g2 = take(pos * c_z);
-  w.wcat = take((size_t)4 * c_h * c_z * esize(dtype));  // p_in and g_in interleaved by 128 rows (the pair GEMM)
   w.total = off;
   return w;
 }
+// what fjx_trimul_fwd_noalloc holds a wide shape to: the tight layout and the
+// copy of the input weights that it once had
+size_t gen_trimul_noalloc_bytes(int64_t batch, int64_t n, int64_t c_z, int64_t c_h, int32_t dtype) {
+  return gen_trimul_ws(batch, n, c_z, c_h, dtype, true).total + align_up((size_t)4 * c_h * c_z * esize(dtype));
+}
 
 template <typename T>
-int trimul_generic_run(const fjx_trimul_args* a, hipStream_t st) {
+int trimul_generic_run(const fjx_trimul_args* a, bool tight, hipStream_t st) {
   const int64_t B = a->batch, n = a->n, nn = n * n, cz = a->c_z, ch = a->c_h, rows = B * nn;
-  const GenTriMulWs ws = gen_trimul_ws(B, n, cz, ch, a->dtype);
+  const GenTriMulWs ws = gen_trimul_ws(B, n, cz, ch, a->dtype, tight);
+  const int64_t pitch = ws.pitch;
   void* W = a->workspace;
   T* xn = at<T>(W, ws.xn);
   T* pg = at<T>(W, ws.pg);
@@ -630,45 +638,42 @@ int trimul_generic_run(const fjx_trimul_args* a, hipStream_t st) {
   int rc = timed(K_TRIMUL_PROLOGUE, st, "trimul_prologue", [&] {
     launch_ln_grid<T>(static_cast<const T*>(a->x), static_cast<const T*>(a->norm_in_weight),
                       static_cast<const T*>(a->norm_in_bias), xn, B, n, (int)cz, a->eps, 0, st);
-    bool fused = false;
     if constexpr (std::is_same<T, bf16>::value) {
-      // (x p_in^T) * sigmoid(x g_in^T) as one GEMM over the interleaved weights
-      T* wcat = at<T>(W, ws.wcat);
-      GemmParams<T, T> g = rows_gemm<T>(xn, rows, cz, wcat, 4 * ch, pg, 2 * ch);
+      // mask * (x p_in^T) * sigmoid(x g_in^T) as one GEMM over both weights,
+      // written as the contraction reads it
+      GemmParams<T, T> g = rows_gemm<T>(xn, B * n * pitch, cz, a->p_in_weight, 4 * ch, acm, 8);
+      g.b2 = static_cast<const T*>(a->g_in_weight);
       g.swiglu = 2;
-      if ((2 * ch) % 128 == 0 && gemm_dma_ok(g)) {
-        const size_t blk = (size_t)128 * cz * sizeof(T);
-        fused = hipMemcpy2DAsync(wcat, 2 * blk, a->p_in_weight, blk, blk, 2 * ch / 128, hipMemcpyDeviceToDevice,
-                                 st) == hipSuccess &&
-                hipMemcpy2DAsync(reinterpret_cast<char*>(wcat) + blk, 2 * blk, a->g_in_weight, blk, blk,
-                                 2 * ch / 128, hipMemcpyDeviceToDevice, st) == hipSuccess &&
-                launch_gemm_dma(g, st);
-      }
+      g.grid_n = n;
+      g.grid_pitch = pitch;
+      g.grid_units = ch;
+      g.grid_t = t;
+      g.grid_mask = mask;
+      g.c2 = bcm;
+      if (launch_gemm_dma(g, st)) return;
     }
-    if (!fused) {
-      GemmParams<T, T> g = rows_gemm<T>(xn, rows, cz, a->g_in_weight, 2 * ch, pg, 2 * ch);
-      g.act = 1;
-      launch_gemm<T, T>(g, st);
-      g = rows_gemm<T>(xn, rows, cz, a->p_in_weight, 2 * ch, pg, 2 * ch);
-      g.gate = pg;  // in place: each element reads its gate, then is overwritten
-      launch_gemm<T, T>(g, st);
-    }
-    launch_to_channel_major<T>(pg, 2 * ch, 0, (int)ch, mask, acm, B, n, t, st);
-    launch_to_channel_major<T>(pg, 2 * ch, (int)ch, (int)ch, mask, bcm, B, n, t, st);
+    GemmParams<T, T> g = rows_gemm<T>(xn, rows, cz, a->g_in_weight, 2 * ch, pg, 2 * ch);
+    g.act = 1;
+    launch_gemm<T, T>(g, st);
+    g = rows_gemm<T>(xn, rows, cz, a->p_in_weight, 2 * ch, pg, 2 * ch);
+    g.gate = pg;  // in place: each element reads its gate, then is overwritten
+    launch_gemm<T, T>(g, st);
+    launch_to_planes<T>(pg, 2 * ch, (int)ch, mask, acm, bcm, B, n, pitch, t, st);
   });
   if (rc) return rc;
 
+  bool blocked = false;
   rc = timed(K_TRIMUL_CONTRACT, st, "trimul_contract", [&] {
     if constexpr (std::is_same<T, bf16>::value) {
-      launch_contract(acm, bcm, ocm, n, n, B * ch, st);
+      blocked = launch_contract(acm, bcm, ocm, n, pitch, B * ch, st, true);
     } else {
       GemmParams<T, T> cp = {};
       cp.a = acm;
       cp.b = bcm;
       cp.c = ocm;
       cp.m = cp.n = cp.k = n;
-      cp.lda = cp.ldb = cp.ldc = n;
-      cp.sa = cp.sb = cp.sc = nn;
+      cp.lda = cp.ldb = cp.ldc = pitch;
+      cp.sa = cp.sb = cp.sc = n * pitch;
       cp.batches = B * ch;
       launch_gemm<T, T>(cp, st);
     }
@@ -676,13 +681,13 @@ int trimul_generic_run(const fjx_trimul_args* a, hipStream_t st) {
   if (rc) return rc;
 
   return timed(K_TRIMUL_EPILOGUE, st, "trimul_epilogue", [&] {
-    launch_to_position_major<T>(ocm, (int)ch, pg, B, nn, st);
-    launch_layernorm_rows<T>(pg, static_cast<const T*>(a->norm_out_weight), static_cast<const T*>(a->norm_out_bias),
-                             acm, rows, (int)ch, a->eps, st);
+    launch_planes_layernorm<T>(ocm, (int)ch, static_cast<const T*>(a->norm_out_weight),
+                               static_cast<const T*>(a->norm_out_bias), pg, pg + rows * ch, B, n, pitch, blocked,
+                               a->eps, st);
     GemmParams<T, T> g = rows_gemm<T>(xn, rows, cz, a->g_out_weight, cz, g2, cz);
     g.act = 1;
     launch_gemm<T, T>(g, st);
-    g = rows_gemm<T>(acm, rows, ch, a->p_out_weight, cz, static_cast<T*>(a->out), cz);
+    g = rows_gemm<T>(pg, rows, ch, a->p_out_weight, cz, static_cast<T*>(a->out), cz);
     g.gate = g2;
     g.residual = static_cast<const T*>(a->residual);
     g.row_gate = static_cast<const T*>(a->out_mask);
@@ -844,7 +849,7 @@ int transition_out_splits(int64_t rows, int64_t c, int64_t hidden, int32_t dtype
 }
 
 struct GenTransitionWs {
-  size_t xn, h, wcat, y, total;
+  size_t xn, h, y, total;
 };
 GenTransitionWs gen_transition_ws(int64_t rows, int64_t c, int64_t hidden, int32_t dtype) {
   const size_t es = esize(dtype);
@@ -857,7 +862,6 @@ GenTransitionWs gen_transition_ws(int64_t rows, int64_t c, int64_t hidden, int32
   };
   w.xn = take((size_t)rows * c * es);
   w.h = take((size_t)rows * hidden * es);
-  w.wcat = take((size_t)2 * hidden * c * es);  // W_a and W_b interleaved by 128 rows (the fused SwiGLU GEMM)
   // the output projection (each of its K splits), when its GEMM cannot apply the epilogue
   w.y = take((size_t)transition_out_splits(rows, c, hidden, dtype) * rows * c * es);
   w.total = off;
@@ -878,18 +882,11 @@ int transition_generic_run(const fjx_transition_args* a, hipStream_t st) {
                              static_cast<const T*>(a->norm_bias), xn, rows, (int)c, a->eps, st);
     bool fused = false;
     if constexpr (std::is_same<T, bf16>::value) {
-      // silu(x W_a^T) * (x W_b^T) as one GEMM over the interleaved weights
-      T* wcat = at<T>(W, ws.wcat);
-      GemmParams<T, T> g = rows_gemm<T>(xn, rows, c, wcat, 2 * hid, h, hid);
+      // silu(x W_a^T) * (x W_b^T) as one GEMM over both weights
+      GemmParams<T, T> g = rows_gemm<T>(xn, rows, c, a->w_a, 2 * hid, h, hid);
+      g.b2 = static_cast<const T*>(a->w_b);
       g.swiglu = 1;
-      if (hid % 128 == 0 && gemm_dma_ok(g)) {
-        const size_t blk = (size_t)128 * c * sizeof(T);  // one block of 128 weight rows
-        fused = hipMemcpy2DAsync(wcat, 2 * blk, a->w_a, blk, blk, hid / 128, hipMemcpyDeviceToDevice, st) ==
-                    hipSuccess &&
-                hipMemcpy2DAsync(reinterpret_cast<char*>(wcat) + blk, 2 * blk, a->w_b, blk, blk, hid / 128,
-                                 hipMemcpyDeviceToDevice, st) == hipSuccess &&
-                launch_gemm_dma(g, st);
-      }
+      fused = launch_gemm_dma(g, st);
     }
     if (!fused) {
       GemmParams<T, T> g = rows_gemm<T>(xn, rows, c, a->w_a, hid, h, hid);
@@ -1084,7 +1081,8 @@ int trimul_check(const fjx_trimul_args* a, const char* fn) {
 
 int trimul_dispatch(const fjx_trimul_args* a, bool tight, hipStream_t st) {
   if (!fused_trimul(a->c_z, a->c_h))
-    return a->dtype == FJX_DTYPE_BF16 ? trimul_generic_run<bf16>(a, st) : trimul_generic_run<float>(a, st);
+    return a->dtype == FJX_DTYPE_BF16 ? trimul_generic_run<bf16>(a, tight, st)
+                                      : trimul_generic_run<float>(a, tight, st);
   return a->dtype == FJX_DTYPE_BF16 ? trimul_run<bf16>(a, tight, st) : trimul_run<float>(a, tight, st);
 }
 
@@ -1363,13 +1361,15 @@ __attribute__((visibility("hidden"))) int trimul_fwd_on_scratch(const fjx_trimul
   // which is also what runs where the padded one does not fit
   const bool fused = fused_trimul(a->c_z, a->c_h);
   const size_t need = fused ? trimul_ws(a->batch, a->n, a->c_z, a->dtype, true).total
-                            : gen_trimul_ws(a->batch, a->n, a->c_z, a->c_h, a->dtype).total;
+                            : gen_trimul_noalloc_bytes(a->batch, a->n, a->c_z, a->c_h, a->dtype);
   if (need > FJX_NOALLOC_MAX_BYTES)
     return fail(FJX_ERR_WORKSPACE,
                 "%s: this shape needs %zu bytes of scratch, the library's static scratch holds %zu "
                 "(use fjx_trimul_fwd with a workspace)",
                 fn, need, (size_t)FJX_NOALLOC_MAX_BYTES);
-  const bool tight = fused && trimul_ws(a->batch, a->n, a->c_z, a->dtype).total > scratch_bytes;
+  const size_t padded = fused ? trimul_ws(a->batch, a->n, a->c_z, a->dtype).total
+                              : gen_trimul_ws(a->batch, a->n, a->c_z, a->c_h, a->dtype).total;
+  const bool tight = padded > scratch_bytes;
   fjx_trimul_args b = *a;
   b.workspace = scratch;
   b.workspace_bytes = scratch_bytes;

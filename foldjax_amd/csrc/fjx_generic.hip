@@ -71,70 +71,152 @@ __global__ __launch_bounds__(256) void ln_grid_kernel(const T* __restrict__ x, c
   }
 }
 
-// dst[b][c][v] = src[b][orig(v)][c0 + c] * mask[b][orig(v)] (c < C), through
-// 64 x 64 LDS tiles so that both sides move whole rows
+// a and b as planes (launch_to_planes), through LDS tiles of 64 columns of one
+// grid row x 64 channels, so that both sides move whole rows: 16-byte accesses
+// where the widths (vs) and the pitch (vd) allow, elements otherwise
 template <typename T>
-__global__ __launch_bounds__(256) void to_channel_major_kernel(const T* __restrict__ src, int64_t ld, int c0, int C,
-                                                               const T* __restrict__ mask, T* __restrict__ dst,
-                                                               int64_t n, int t) {
+__global__ __launch_bounds__(256) void to_planes_kernel(const T* __restrict__ src, int64_t ld, int C,
+                                                        const T* __restrict__ mask, T* __restrict__ A,
+                                                        T* __restrict__ B, int64_t n, int64_t pitch, int t, bool vs,
+                                                        bool vd) {
   __shared__ float tile[64][65];
-  const int64_t nn = n * n;
-  const int64_t vtiles = (nn + 63) / 64;
-  const int ctiles = (C + 63) / 64;
+  const int ctiles = (2 * C + 63) / 64;
+  const int64_t stiles = (pitch + 63) / 64;
   int64_t id = blockIdx.x;
-  const int ct = (int)(id % ctiles);
+  const int cb = (int)(id % ctiles) * 64;
   id /= ctiles;
-  const int64_t vt = id % vtiles;
-  const int64_t bb = id / vtiles;
-  const int64_t v0 = vt * 64;
-  const int cb = ct * 64;
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int pv = e >> 6, pc = e & 63;
-    const int64_t v = v0 + pv;
-    const int c = cb + pc;
-    float val = 0.f;
-    if (v < nn && c < C) {
-      const int64_t o = bb * nn + orig_pos(v, n, t);
-      val = to_f32(src[o * ld + c0 + c]);
-      if (mask) val *= to_f32(mask[o]);
+  const int64_t s0 = id % stiles * 64;
+  id /= stiles;
+  const int64_t r = id % n, bb = id / n;
+  const int tx = threadIdx.x;
+  if (vs) {
+    for (int e = tx; e < 512; e += 256) {
+      const int ps = e >> 3, c = cb + 8 * (e & 7);
+      const int64_t s = s0 + ps;
+      float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (s < n && c < 2 * C) {
+        const int64_t o = bb * n * n + (t ? s * n + r : r * n + s);
+        to_f32x8(load8(src + o * ld + c), v);
+        const float m = mask ? to_f32(mask[o]) : 1.f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] *= m;
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) tile[ps][8 * (e & 7) + k] = v[k];
     }
-    tile[pv][pc] = val;
+  } else {
+    for (int e = tx; e < 4096; e += 256) {
+      const int ps = e >> 6, c = cb + (e & 63);
+      const int64_t s = s0 + ps;
+      float v = 0.f;
+      if (s < n && c < 2 * C) {
+        const int64_t o = bb * n * n + (t ? s * n + r : r * n + s);
+        v = to_f32(src[o * ld + c]);
+        if (mask) v *= to_f32(mask[o]);
+      }
+      tile[ps][e & 63] = v;
+    }
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int pc = e >> 6, pv = e & 63;
-    const int64_t v = v0 + pv;
-    const int c = cb + pc;
-    if (v < nn && c < C) dst[(bb * C + c) * nn + v] = from_f32<T>(tile[pv][pc]);
+  auto row_of = [&](int c) { return (c < C ? A + (bb * C + c) * n * pitch : B + (bb * C + c - C) * n * pitch) + r * pitch; };
+  if (vd) {
+    for (int e = tx; e < 512; e += 256) {
+      const int pc = e >> 3, vv = 8 * (e & 7);
+      if (s0 + vv >= pitch || cb + pc >= 2 * C) continue;
+      float o8[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) o8[k] = tile[vv + k][pc];
+      store8(row_of(cb + pc) + s0 + vv, pack8<T>(o8));
+    }
+  } else {
+    for (int e = tx; e < 4096; e += 256) {
+      const int pc = e >> 6, ps = e & 63;
+      if (s0 + ps < pitch && cb + pc < 2 * C) row_of(cb + pc)[s0 + ps] = from_f32<T>(tile[ps][pc]);
+    }
   }
 }
 
-// dst[b][v][c] = src[b][c][v]
+// positions per tile of planes_layernorm_kernel: one 128-byte piece of a plane
 template <typename T>
-__global__ __launch_bounds__(256) void to_position_major_kernel(const T* __restrict__ src, int C, T* __restrict__ dst,
-                                                                int64_t nn) {
-  __shared__ float tile[64][65];
-  const int64_t vtiles = (nn + 63) / 64;
-  const int ctiles = (C + 63) / 64;
-  int64_t id = blockIdx.x;
-  const int ct = (int)(id % ctiles);
-  id /= ctiles;
-  const int64_t vt = id % vtiles;
-  const int64_t bb = id / vtiles;
-  const int64_t v0 = vt * 64;
-  const int cb = ct * 64;
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int pc = e >> 6, pv = e & 63;
-    const int64_t v = v0 + pv;
-    const int c = cb + pc;
-    tile[pc][pv] = (v < nn && c < C) ? to_f32(src[(bb * C + c) * nn + v]) : 0.f;
+constexpr int kLnCols = 128 / (int)sizeof(T);
+
+// position-major rows from planes, with the LayerNorm over the channels
+// (w null: none; channels blockIdx.y * 512 .. of more than 512). A workgroup
+// takes kLnCols columns of one grid row: the planes' 128-byte pieces go to LDS
+// as they are, chunk q (16 bytes) of channel c in slot q ^ (c / 8) % 8, so that
+// 8 lanes reading the same position of channels 8 apart hit different banks; a
+// position's channels are then in the registers of 8 lanes, 8 consecutive ones
+// each at a time, and leave as 16-byte stores.
+template <typename T>
+__global__ __launch_bounds__(256) void planes_layernorm_kernel(const T* __restrict__ src, int C,
+                                                               const T* __restrict__ w, const T* __restrict__ b,
+                                                               T* __restrict__ dst, int64_t n, int64_t pitch,
+                                                               bool blocked, bool vec, float eps) {
+  constexpr int PB = kLnCols<T>, E = 16 / (int)sizeof(T);  // columns per tile, elements per chunk
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  T* S = reinterpret_cast<T*>(smem);
+  const int64_t stiles = (n + PB - 1) / PB;
+  const int64_t s0 = blockIdx.x % stiles * PB;
+  const int64_t br = blockIdx.x / stiles, r = br % n, bb = br / n;
+  const int c0 = blockIdx.y * 512, cn = C - c0 < 512 ? C - c0 : 512;
+  // channel c of the item at (p / 128) gs + (p % 128) cs, p = item C + c
+  const int64_t cs = blocked ? 64 : n * pitch, gs = 128 * n * pitch;
+  const T* base = src + (blocked ? r * pitch * 128 + s0 / 64 * 64 * 128 + s0 % 64 : r * pitch + s0);
+  for (int e = threadIdx.x; e < cn * 8; e += 256) {
+    const int c = e >> 3, q = e & 7;
+    const int64_t p = bb * C + c0 + c;
+    const T* g = base + (p >> 7) * gs + (p & 127) * cs + q * E;
+    T* d = S + c * PB + (q ^ ((c >> 3) & 7)) * E;
+    if (vec) {
+      if (s0 + q * E < pitch) *reinterpret_cast<u32x4*>(d) = *reinterpret_cast<const u32x4*>(g);
+    } else {
+#pragma unroll
+      for (int k = 0; k < E; ++k) d[k] = s0 + q * E + k < n ? g[k] : from_f32<T>(0.f);
+    }
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int pv = e >> 6, pc = e & 63;
-    const int64_t v = v0 + pv;
-    const int c = cb + pc;
-    if (v < nn && c < C) dst[(bb * nn + v) * C + c] = from_f32<T>(tile[pc][pv]);
+  const int lane = threadIdx.x & 63, l8 = lane & 7;
+  for (int ps = (threadIdx.x >> 6) * 8 + (lane >> 3); ps < PB; ps += 32) {
+    float v[8][8], sum = 0.f;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int c = 64 * u + 8 * l8;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        v[u][k] = c < cn ? to_f32(S[(c + k) * PB + ((ps / E) ^ l8) * E + ps % E]) : 0.f;
+        sum += v[u][k];
+      }
+    }
+    float mean = 0.f, rstd = 1.f;
+    if (w) {
+#pragma unroll
+      for (int o = 4; o >= 1; o >>= 1) sum += shfl_xor(sum, o);
+      mean = sum / C;
+      float q2 = 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (64 * u + 8 * l8 < cn) q2 += (v[u][k] - mean) * (v[u][k] - mean);
+#pragma unroll
+      for (int o = 4; o >= 1; o >>= 1) q2 += shfl_xor(q2, o);
+      rstd = __builtin_amdgcn_rsqf(q2 / C + eps);
+    }
+    if (s0 + ps >= n) continue;
+    T* out = dst + ((bb * n + r) * n + s0 + ps) * C + c0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int c = 64 * u + 8 * l8;
+      if (c >= cn) continue;
+      if (w) {
+        float wv[8], bv[8];
+        to_f32x8(load8(w + c), wv);
+        to_f32x8(load8(b + c), bv);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[u][k] = (v[u][k] - mean) * rstd * wv[k] + bv[k];
+      }
+      store8(out + c, pack8<T>(v[u]));
+    }
   }
 }
 
@@ -287,91 +369,6 @@ __global__ void gate_rows8_kernel(T* __restrict__ o, const T* __restrict__ g, in
   }
 }
 
-// to_channel_major_kernel and to_position_major_kernel with 16-byte global
-// accesses (8 channels of a position, 8 positions of a channel per thread);
-// the float tile's 65-float rows keep both LDS phases conflict-free
-template <typename T>
-__global__ __launch_bounds__(256) void to_channel_major8_kernel(const T* __restrict__ src, int64_t ld, int c0, int C,
-                                                                const T* __restrict__ mask, T* __restrict__ dst,
-                                                                int64_t n, int t) {
-  __shared__ float tile[64][65];
-  const int64_t nn = n * n;
-  const int64_t vtiles = (nn + 63) / 64;
-  const int ctiles = (C + 63) / 64;
-  int64_t id = blockIdx.x;
-  const int ct = (int)(id % ctiles);
-  id /= ctiles;
-  const int64_t vt = id % vtiles;
-  const int64_t bb = id / vtiles;
-  const int64_t v0 = vt * 64;
-  const int cb = ct * 64;
-  for (int e = threadIdx.x; e < 512; e += 256) {
-    const int pv = e >> 3, cc = (e & 7) * 8;
-    const int64_t v = v0 + pv;
-    const int c = cb + cc;
-    float val[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (v < nn && c < C) {
-      const int64_t o = bb * nn + orig_pos(v, n, t);
-      to_f32x8(load8(src + o * ld + c0 + c), val);
-      if (mask) {
-        const float m = to_f32(mask[o]);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) val[k] *= m;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) tile[pv][cc + k] = val[k];
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < 512; e += 256) {
-    const int pc = e >> 3, vv = (e & 7) * 8;
-    const int64_t v = v0 + vv;
-    const int c = cb + pc;
-    if (v < nn && c < C) {
-      float o8[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) o8[k] = tile[vv + k][pc];
-      store8(dst + (bb * C + c) * nn + v, pack8<T>(o8));
-    }
-  }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void to_position_major8_kernel(const T* __restrict__ src, int C, T* __restrict__ dst,
-                                                                 int64_t nn) {
-  __shared__ float tile[64][65];
-  const int64_t vtiles = (nn + 63) / 64;
-  const int ctiles = (C + 63) / 64;
-  int64_t id = blockIdx.x;
-  const int ct = (int)(id % ctiles);
-  id /= ctiles;
-  const int64_t vt = id % vtiles;
-  const int64_t bb = id / vtiles;
-  const int64_t v0 = vt * 64;
-  const int cb = ct * 64;
-  for (int e = threadIdx.x; e < 512; e += 256) {
-    const int pc = e >> 3, vv = (e & 7) * 8;
-    const int64_t v = v0 + vv;
-    const int c = cb + pc;
-    float val[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (v < nn && c < C) to_f32x8(load8(src + (bb * C + c) * nn + v), val);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) tile[pc][vv + k] = val[k];
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < 512; e += 256) {
-    const int pv = e >> 3, cc = (e & 7) * 8;
-    const int64_t v = v0 + pv;
-    const int c = cb + cc;
-    if (v < nn && c < C) {
-      float o8[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) o8[k] = tile[cc + k][pv];
-      store8(dst + (bb * nn + v) * C + c, pack8<T>(o8));
-    }
-  }
-}
-
 // out[b][orig(v)][c] = (T(y[b][v][c] * m) + residual[b][orig(v)][c]) * (g != 0),
 // with m the row mask and g the output mask at the output position (1 without);
 // y the sum of `splits` partial products ss elements apart
@@ -446,23 +443,24 @@ void launch_ln_grid(const T* x, const T* w, const T* b, T* y, int64_t batch, int
                        eps, t);
 }
 template <typename T>
-void launch_to_channel_major(const T* src, int64_t ld, int c0, int C, const T* mask, T* dst, int64_t batch, int64_t n,
-                             int t, hipStream_t st) {
-  const int64_t blocks = batch * ((n * n + 63) / 64) * ((C + 63) / 64);
-  if (C % 8 == 0 && ld % 8 == 0 && c0 % 8 == 0 && (n * n) % 8 == 0 && al16(src) && al16(dst))
-    hipLaunchKernelGGL(to_channel_major8_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, src, ld, c0, C, mask,
-                       dst, n, t);
-  else
-    hipLaunchKernelGGL(to_channel_major_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, src, ld, c0, C, mask, dst,
-                       n, t);
+void launch_to_planes(const T* src, int64_t ld, int C, const T* mask, T* a, T* b, int64_t batch, int64_t n,
+                      int64_t pitch, int t, hipStream_t st) {
+  const int64_t blocks = batch * n * ((pitch + 63) / 64) * ((2 * C + 63) / 64);
+  const bool vs = C % 8 == 0 && ld % 8 == 0 && al16(src), vd = pitch % 8 == 0 && al16(a) && al16(b);
+  hipLaunchKernelGGL(to_planes_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, src, ld, C, mask, a, b, n, pitch,
+                     t, vs, vd);
 }
 template <typename T>
-void launch_to_position_major(const T* src, int C, T* dst, int64_t batch, int64_t nn, hipStream_t st) {
-  const int64_t blocks = batch * ((nn + 63) / 64) * ((C + 63) / 64);
-  if (C % 8 == 0 && nn % 8 == 0 && al16(src) && al16(dst))
-    hipLaunchKernelGGL(to_position_major8_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, src, C, dst, nn);
-  else
-    hipLaunchKernelGGL(to_position_major_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, src, C, dst, nn);
+void launch_planes_layernorm(const T* src, int C, const T* w, const T* b, T* dst, T* tmp, int64_t batch, int64_t n,
+                             int64_t pitch, bool blocked, float eps, hipStream_t st) {
+  // C is a multiple of 8 (checked at the entry point); a row of more than 512
+  // channels is moved 512 at a time and normalized afterwards
+  const bool fused = C <= 512;
+  const int64_t blocks = batch * n * ((n + kLnCols<T> - 1) / kLnCols<T>);
+  const size_t lds = (size_t)(C < 512 ? C : 512) * 128;
+  hipLaunchKernelGGL(planes_layernorm_kernel<T>, dim3((unsigned)blocks, (unsigned)((C + 511) / 512)), dim3(256), lds,
+                     st, src, C, fused ? w : nullptr, b, fused ? dst : tmp, n, pitch, blocked, pitch % 8 == 0 && al16(src), eps);
+  if (!fused) launch_layernorm_rows<T>(tmp, w, b, dst, batch * n * n, C, eps, st);
 }
 template <typename T>
 void launch_split_qk(const T* src, int64_t ld, int64_t c0, T* dst, int64_t rows, int64_t n, int64_t np, int heads,
@@ -514,9 +512,10 @@ void launch_scatter_add(const T* y, const T* row_mask, const T* residual, const 
 
 #define FJX_INST(T)                                                                                                \
   template void launch_ln_grid<T>(const T*, const T*, const T*, T*, int64_t, int64_t, int, float, int, hipStream_t); \
-  template void launch_to_channel_major<T>(const T*, int64_t, int, int, const T*, T*, int64_t, int64_t, int,        \
-                                           hipStream_t);                                                           \
-  template void launch_to_position_major<T>(const T*, int, T*, int64_t, int64_t, hipStream_t);                    \
+  template void launch_to_planes<T>(const T*, int64_t, int, const T*, T*, T*, int64_t, int64_t, int64_t, int,        \
+                                    hipStream_t);                                                                   \
+  template void launch_planes_layernorm<T>(const T*, int, const T*, const T*, T*, T*, int64_t, int64_t, int64_t,   \
+                                           bool, float, hipStream_t);                                                     \
   template void launch_split_qk<T>(const T*, int64_t, int64_t, T*, int64_t, int64_t, int64_t, int, float,           \
                                    hipStream_t);                                                                   \
   template void launch_split_vt<T>(const T*, int64_t, int64_t, T*, int64_t, int64_t, int64_t, int, hipStream_t);   \

@@ -114,12 +114,22 @@ struct GemmParams {
   // r = b N^2 + i N + j goes to b N^2 + j N + i (the ending node's grid)
   int map_t;
   int64_t map_n;
-  // pair mode (launch_gemm_dma only): B holds two weights interleaved in
-  // blocks of 128 rows (a block of the first, then the block of the second
-  // for the same 128 output units), n = 2 units, and C[i][u] combines a and b
-  // (both rounded to TO first): 1 = silu(a) * b (SwiGLU), 2 = a * sigmoid(b)
-  // (a gated projection); C has `units` columns
+  // pair mode (launch_gemm_dma only): b and b2 are two weights of `units`
+  // rows, n = 2 units, and C[i][u] combines a = A b^T and b = A b2^T (both
+  // rounded to TO first): 1 = silu(a) * b (SwiGLU), 2 = a * sigmoid(b) (a gated
+  // projection); C has `units` columns
   int swiglu;
+  const T* b2;
+  // with swiglu 2 and grid_pitch > 0: the product goes out channel by channel,
+  // the layout of the triangle contraction. A is a pair grid [item][grid_n]
+  // [grid_n] of rows, m counts the rows of the padded grid [item][r][grid_pitch],
+  // whose column s of row r is A's position (r, s), or (s, r) with grid_t. Unit
+  // u times the position's mask goes to c, or from grid_units on to c2, at
+  // [item][u % grid_units][r][s]; zeros past grid_n
+  int64_t grid_n, grid_pitch, grid_units;
+  int grid_t;
+  const T* grid_mask;  // [item][grid_n][grid_n] or null
+  TO* c2;
 };
 
 template <typename T>
@@ -264,11 +274,18 @@ int probe_hbm_stream(int mode, int wgs_per_cu, int64_t bytes, float* ms, hipStre
 template <typename T>
 void launch_ln_grid(const T* x, const T* w, const T* b, T* y, int64_t batch, int64_t n, int c, float eps, int t,
                     hipStream_t st);
+// a and b of a triangle product, channel by channel with rows `pitch` apart:
+// dst[item][c][r][s] = src[item][(r, s) or, with t, (s, r)][c] * mask, zeros for
+// n <= s < pitch; channels 0 .. C-1 go to a, C .. 2C-1 to b
 template <typename T>
-void launch_to_channel_major(const T* src, int64_t ld, int c0, int C, const T* mask, T* dst, int64_t batch, int64_t n,
-                             int t, hipStream_t st);
+void launch_to_planes(const T* src, int64_t ld, int C, const T* mask, T* a, T* b, int64_t batch, int64_t n,
+                      int64_t pitch, int t, hipStream_t st);
+// dst[item][(r, s)][c] = LayerNorm over c of the planes [item][c][r][pitch], or
+// with `blocked` [128 planes][r][64-column block][plane][64]; tmp: as large as
+// dst, used from 513 channels on
 template <typename T>
-void launch_to_position_major(const T* src, int C, T* dst, int64_t batch, int64_t nn, hipStream_t st);
+void launch_planes_layernorm(const T* src, int C, const T* w, const T* b, T* dst, T* tmp, int64_t batch, int64_t n,
+                             int64_t pitch, bool blocked, float eps, hipStream_t st);
 template <typename T>
 void launch_split_qk(const T* src, int64_t ld, int64_t c0, T* dst, int64_t rows, int64_t n, int64_t np, int heads,
                      float mul, hipStream_t st);

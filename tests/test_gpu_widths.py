@@ -16,7 +16,7 @@ import numpy as np
 import pytest
 import torch
 
-from foldjax_amd import kernels, protenix
+from foldjax_amd import _lib, kernels, protenix
 from foldjax_amd import params as P
 from foldjax_amd import synthetic as syn
 from oracle import triangle as O
@@ -316,3 +316,66 @@ def test_general_triattn_weights_back_to_back_match_separate(starting):
     b = kernels.triattn(z, m, b2b, starting=starting, residual=z)
     torch.cuda.synchronize()
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("direction", ["outgoing", "incoming"])
+@pytest.mark.parametrize("dt,c_z,c_h,n,batch", [
+    ("bf16", 384, 384, 65, 3),    # planes from the GEMM, 256-wide tiles, rows half padding
+    ("bf16", 384, 384, 90, 1),    # 128-wide tiles, a short last row tile
+    ("bf16", 264, 192, 127, 1),   # a k tail of 8, planes past one and a half blocks of 128
+    ("bf16", 128, 64, 129, 2),    # 128 planes over two items
+    ("bf16", 256, 576, 64, 1),    # more channels than one LayerNorm tile
+    ("bf16", 384, 72, 63, 1),     # a width the paired GEMM does not take
+    ("fp32", 264, 72, 33, 2), ("fp32", 128, 520, 17, 1),
+])
+def test_trimul_wide_planes(dt, c_z, c_h, n, batch, direction):
+    """The general tri-mul's layouts (operands channel by channel with padded
+    rows, from the gated product or a pass of its own, and the LayerNorm back
+    to positions) at widths and lengths off every tile, against the oracle."""
+    dtype = DTYPES[dt]
+    say(f"trimul wide planes c_z={c_z} c_h={c_h} n={n} batch={batch} {dt} {direction}")
+    z = np.stack([syn.pair_input(n, c_z, seed=81 + b) for b in range(batch)])
+    m = np.stack([mask_case("random", n) for _ in range(batch)])
+    w = syn.trimul_weights(c_z, c_h, seed=82)
+    got = protenix.triangle_multiplication(device_tensor(z, dtype), device_tensor(m, dtype),
+                                           P.trimul_to_protenix(w), direction)
+    torch.cuda.synchronize()
+    want = np.stack([O.protenix_triangle_multiplication(prep(z[b], dtype), prep(m[b], dtype), prep_tree(w, dtype),
+                                                        direction) for b in range(batch)])
+    assert_parity(to_np(got), want, dtype, f"trimul c_z={c_z} c_h={c_h} n={n} {direction}")
+
+
+@pytest.mark.parametrize("direction", ["outgoing", "incoming"])
+def test_trimul_wide_without_row_padding(direction):
+    """Eleven 65-token items of 384 channels: their scratch fits the static one
+    on rows of exactly n elements only, against the oracle."""
+    dtype, c, n, batch = DTYPES["bf16"], 384, 65, 11
+    say(f"trimul wide unpadded rows {direction}")
+    lib = _lib.load()
+    assert lib.fjx_trimul_workspace_size(batch, n, c, c, _lib.FJX_DTYPE_BF16) > _lib.NOALLOC_SCRATCH_BYTES
+    z = np.stack([syn.pair_input(n, c, seed=91 + b) for b in range(batch)])
+    m = mask_case("tail", n)
+    w = syn.trimul_weights(c, c, seed=92)
+    tw = P.pack_trimul_torch(P.trimul_to_protenix(w), dtype, "cuda")
+    mt = device_tensor(np.stack([m] * batch), dtype)
+    got = kernels.trimul(device_tensor(z, dtype), mt, tw, direction, no_alloc=True)
+    torch.cuda.synchronize()
+    for b in (0, batch - 1):
+        want = O.protenix_triangle_multiplication(prep(z[b], dtype), prep(m, dtype), prep_tree(w, dtype), direction)
+        assert_parity(to_np(got)[b], want, dtype, f"trimul unpadded rows item {b}")
+
+
+@pytest.mark.parametrize("c,rows", [(384, 16500), (264, 33000)])
+def test_transition_wide_256_wide_tiles_bf16(c, rows):
+    """Row counts at which the paired GEMM takes its 256-wide tiles (the
+    counts above take the 128-wide ones), ending off a tile."""
+    dtype = DTYPES["bf16"]
+    say(f"transition 256-wide tiles c={c} rows={rows}")
+    x = np.random.default_rng(c).standard_normal((rows, c)).astype(np.float32)
+    w = syn.transition_weights(c, 4, seed=23)
+    tw = P.pack_transition_torch({k: w[k] for k in ("layer_norm", "linear_a", "linear_b", "linear_out")}, dtype, "cuda")
+    got = kernels.transition(device_tensor(x, dtype), tw)
+    torch.cuda.synchronize()
+    pick = np.r_[0:300, rows - 300:rows]
+    want = O.transition(prep(x[pick], dtype), prep_tree(w, dtype), mask=None)
+    assert_parity(to_np(got)[pick], want, dtype, f"transition c={c} rows={rows}")
