@@ -66,15 +66,15 @@ namespace {
 // belong to this one workgroup and would otherwise run the VALU-only
 // LayerNorm and the MFMA phase in lockstep, one after the other.
 // ---------------------------------------------------------------------------
-template <typename T, bool kNarrow, int NB = 4>
+template <typename T, bool kNarrow, int NB = 4, int TP = kTP>
 __global__ __launch_bounds__(512) void trimul_prologue_kernel(TriMulPrologueParams<T> P, int64_t ntiles) {
-  __shared__ __attribute__((aligned(16))) T xs[2][kTP][kLd];
-  __shared__ __attribute__((aligned(16))) float mrow[2][kTP];
+  __shared__ __attribute__((aligned(16))) T xs[2][TP][kLd];
+  __shared__ __attribute__((aligned(16))) float mrow[2][TP];
   __shared__ __attribute__((aligned(16))) LnAffine ln;
 
   const int64_t n = P.n;
   const int64_t nn = n * n;
-  const int64_t ntx = (n + kTP - 1) / kTP;
+  const int64_t ntx = (n + TP - 1) / TP;
   const int t = threadIdx.x;
   const int wave = t >> 6;
   const int lane = t & 63;
@@ -105,9 +105,9 @@ __global__ __launch_bounds__(512) void trimul_prologue_kernel(TriMulProloguePara
   T mraw = from_f32<T>(0.f);
   bool mvalid = false;
   auto fetch = [&](int64_t tile) {
-    const TileRS tl = tile_at(tile, ntx, n);
+    const TileRS tl = tile_at(tile, ntx, n, TP);
     const int s = tl.s0 + p;
-    const bool valid = s < n;
+    const bool valid = p < TP && s < n;
     auto pos_of = [&](int ss) {
       return (int64_t)tl.b * nn + (P.transpose ? (int64_t)ss * n + tl.r : (int64_t)tl.r * n + ss);
     };
@@ -123,6 +123,7 @@ __global__ __launch_bounds__(512) void trimul_prologue_kernel(TriMulProloguePara
   auto ln_tile = [&](int buf) {
     // two-pass statistics: the dot2 form measured 8 % slower here, where
     // this LayerNorm runs between the current tile's MFMA phases
+    if (p >= TP) return;
     ln_quad<T, T, NB, false>(xr, ln, P.eps, &xs[buf][p][0], cw);
     if ((t & 3) == 0) mrow[buf][p] = mvalid ? (P.mask ? to_f32(mraw) : 1.0f) : 0.f;
   };
@@ -132,9 +133,9 @@ __global__ __launch_bounds__(512) void trimul_prologue_kernel(TriMulProloguePara
   }
   __syncthreads();
   for (int cur = 0; tile < ntiles; tile += gridDim.x, cur ^= 1) {
-    const TileRS tl = tile_at(tile, ntx, n);
+    const TileRS tl = tile_at(tile, ntx, n, TP);
     // columns stored: up to the pitch, the ones past n zero (mrow is 0 there)
-    const int nstore = (int)min<int64_t>(kTP, pitch - tl.s0);
+    const int nstore = (int)min<int64_t>(TP, pitch - tl.s0);
     T* dst = (half == 0 ? P.a_cm : P.b_cm) + (int64_t)tl.b * kC * plane + (int64_t)tl.r * pitch + tl.s0;
     auto pair = [&](int j) {
       f32x4 ap[2][2], ag[2][2];
@@ -155,14 +156,15 @@ __global__ __launch_bounds__(512) void trimul_prologue_kernel(TriMulProloguePara
         store8_masked<T>(dst + (int64_t)(col0 + 16 * ct + (lane & 15)) * plane + p0, v, nstore - p0, vec8, vec4);
       }
     };
-    pair(0);
-    pair(1);
+#pragma unroll
+    for (int j = 0; j < TP / 64; ++j) pair(j);
     if (tile + gridDim.x < ntiles) {
       ln_tile(cur ^ 1);  // the next tile's LayerNorm, under this tile's MFMAs
       if (tile + 2 * gridDim.x < ntiles) fetch(tile + 2 * gridDim.x);
     }
-    pair(2);
-    pair(3);
+#pragma unroll
+    for (int j = TP / 64; j < TP / 32; ++j)
+      if (32 * j < nstore) pair(j);
     __syncthreads();  // the next tile's rows are in LDS; this tile's buffer is free
   }
 }
@@ -177,11 +179,11 @@ __global__ __launch_bounds__(512) void trimul_prologue_kernel(TriMulProloguePara
 //   bias [B][H][Np][Np]  x_ln w_bias^T times log2 e (in T)
 //   mb [B][N][Np] fp32   inf*(mask-1)*log2 e, -inf for keys >= N
 // Np = N rounded up to 64; key slots in [N, Np) are written as zeros.
-// kNarrow and NB: x has P.cw < 128 channels, as for the tri-mul prologue.
+// kNarrow, NB and TP as for the tri-mul prologue.
 // ---------------------------------------------------------------------------
-template <typename T, bool kNarrow, int NB = 4>
+template <typename T, bool kNarrow, int NB = 4, int TP = kTP>
 __global__ __launch_bounds__(512) void triattn_prologue_kernel(TriAttnPrologueParams<T> P, int64_t ntiles) {
-  __shared__ __attribute__((aligned(16))) T xs[kTP][kLd];
+  __shared__ __attribute__((aligned(16))) T xs[TP][kLd];
   __shared__ __attribute__((aligned(16))) LnAffine ln;
   constexpr int D = 32;
   constexpr int H = 4;
@@ -189,7 +191,7 @@ __global__ __launch_bounds__(512) void triattn_prologue_kernel(TriAttnProloguePa
   const int64_t n = P.n;
   const int64_t np = P.np;
   const int64_t nn = n * n;
-  const int64_t ntx = (np + kTP - 1) / kTP;
+  const int64_t ntx = (np + TP - 1) / TP;
   const int t = threadIdx.x;
   const int wave = t >> 6;
   const int lane = t & 63;
@@ -231,9 +233,9 @@ __global__ __launch_bounds__(512) void triattn_prologue_kernel(TriAttnProloguePa
   T mraw = from_f32<T>(0.f);
   bool mvalid = false;
   auto fetch = [&](int64_t tile) {
-    const TileRS tl = tile_at(tile, ntx, n);
+    const TileRS tl = tile_at(tile, ntx, n, TP);
     const int s = tl.s0 + p;
-    const bool valid = s < n;
+    const bool valid = p < TP && s < n;
     auto pos_of = [&](int ss) {
       return (int64_t)tl.b * nn + (P.transpose ? (int64_t)ss * n + tl.r : (int64_t)tl.r * n + ss);
     };
@@ -247,10 +249,10 @@ __global__ __launch_bounds__(512) void triattn_prologue_kernel(TriAttnProloguePa
   if (tile < ntiles) fetch(tile);
   __syncthreads();
   for (; tile < ntiles; tile += gridDim.x) {
-    const TileRS tl = tile_at(tile, ntx, n);
-    const int nstore = (int)min<int64_t>(kTP, np - tl.s0);  // incl. zero padding; a multiple of 64
-    const int nreal = (int)max<int64_t>(0, min<int64_t>(kTP, n - tl.s0));
-    ln_quad<T, T, NB>(xr, ln, P.eps, &xs[p][0], cw);
+    const TileRS tl = tile_at(tile, ntx, n, TP);
+    const int nstore = (int)min<int64_t>(TP, np - tl.s0);  // incl. zero padding; a multiple of 64
+    const int nreal = (int)max<int64_t>(0, min<int64_t>(TP, n - tl.s0));
+    if (p < TP) ln_quad<T, T, NB>(xr, ln, P.eps, &xs[p][0], cw);
     if ((t & 3) == 0 && p < nstore) {
       const float mv = P.mask ? to_f32(mraw) : 1.0f;
       P.mb[((int64_t)tl.b * n + tl.r) * np + tl.s0 + p] = mvalid ? P.inf * (mv - 1.0f) * kLog2e : -INFINITY;
@@ -266,11 +268,11 @@ __global__ __launch_bounds__(512) void triattn_prologue_kernel(TriAttnProloguePa
       T* qb = P.q + head_off;
       T* kb = P.k + head_off;
 #pragma unroll 2
-      for (int rt = 0; rt < 8; ++rt) {
+      for (int rt = 0; rt < nstore / 16; ++rt) {
         const int pp = 16 * rt + (lane & 15);
         f32x4 aq[2], ak[2];
         tile_mma2<T, true, NB>(xs, rt, w1, w2, aq, ak);
-        if (pp < nstore) {
+        {
           const bool real = pp < nreal;
           float vq[8], vk[8];
 #pragma unroll
@@ -290,12 +292,12 @@ __global__ __launch_bounds__(512) void triattn_prologue_kernel(TriAttnProloguePa
       // rows, so lane group g holds positions 32j + 8g .. +7 of its channel
       T* vdst = P.vt + ((int64_t)tl.b * n + tl.r) * kC * np + tl.s0;
 #pragma unroll 1
-      for (int j = 0; j < kTP / 32; ++j) {
+      for (int j = 0; j < nstore / 32; ++j) {
         const int p0 = 32 * j + 8 * (lane >> 4);
         f32x4 av[2][2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) tile_mma_row<T, false, NB>(xs, paired_row(j, h, lane & 15), w1, av[h]);
-        if (p0 < nstore) {  // nstore is a multiple of 64: all 8 positions are stored
+        {  // nstore is a multiple of 64: all 8 positions are stored
 #pragma unroll
           for (int ct = 0; ct < 2; ++ct) {
             float v[8];
@@ -307,14 +309,14 @@ __global__ __launch_bounds__(512) void triattn_prologue_kernel(TriAttnProloguePa
       }
       // triangle bias, pair j = wave & 3: lane holds positions 32j + 8g .. +7
       // of head l%16
-      {
+      if (32 * (wave & 3) < nstore) {
         const int j = wave & 3;
         const int p0 = 32 * j + 8 * (lane >> 4);
         f32x4 ab[2][2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) tile_mma_row<T, false, NB>(xs, paired_row(j, h, lane & 15), w2, ab[h]);
         const int hd = lane & 15;
-        if (hd < H && p0 < nstore) {
+        if (hd < H) {
           float v[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = p0 + e < nreal ? ab[e >> 2][0][e & 3] * kLog2e : 0.f;
@@ -661,9 +663,26 @@ void launch_persistent(void (*kern)(P, int64_t), const P& p, int threads, int64_
   hipLaunchKernelGGL(kern, dim3(persistent_grid(k, threads, ntiles)), dim3(threads), 0, st, p, ntiles);
 }
 
+// The bf16 prologues take tiles of 64 positions where 128-wide ones leave CUs
+// without one (or few with two): a tile is a serial chain of loads, LayerNorm
+// and MFMAs, and half of it is half the chain. Whole calls in a graph, 128
+// against 64: tri-mul 25.9 / 24.2 us at n = 77, 28.8 / 27.1 at 128, 39.6 / 38.3 at
+// 150 (300 tiles of 128), 41.2 / 43.5 at 180 (360); tri-attn 29.2 / 27.9 at 77,
+// 32.1 / 31.1 at 128, and with 64 channels 41.4 / 41.9 at 150; 153.6 / 159.3 and
+// 234.4 / 243.5 at 499.
+constexpr int64_t kHalfTilesTriMul = 320, kHalfTilesTriAttn = 256;
+
 template <typename T>
 void launch_trimul_prologue(const TriMulPrologueParams<T>& p, int64_t batch, hipStream_t st) {
   const int64_t ntiles = (p.n + kTP - 1) / kTP * p.n * batch;
+  if constexpr (std::is_same<T, bf16>::value) {
+    if (ntiles <= kHalfTilesTriMul) {
+      launch_persistent(p.cw == 64 ? trimul_prologue_kernel<T, true, 2, 64>
+                        : p.cw ? trimul_prologue_kernel<T, true, 4, 64> : trimul_prologue_kernel<T, false, 4, 64>,
+                        p, 512, (p.n + 63) / 64 * p.n * batch, st);
+      return;
+    }
+  }
   launch_persistent(p.cw == 64 ? trimul_prologue_kernel<T, true, 2>
                     : p.cw ? trimul_prologue_kernel<T, true> : trimul_prologue_kernel<T, false>,
                     p, 512, ntiles, st);
@@ -671,6 +690,14 @@ void launch_trimul_prologue(const TriMulPrologueParams<T>& p, int64_t batch, hip
 template <typename T>
 void launch_triattn_prologue(const TriAttnPrologueParams<T>& p, int64_t batch, hipStream_t st) {
   const int64_t ntiles = (p.np + kTP - 1) / kTP * p.n * batch;
+  if constexpr (std::is_same<T, bf16>::value) {
+    if (ntiles <= kHalfTilesTriAttn) {
+      launch_persistent(p.cw == 64 ? triattn_prologue_kernel<T, true, 2, 64>
+                        : p.cw ? triattn_prologue_kernel<T, true, 4, 64> : triattn_prologue_kernel<T, false, 4, 64>,
+                        p, 512, p.np / 64 * p.n * batch, st);
+      return;
+    }
+  }
   launch_persistent(p.cw == 64 ? triattn_prologue_kernel<T, true, 2>
                     : p.cw ? triattn_prologue_kernel<T, true> : triattn_prologue_kernel<T, false>,
                     p, 512, ntiles, st);

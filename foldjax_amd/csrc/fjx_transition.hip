@@ -185,11 +185,12 @@ __device__ __forceinline__ void wz_put(const TransitionParams<bf16>& P, f32x4 w,
 }
 
 // ---------------------------------------------------------------------------
-// Pair-track transition (C = 128, hidden 512): 128-row tiles, 512 threads.
+// Pair-track transition (C = 128, hidden 512): tiles of 16 RT rows (128, or
+// fewer for small row counts), 512 threads.
 // Wave w owns hidden columns 16w .. 16w+15 of every 128-wide hidden chunk and
 // output channels 16w .. 16w+15, so per chunk it holds just three 16-column
 // weight tiles (W_a, W_b rows of its hidden columns, W_o rows of its output
-// channels) in registers while the 8 row tiles of 16 stream past. Both
+// channels) in registers while the RT row tiles of 16 stream past. Both
 // products use the transposed accumulator form (a lane holds 4 consecutive
 // columns of one row), so silu(a)*b and the output go out 8 bytes per lane.
 // ---------------------------------------------------------------------------
@@ -199,7 +200,7 @@ __device__ __forceinline__ void wz_put(const TransitionParams<bf16>& P, f32x4 w,
 // the hidden width is 4 cw; the tile works at 128 channels with the ones past
 // cw at zero (zero affine, zero weight rows and columns), in cw / 32 hidden
 // chunks, and stores only the first cw channels
-template <typename T, bool kPbF32, bool kNarrow = false, int NB = 4>
+template <typename T, bool kPbF32, bool kNarrow = false, int NB = 4, int RT = 8>
 __device__ __forceinline__ void transition128_body(const TransitionParams<T>& P) {
   using namespace tile;
   __shared__ __attribute__((aligned(16))) T xs[kTP][kLd];  // LN(x)
@@ -208,8 +209,8 @@ __device__ __forceinline__ void transition128_body(const TransitionParams<T>& P)
   __shared__ __attribute__((aligned(16))) LnAffine pb_ln;  // the pair-bias epilogue's norm
   // (the fp32-bias form's split weight: the padding columns of xs and hs, wz_at)
 
-  const int64_t m0 = (int64_t)blockIdx.x * kTP;
-  const int nvalid = (int)min<int64_t>(kTP, P.rows - m0);
+  const int64_t m0 = (int64_t)blockIdx.x * (16 * RT);
+  const int nvalid = (int)min<int64_t>(16 * RT, P.rows - m0);
   const int t = threadIdx.x;
   const int wave = t >> 6;
   const int lane = t & 63;
@@ -245,9 +246,9 @@ __device__ __forceinline__ void transition128_body(const TransitionParams<T>& P)
   }
   __syncthreads();
 
-  f32x4 out[8];
+  f32x4 out[RT];
 #pragma unroll
-  for (int rt = 0; rt < 8; ++rt) out[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int rt = 0; rt < RT; ++rt) out[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
 #pragma unroll 1
   for (int ch = 0; ch < nch; ++ch) {
@@ -262,7 +263,7 @@ __device__ __forceinline__ void transition128_body(const TransitionParams<T>& P)
       load_wcol<T>(P.w_o, 4 * kC, col, ch * kC, wo);
     }
 #pragma unroll 2
-    for (int rt = 0; rt < 8; ++rt) {
+    for (int rt = 0; rt < RT; ++rt) {
       f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f}, b = f32x4{0.f, 0.f, 0.f, 0.f};
       tile_mma1_acc<T, NB>(xs, rt, wa, a);
       tile_mma1_acc<T, NB>(xs, rt, wb, b);
@@ -273,7 +274,7 @@ __device__ __forceinline__ void transition128_body(const TransitionParams<T>& P)
     }
     __syncthreads();
 #pragma unroll
-    for (int rt = 0; rt < 8; ++rt) tile_mma1_acc<T>(hs, rt, wo, out[rt]);
+    for (int rt = 0; rt < RT; ++rt) tile_mma1_acc<T>(hs, rt, wo, out[rt]);
     __syncthreads();  // hs is rewritten by the next chunk
   }
 
@@ -292,9 +293,9 @@ __device__ __forceinline__ void transition128_body(const TransitionParams<T>& P)
   // waits on, so loads between stores would each wait for the stores
   // before (rows past the tile's end read the last valid row, unused), with
   // no per-lane branch around them
-  float res[8][4], msk[8];
+  float res[RT][4], msk[RT];
 #pragma unroll
-  for (int rt = 0; rt < 8; ++rt) {
+  for (int rt = 0; rt < RT; ++rt) {
     msk[rt] = 1.0f;
 #pragma unroll
     for (int q = 0; q < 4; ++q) res[rt][q] = 0.f;
@@ -303,28 +304,28 @@ __device__ __forceinline__ void transition128_body(const TransitionParams<T>& P)
   if (kNarrow && col >= cw) return;
   if (P.residual) {
 #pragma unroll
-    for (int rt = 0; rt < 8; ++rt) {
+    for (int rt = 0; rt < RT; ++rt) {
       const int row = min(16 * rt + (lane & 15), nvalid - 1);
       load4f(P.residual + (m0 + row) * cw + col + 4 * (lane >> 4), res[rt]);
     }
   }
   if (P.row_mask) {
 #pragma unroll
-    for (int rt = 0; rt < 8; ++rt) msk[rt] = to_f32(P.row_mask[m0 + min(16 * rt + (lane & 15), nvalid - 1)]);
+    for (int rt = 0; rt < RT; ++rt) msk[rt] = to_f32(P.row_mask[m0 + min(16 * rt + (lane & 15), nvalid - 1)]);
   }
-  float gate[8];
+  float gate[RT];
 #pragma unroll
-  for (int rt = 0; rt < 8; ++rt) gate[rt] = 1.0f;
+  for (int rt = 0; rt < RT; ++rt) gate[rt] = 1.0f;
   if (P.out_mask) {
 #pragma unroll
-    for (int rt = 0; rt < 8; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
       gate[rt] = to_f32(P.out_mask[m0 + min(16 * rt + (lane & 15), nvalid - 1)]) != 0.f ? 1.f : 0.f;
   }
 
   // the update is rounded to T (the reference's projection output is), then
   // the residual is added
 #pragma unroll
-  for (int rt = 0; rt < 8; ++rt) {
+  for (int rt = 0; rt < RT; ++rt) {
     const int row = 16 * rt + (lane & 15);
     if (row < nvalid) {
       const int64_t off = (m0 + row) * cw + col + 4 * (lane >> 4);
@@ -348,41 +349,58 @@ __device__ __forceinline__ void transition128_body(const TransitionParams<T>& P)
   }
 }
 
-template <typename T>
+template <typename T, int RT = 8>
 __global__ __launch_bounds__(512) void transition128_kernel(TransitionParams<T> P) {
-  transition128_body<T, false>(P);
+  transition128_body<T, false, false, 4, RT>(P);
 }
-template <typename T, int NB>
+template <typename T, int NB, int RT = 8>
 __global__ __launch_bounds__(512) void transition_narrow_kernel(TransitionParams<T> P) {
-  transition128_body<T, false, true, NB>(P);
+  transition128_body<T, false, true, NB, RT>(P);
 }
 // two 512-thread workgroups (70 KB of LDS each) share a CU only at 4 waves
 // per SIMD, so this variant is held to 128 VGPRs as the plain one fits
+template <int RT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void transition128_pbf32_kernel(TransitionParams<bf16> P) {
-  transition128_body<bf16, true>(P);
+  transition128_body<bf16, true, false, 4, RT>(P);
 }
 
 // C = 128, or a narrow C (32, 64, 96: p.cw) with a 4C hidden width; other
 // widths take the general path of the C ABI layer (row LayerNorm and three
 // GEMMs), which also measured faster than a fused kernel for the single
 // track's C = 384 at every row count tried (1 K to 1 M rows).
-template <typename T>
-void launch_transition(const TransitionParams<T>& p, int c, hipStream_t st) {
-  const dim3 grid((unsigned)((p.rows + tile::kTP - 1) / tile::kTP));
+template <typename T, int RT>
+static void launch_transition_rt(const TransitionParams<T>& p, int c, hipStream_t st) {
+  const dim3 grid((unsigned)((p.rows + 16 * RT - 1) / (16 * RT)));
   if (c < tile::kC) {
     // c = 64 (the template stack): the x side compiled for its 2 blocks of 32
-    if (c == 64) hipLaunchKernelGGL((transition_narrow_kernel<T, 2>), grid, dim3(512), 0, st, p);
-    else hipLaunchKernelGGL((transition_narrow_kernel<T, 4>), grid, dim3(512), 0, st, p);
+    if (c == 64) hipLaunchKernelGGL((transition_narrow_kernel<T, 2, RT>), grid, dim3(512), 0, st, p);
+    else hipLaunchKernelGGL((transition_narrow_kernel<T, 4, RT>), grid, dim3(512), 0, st, p);
     return;
   }
   if constexpr (std::is_same<T, bf16>::value) {
     if (p.pbf_out) {
-      hipLaunchKernelGGL(transition128_pbf32_kernel, grid, dim3(512), 0, st, p);
+      hipLaunchKernelGGL(transition128_pbf32_kernel<RT>, grid, dim3(512), 0, st, p);
       return;
     }
   }
-  hipLaunchKernelGGL(transition128_kernel<T>, grid, dim3(512), 0, st, p);
+  hipLaunchKernelGGL((transition128_kernel<T, RT>), grid, dim3(512), 0, st, p);
+}
+
+template <typename T>
+void launch_transition(const TransitionParams<T>& p, int c, hipStream_t st) {
+  if constexpr (std::is_same<T, bf16>::value) {
+    // 64- and 32-row tiles while they still go one (the narrow forms: two) to a
+    // CU: the tile is a serial walk over the hidden chunks, shorter with fewer
+    // rows, but its weights are read once a tile. 128 / 64 / 32 rows: 23.0 / 18.0 /
+    // 14.9 us at 77^2 rows (32: 186 tiles), 23.2 / 18.1 / 25.2 at 100^2 (32: 313),
+    // 23.6 / 28.3 / 36.9 at 150^2 (64: 352); 64 channels 10.8 / 8.2 / 7.0 at 77^2,
+    // 11.1 / 10.3 / 14.0 at 150^2, 11.4 / 10.5 / 16.6 at 180^2 (64: 507)
+    const int rt = p.rows <= 256 * 32 ? 2 : p.rows <= (c < tile::kC ? 512 : 256) * 64 ? 4 : 8;
+    if (rt == 2) return launch_transition_rt<T, 2>(p, c, st);
+    if (rt == 4) return launch_transition_rt<T, 4>(p, c, st);
+  }
+  launch_transition_rt<T, 8>(p, c, st);
 }
 
 template void launch_transition<bf16>(const TransitionParams<bf16>&, int, hipStream_t);

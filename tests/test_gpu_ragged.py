@@ -203,3 +203,34 @@ def test_transition_fp32_with_pair_bias(n, heads):
     assert float((out.double() - y).norm() / y.norm()) <= 1e-5
     assert float((pb[:, :, :n, :n].double() - bias).norm() / bias.norm()) <= 1e-5
     assert not pb[:, :, n:].any() and not pb[..., n:].any()
+
+
+@pytest.mark.parametrize("c,bias", [(128, torch.float32), (128, torch.bfloat16), (128, None), (64, None), (96, None)])
+@pytest.mark.parametrize("n", [1, 5, 90, 91, 128, 150])
+def test_transition_rows_do_not_depend_on_the_tile(n, c, bias):
+    """A row's arithmetic is its own, so one item alone (32- and 64-row tiles at
+    these lengths) has the bits it has among enough items for 128-row tiles."""
+    say(f"transition tiles n={n} c={c} bias={bias}")
+    dtype = torch.bfloat16
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    batch = 33000 // (n * n) + 2
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)  # noqa: E731
+    w = P.pack_transition_torch(P.transition_to_protenix(syn.transition_weights(c, seed=3)), dtype, "cuda")
+    x, res = rnd(batch, n, n, c), rnd(batch, n, n, c)
+    rm, om = (rnd(batch, n, n) > 0).to(dtype) * 0.5, (rnd(batch, n, n) > -1).to(dtype)
+    aw = None
+    if bias is not None:
+        aw = kernels.SingleAttentionWeights(
+            pre_norm_weight=None, pre_norm_bias=None, z_norm_weight=1 + 0.1 * rnd(c), z_norm_bias=0.1 * rnd(c),
+            z_weight=rnd(16, c), q_weight=rnd(64, 64), q_bias=None, k_weight=rnd(64, 64), v_weight=rnd(64, 64),
+            g_weight=rnd(64, 64), o_weight=rnd(64, 64)).to(bias, "cuda")
+    want = kernels.transition(x, w, row_mask=rm, residual=res, out_mask=om, pair_bias_for=aw)
+    one = [t[1:2].contiguous() for t in (x, res, rm, om)]
+    got = kernels.transition(one[0], w, row_mask=one[2], residual=one[1], out_mask=one[3], pair_bias_for=aw)
+    torch.cuda.synchronize()
+    if aw is not None:
+        (want, want_pb), (got, got_pb) = want, got
+        assert torch.equal(getattr(got_pb, "bias", got_pb)[0], getattr(want_pb, "bias", want_pb)[1])
+    assert torch.isfinite(got.float()).all()
+    assert torch.equal(got[0], want[1])
