@@ -48,23 +48,18 @@ __device__ __forceinline__ void mma(f32x4& acc, const f32x8& a, const f32x8& b) 
 //   x y = h h' + (h m' + m h') + (h l' + l h' + m m')
 // whose dropped terms are below 2^-25 |x y|: products as good as fp32's, six
 // 16-cycle v_mfma_f32_16x16x32_bf16 in place of eight 32-cycle
-// v_mfma_f32_16x16x4_f32 per 32 k. kInf: an infinite value keeps m = l = 0 (its
-// remainder is NaN); without it, an infinity gives NaN products, for operands
-// that are finite unless the result is lost anyway (LayerNormed activations,
-// weights).
+// v_mfma_f32_16x16x4_f32 per 32 k. An infinity gives NaN products: the operands
+// are finite unless the result is lost anyway (LayerNormed activations, gated
+// projections of them, weights).
 struct Split8 {
   bf16x8 p[3];
 };
-template <bool kInf = false>
 __device__ __forceinline__ Split8 split8(const f32x8& x) {
-  constexpr float kBig = 3.3e38f;  // below the largest bf16
   Split8 s;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     s.p[0][e] = static_cast<bf16>(x[e]);
-    const float h = static_cast<float>(s.p[0][e]);
-    const float r = kInf ? __builtin_amdgcn_fmed3f(x[e], -kBig, kBig) - __builtin_amdgcn_fmed3f(h, -kBig, kBig)
-                         : x[e] - h;
+    const float r = x[e] - static_cast<float>(s.p[0][e]);
     s.p[1][e] = static_cast<bf16>(r);
     s.p[2][e] = static_cast<bf16>(r - static_cast<float>(s.p[1][e]));
   }
