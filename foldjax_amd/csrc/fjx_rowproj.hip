@@ -268,11 +268,11 @@ __global__ __launch_bounds__(512) void triattn_prologue_kernel(TriAttnProloguePa
       T* qb = P.q + head_off;
       T* kb = P.k + head_off;
 #pragma unroll 2
-      for (int rt = 0; rt < nstore / 16; ++rt) {
+      for (int rt = 0; rt < TP / 16; ++rt) {
         const int pp = 16 * rt + (lane & 15);
         f32x4 aq[2], ak[2];
         tile_mma2<T, true, NB>(xs, rt, w1, w2, aq, ak);
-        {
+        if (pp < nstore) {
           const bool real = pp < nreal;
           float vq[8], vk[8];
 #pragma unroll
@@ -292,12 +292,12 @@ __global__ __launch_bounds__(512) void triattn_prologue_kernel(TriAttnProloguePa
       // rows, so lane group g holds positions 32j + 8g .. +7 of its channel
       T* vdst = P.vt + ((int64_t)tl.b * n + tl.r) * kC * np + tl.s0;
 #pragma unroll 1
-      for (int j = 0; j < nstore / 32; ++j) {
+      for (int j = 0; j < TP / 32; ++j) {
         const int p0 = 32 * j + 8 * (lane >> 4);
         f32x4 av[2][2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) tile_mma_row<T, false, NB>(xs, paired_row(j, h, lane & 15), w1, av[h]);
-        {  // nstore is a multiple of 64: all 8 positions are stored
+        if (p0 < nstore) {  // nstore is a multiple of 64: all 8 positions are stored
 #pragma unroll
           for (int ct = 0; ct < 2; ++ct) {
             float v[8];
@@ -309,14 +309,14 @@ __global__ __launch_bounds__(512) void triattn_prologue_kernel(TriAttnProloguePa
       }
       // triangle bias, pair j = wave & 3: lane holds positions 32j + 8g .. +7
       // of head l%16
-      if (32 * (wave & 3) < nstore) {
+      if (32 * (wave & 3) < TP) {
         const int j = wave & 3;
         const int p0 = 32 * j + 8 * (lane >> 4);
         f32x4 ab[2][2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) tile_mma_row<T, false, NB>(xs, paired_row(j, h, lane & 15), w2, ab[h]);
         const int hd = lane & 15;
-        if (hd < H) {
+        if (hd < H && p0 < nstore) {
           float v[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] = p0 + e < nreal ? ab[e >> 2][0][e & 3] * kLog2e : 0.f;
