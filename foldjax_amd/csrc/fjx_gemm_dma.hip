@@ -361,7 +361,8 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams<bf16, bf16>& P, c
       // this lane holds row m0 + wm + 16 i + lrow, columns n0 + wn + 32 s + lcol
       // .. +7 in acc[2s][i] (the first 4) and acc[2s+1][i]. What the epilogue
       // reads is loaded for 4 rows before the first is used: one
-      // row at a time, every load's latency was in line
+      // row at a time, every load's latency was in line (with the selects
+      // below 64 -> 54 us for 60025 x 384 x 384 with a gate and a residual)
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const int64_t col = cur.n0 + wn + 32 * s + lcol;
