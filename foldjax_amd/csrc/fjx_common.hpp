@@ -74,6 +74,23 @@ __device__ __forceinline__ void mma(f32x4& acc, const Split8& a, const Split8& b
   mma(acc, a.p[0], b.p[0]);
 }
 
+// The LDS-DMA kernels pass their LDS stages on by hand: a fenced __syncthreads
+// would wait for every DMA still in flight. lds_wait leaves the VM youngest
+// vector-memory operations (DMA, loads and stores, in issue order; 63: all) in
+// flight and completes every LDS access of this wave, its fragment reads among
+// them: behind the barrier other waves overwrite what they read. The compiler
+// waits for a read only before its first use, which it may move past a bare
+// s_barrier; the empty asm keeps the reads themselves on their side.
+template <int VM>
+__device__ __forceinline__ void lds_wait() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0070 | ((VM >> 4) << 14) | (VM & 15));  // vmcnt(VM) lgkmcnt(0)
+}
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 __device__ __forceinline__ float to_f32(float x) { return x; }
 __device__ __forceinline__ float to_f32(bf16 x) { return static_cast<float>(x); }
 

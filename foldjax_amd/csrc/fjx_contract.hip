@@ -339,9 +339,8 @@ __global__ __launch_bounds__(512) void contract_kernel(const bf16* __restrict__ 
 // are buffer stores, issued also where no lane is in range, so that the count
 // is fixed), and the stores drain under the next k-loop.
 //
-// Synchronisation: each wave waits for its own DMA with an explicit vmcnt,
-// then a bare s_barrier (a fenced __syncthreads would wait for every DMA
-// still in flight).
+// Synchronisation: each wave waits for its own DMA and LDS reads, then a bare
+// s_barrier (lds_wait).
 // ---------------------------------------------------------------------------
 // an SGPR value the compiler can not see through (the constraint letter means
 // something else to the host pass, which only parses this)
@@ -483,12 +482,11 @@ __device__ __forceinline__ void contract_dma_body(const bf16* __restrict__ A, co
         if (st == 1 && kt >= ktiles) break;  // an odd number of k-tiles ends in stage 0
         // this wave's DMA of stage st is complete; on a tile's first k-step
         // the previous tile's stores, issued after that DMA, may still run
-        if (st == 0 && pend) __builtin_amdgcn_s_waitcnt(0x0F70 | ((kStores >> 4) << 14) | (kStores & 15));
-        else __builtin_amdgcn_s_waitcnt(0xF70);
+        if (st == 0 && pend) lds_wait<kStores>();
+        else lds_wait<0>();
         pend = 0;
         opaque_sgpr(pend);
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");  // no LDS read moves above the barrier
+        lds_barrier();
         if (kt + 1 < ktiles) issue(cur, kt + 1, st ^ 1);
         else if (has_next && st == 1) issue(nxt, 0, 0);  // stage 0 of the next tile
         const bf16* As_ = &S[st][0][0];
@@ -512,8 +510,8 @@ __device__ __forceinline__ void contract_dma_body(const bf16* __restrict__ A, co
     if (ktiles & 1) {
       // an odd number of k-tiles: the last one is in stage 0, where the next
       // tile's first stage goes once every wave is past its reads
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
+      lds_wait<63>();
+      lds_barrier();
       if (has_next) issue(nxt, 0, 0);
     }
 
@@ -664,12 +662,11 @@ __global__ __launch_bounds__(512) void contract_split_kernel(const bf16* __restr
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
         const int kt = kb + st;
-        if (st == 0 && pend) __builtin_amdgcn_s_waitcnt(0x0F70 | ((kStores >> 4) << 14) | (kStores & 15));
-        else __builtin_amdgcn_s_waitcnt(0xF70);
+        if (st == 0 && pend) lds_wait<kStores>();
+        else lds_wait<0>();
         pend = 0;
         opaque_sgpr(pend);
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");  // no LDS read moves above the barrier
+        lds_barrier();
         if (kt + 1 < ktiles) issue(cur, kt + 1, st ^ 1);
         else if (has_next) issue(nxt, 0, 0);  // ktiles is even: st is 1 here
         Split8 af[MI], bfr[NJ];

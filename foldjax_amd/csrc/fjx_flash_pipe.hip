@@ -363,9 +363,8 @@ __device__ __forceinline__ void flash_pipe_body(const FlashParams<bf16>& P) {
         // tile in the previous step) is free for block blk + 2. The wait
         // leaves the next block's 4 V loads (the youngest, issued in step 1)
         // in flight: their first reader waits for them itself.
-        __builtin_amdgcn_s_waitcnt(0xF70 | 4);  // vmcnt(4)
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");  // no LDS read moves above the barrier
+        lds_wait<4>();
+        lds_barrier();
         dma_bias(b2, IC<SET>());
         load_mb(b2, IC<SET>());
       }

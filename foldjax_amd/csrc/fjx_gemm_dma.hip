@@ -256,14 +256,11 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams<bf16, bf16>& P, c
         if (st == 1 && kt >= ktiles) break;  // an odd number of k-tiles ends in stage 0
         // this wave's DMA of stage st is complete; on a tile's first k-step
         // the previous tile's stores, issued after that DMA, may still run
-        if (kPaired && st == 0 && pend)
-          __builtin_amdgcn_s_waitcnt(0x0F70 | ((kStores >> 4) << 14) | (kStores & 15));
-        else
-          __builtin_amdgcn_s_waitcnt(0xF70);
+        if (kPaired && st == 0 && pend) lds_wait<kStores>();
+        else lds_wait<0>();
         pend = 0;
         gopaque(pend);
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");  // no LDS read moves above the barrier
+        lds_barrier();
         if (kt + 1 < ktiles) issue(cur, kt + 1, st ^ 1);
         else if (has_next && st == 1) issue(nxt, 0, 0);
         const bf16* As_ = &S[st][0][0];
@@ -290,8 +287,8 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams<bf16, bf16>& P, c
     if (ktiles & 1) {
       // an odd number of k-tiles: the last one is in stage 0, where the next
       // tile's first stage goes once every wave is past its reads
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
+      lds_wait<63>();
+      lds_barrier();
       if (has_next) issue(nxt, 0, 0);
     }
 
@@ -318,9 +315,8 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams<bf16, bf16>& P, c
       // tiles i = 2s, 2s + 1 hold columns 32 s + lcol .. +7 of a grid row, of
       // unit u0 + 8 (li / 4) + 4 j + li % 4 (j: 0, 1)
       if (wave < BT / 64) Mk[64 * wave + lane] = mk;
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
+      lds_wait<63>();
+      lds_barrier();
       const int n = (int)P.grid_n, pitch = (int)P.grid_pitch;
       const int64_t half = P.grid_units, plane = (int64_t)n * pitch;
       const int u0 = cur.n0 / 2 + wn / 2;
