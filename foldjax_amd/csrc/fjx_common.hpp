@@ -44,17 +44,24 @@ __device__ __forceinline__ void mma(f32x4& acc, const f32x8& a, const f32x8& b) 
 }
 
 // fp32 products on the bf16 matrix cores: x = h + m + l with h = bf16(x),
-// m = bf16(x - h), l = bf16(x - h - m), which leaves less than 2^-26 |x|, and
+// m = bf16(x - h), l = bf16(x - h - m), exact (8 + 8 + 8 bits) where l is no
+// subnormal, and
 //   x y = h h' + (h m' + m h') + (h l' + l h' + m m')
-// whose dropped terms are below 2^-25 |x y|: products as good as fp32's, six
-// 16-cycle v_mfma_f32_16x16x32_bf16 in place of eight 32-cycle
-// v_mfma_f32_16x16x4_f32 per 32 k. An infinity gives NaN products: the operands
-// are finite unless the result is lost anyway (LayerNormed activations, gated
-// projections of them, weights).
+// whose dropped terms m l' + l m' + l l' stay within 2^-24 |x y| (|m| <= 2^-8,
+// |l| <= 2^-17 of x's binade), fp32's own unit roundoff: products as good as
+// fp32's, six 16-cycle v_mfma_f32_16x16x32_bf16 in place of eight 32-cycle
+// v_mfma_f32_16x16x4_f32 per 32 k.
+// Values that round past the largest bf16 take their h one step lower, and an
+// infinity is the l of a unit h: no other plane of it meets a term of the
+// opposite sign, so its products are fp32's infinities (and NaN with 0). The
+// test for such values costs 1 % of a float32 tri-mul at N = 256 (126.4 ->
+// 127.7 us).
 struct Split8 {
   bf16x8 p[3];
 };
-__device__ __forceinline__ Split8 split8(const f32x8& x) {
+constexpr float kSplitOver = 0x1.FFp127f;  // rounds past the largest bf16
+// of values below kSplitOver (or NaN)
+__device__ __forceinline__ Split8 split8_plain(const f32x8& x) {
   Split8 s;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -65,6 +72,35 @@ __device__ __forceinline__ Split8 split8(const f32x8& x) {
   }
   return s;
 }
+// of any values
+__device__ __forceinline__ Split8 split8_any(const f32x8& x) {
+  Split8 s;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const bool over = fabsf(x[e]) >= kSplitOver, inf = fabsf(x[e]) > 0x1.FFFFFEp127f;
+    s.p[0][e] = static_cast<bf16>(over ? copysignf(inf ? 1.f : 0x1.FEp127f, x[e]) : x[e]);
+    const float r = x[e] - static_cast<float>(s.p[0][e]);
+    s.p[1][e] = static_cast<bf16>(inf ? 0.f : r);
+    s.p[2][e] = static_cast<bf16>(r - static_cast<float>(s.p[1][e]));
+  }
+  return s;
+}
+// whether the former will do for every lane's values (practically always)
+template <int N>
+__device__ __forceinline__ bool split_plain(const f32x8 (&x)[N]) {
+  float big = 0.f;
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) big = fmaxf(big, fabsf(x[u][e]));
+  return __builtin_amdgcn_ballot_w64(big >= kSplitOver) == 0;
+}
+__device__ __forceinline__ Split8 split8(const f32x8& x, bool plain) {
+  Split8 s = split8_plain(x);
+  if (__builtin_expect(!plain, 0)) s = split8_any(x);
+  return s;
+}
+__device__ __forceinline__ Split8 split8(const f32x8& x) { return split8(x, split_plain<1>({x})); }
 __device__ __forceinline__ void mma(f32x4& acc, const Split8& a, const Split8& b) {
   mma(acc, a.p[2], b.p[0]);
   mma(acc, a.p[0], b.p[2]);

@@ -45,13 +45,20 @@ __device__ __forceinline__ float part_sum(float v) {
   v = quad_sum(v);
   return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false));
 }
-__device__ __forceinline__ void put_planes(Planes& xs, int row, int c, const f32x8& o) {
-  const Split8 s = split8(o);
+__device__ __forceinline__ void put_planes(Planes& xs, int row, int c, const f32x8& o, bool plain) {
+  const Split8 s = split8(o, plain);
 #pragma unroll
   for (int u = 0; u < 3; ++u) store8(&xs[u][row][c], s.p[u]);
 }
+// whether this LayerNorm's outputs (the affine of values within sqrt(127)) stay
+// far from what split8_plain does not take; wave-uniform
+__device__ __forceinline__ bool ln_plain(const LnAffine& l) {
+  const int c = threadIdx.x & 63;
+  const float big = fmaxf(fmaxf(fabsf(l.w[c]), fabsf(l.w[c + 64])), fmaxf(fabsf(l.b[c]), fabsf(l.b[c + 64])));
+  return __builtin_amdgcn_ballot_w64(!(big < 0x1p120f)) == 0;
+}
 // LayerNorm (two-pass statistics) of the position t / 8 into row t / 8
-__device__ __forceinline__ void ln_planes(const Part& r, const LnAffine& l, float eps, Planes& xs) {
+__device__ __forceinline__ void ln_planes(const Part& r, const LnAffine& l, float eps, Planes& xs, bool plain) {
   float s = 0.f, q2 = 0.f;
 #pragma unroll
   for (int q = 0; q < 2; ++q)
@@ -74,18 +81,28 @@ __device__ __forceinline__ void ln_planes(const Part& r, const LnAffine& l, floa
     f32x8 o;
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = fmaf(fmaf(r.f[q][e], rstd, shift), w[e], b[e]);
-    put_planes(xs, threadIdx.x >> 3, c, o);
+    put_planes(xs, threadIdx.x >> 3, c, o, plain);
   }
 }
 
-// one 16-channel column tile of a weight over K = 128, split
+// one 16-channel column tile of a weight over K = 128, as loaded and split (all
+// of a kernel's tiles are loaded before the first is split: the rare branch of
+// a split would otherwise keep the next loads behind it)
+struct RawTile {
+  f32x8 f[4];
+};
 struct WTile {
   Split8 f[4];
 };
-__device__ __forceinline__ void load_wtile(const float* w, int64_t ldw, int row, int64_t k0, WTile& wt) {
+__device__ __forceinline__ void load_raw(const float* w, int64_t ldw, int row, int64_t k0, RawTile& r) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) wt.f[ks] = split8(load8(w + row * ldw + k0 + 32 * ks + 8 * (lane >> 4)));
+  for (int ks = 0; ks < 4; ++ks) r.f[ks] = load8(w + row * ldw + k0 + 32 * ks + 8 * (lane >> 4));
+}
+__device__ __forceinline__ void split_tile(const RawTile& r, WTile& wt) {
+  const bool plain = split_plain(r.f);
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) wt.f[ks] = split8(r.f[ks], plain);
 }
 __device__ __forceinline__ Split8 xfrag(const Planes& xs, int row, int ks) {
   Split8 x;
@@ -128,8 +145,11 @@ __global__ __launch_bounds__(512) void trimul_prologue_split_kernel(TriMulProlog
   const int64_t stride = gridDim.x >> 1;
 
   WTile wp, wg;
-  load_wtile(P.w_p, kC, half * kC + ch, 0, wp);
-  load_wtile(P.w_g, kC, half * kC + ch, 0, wg);
+  RawTile rp, rg;
+  load_raw(P.w_p, kC, half * kC + ch, 0, rp);
+  load_raw(P.w_g, kC, half * kC + ch, 0, rg);
+  split_tile(rp, wp);
+  split_tile(rg, wg);
   stage_ln<float>(P.ln_w, P.ln_b, ln);
 
   Part xr;
@@ -144,13 +164,15 @@ __global__ __launch_bounds__(512) void trimul_prologue_split_kernel(TriMulProlog
     load_part(mvalid ? P.x + pos * kC : nullptr, xr);
     if (P.mask) mraw = P.mask[pos];
   };
+  bool plain;
   auto ln_tile = [&](int buf) {
-    ln_planes(xr, ln, P.eps, xs[buf]);
+    ln_planes(xr, ln, P.eps, xs[buf], plain);
     if ((t & 7) == 0) mrow[buf][p] = mvalid ? (P.mask ? mraw : 1.0f) : 0.f;
   };
   int64_t tile = blockIdx.x >> 1;
   if (tile < ntiles) fetch(tile);
   __syncthreads();  // LayerNorm affine staged
+  plain = ln_plain(ln);
   if (tile < ntiles) {
     ln_tile(0);
     if (tile + stride < ntiles) fetch(tile + stride);
@@ -212,8 +234,11 @@ __global__ __launch_bounds__(512) void trimul_epilogue_split_kernel(TriMulEpilog
   const int p = t >> 3;
 
   WTile wg, wp;
-  load_wtile(P.w_gout, kC, 16 * wave + li, 0, wg);
-  load_wtile(P.w_pout, kC, 16 * wave + li, 0, wp);
+  RawTile rg, rp;
+  load_raw(P.w_gout, kC, 16 * wave + li, 0, rg);
+  load_raw(P.w_pout, kC, 16 * wave + li, 0, rp);
+  split_tile(rg, wg);
+  split_tile(rp, wp);
   stage_ln<float>(P.ln_in_w, P.ln_in_b, ln_in);
   stage_ln<float>(P.ln_out_w, P.ln_out_b, ln_out);
 
@@ -230,6 +255,7 @@ __global__ __launch_bounds__(512) void trimul_epilogue_split_kernel(TriMulEpilog
   int64_t tile = blockIdx.x;
   if (tile < ntiles) fetch(tile);
   __syncthreads();
+  const bool plain_in = ln_plain(ln_in), plain_out = ln_plain(ln_out);
   for (; tile < ntiles; tile += gridDim.x) {
     const TileRS tl = tile_at(tile, ntx, n, kTS);
     const int nvalid = (int)min<int64_t>(kTS, n - tl.s0);
@@ -238,7 +264,7 @@ __global__ __launch_bounds__(512) void trimul_epilogue_split_kernel(TriMulEpilog
 #pragma unroll
     for (int c = 0; c < 16; ++c) s += ov[c];
     red[0][wave][lane] = s;
-    ln_planes(xr, ln_in, P.eps, xg);
+    ln_planes(xr, ln_in, P.eps, xg, plain_in);
     __syncthreads();
     float mean = 0.f;
 #pragma unroll
@@ -262,7 +288,7 @@ __global__ __launch_bounds__(512) void trimul_epilogue_split_kernel(TriMulEpilog
         const int c = 16 * wave + 8 * q + e;
         o[e] = fmaf(fmaf(ov[8 * q + e], rstd, shift), ln_out.w[c], ln_out.b[c]);
       }
-      put_planes(xp, lane, 16 * wave + 8 * q, o);
+      put_planes(xp, lane, 16 * wave + 8 * q, o, plain_out);
     }
     if (tile + gridDim.x < ntiles) fetch(tile + gridDim.x);
     __syncthreads();
@@ -324,8 +350,11 @@ __global__ __launch_bounds__(512) void triattn_prologue_split_kernel(TriAttnProl
   // role 0: q and k; role 1: v and the bias weight (rows past the 4 heads are
   // computed on head 0's and dropped)
   WTile w1, w2;
-  load_wtile(role == 0 ? P.w_q : P.w_v, kC, 16 * wave + li, 0, w1);
-  load_wtile(role == 0 ? P.w_k : P.w_bias, kC, role == 0 ? 16 * wave + li : (li < H ? li : 0), 0, w2);
+  RawTile r1, r2;
+  load_raw(role == 0 ? P.w_q : P.w_v, kC, 16 * wave + li, 0, r1);
+  load_raw(role == 0 ? P.w_k : P.w_bias, kC, role == 0 ? 16 * wave + li : (li < H ? li : 0), 0, r2);
+  split_tile(r1, w1);
+  split_tile(r2, w2);
   stage_ln<float>(P.ln_w, P.ln_b, ln);
 
   Part xr;
@@ -340,8 +369,9 @@ __global__ __launch_bounds__(512) void triattn_prologue_split_kernel(TriAttnProl
     load_part(mvalid ? P.x + pos * kC : nullptr, xr);
     if (P.mask) mraw = P.mask[pos];
   };
+  bool plain;
   auto ln_tile = [&](int64_t tile, int buf) {
-    ln_planes(xr, ln, P.eps, xs[buf]);
+    ln_planes(xr, ln, P.eps, xs[buf], plain);
     if (role == 1 && (t & 7) == 0) {
       const TileRS tl = tile_at(tile, ntx, n, kTS);
       P.mb[(tl.b * n + tl.r) * np + tl.s0 + p] =
@@ -351,6 +381,7 @@ __global__ __launch_bounds__(512) void triattn_prologue_split_kernel(TriAttnProl
   int64_t tile = blockIdx.x >> 1;
   if (tile < ntiles) fetch(tile);
   __syncthreads();
+  plain = ln_plain(ln);
   if (tile < ntiles) {
     ln_tile(tile, 0);
     if (tile + stride < ntiles) fetch(tile + stride);
@@ -453,8 +484,11 @@ __global__ __launch_bounds__(512) void triattn_epilogue_split_kernel(TriAttnEpil
   const int p = t >> 3;
 
   WTile wg, wo;
-  load_wtile(P.w_g, kC, 16 * wave + li, 0, wg);
-  load_wtile(P.w_o, kC, 16 * wave + li, 0, wo);
+  RawTile rg, ro;
+  load_raw(P.w_g, kC, 16 * wave + li, 0, rg);
+  load_raw(P.w_o, kC, 16 * wave + li, 0, ro);
+  split_tile(rg, wg);
+  split_tile(ro, wo);
   stage_ln<float>(P.ln_w, P.ln_b, ln);
 
   auto orig_of = [&](const TileRS& tl, int pp) -> int64_t {
@@ -477,10 +511,11 @@ __global__ __launch_bounds__(512) void triattn_epilogue_split_kernel(TriAttnEpil
   int64_t tile = blockIdx.x;
   if (tile < ntiles) fetch(tile);
   __syncthreads();
+  const bool plain = ln_plain(ln);
   for (; tile < ntiles; tile += gridDim.x) {
     const TileRS tl = tile_at(tile, ntx, n, kTS);
     const int nvalid = (int)min<int64_t>(kTS, n - tl.s0);
-    ln_planes(xr, ln, P.eps, xs);
+    ln_planes(xr, ln, P.eps, xs, plain);
     __syncthreads();
 #pragma unroll 2
     for (int rt = 0; rt < kTS / 16; ++rt) {
@@ -550,7 +585,7 @@ __global__ __launch_bounds__(512) void transition_split_kernel(TransitionParams<
     stage_ln<float>(P.ln_w, P.ln_b, ln);
     if (P.pb_out) stage_ln<float>(P.pb_ln_w, P.pb_ln_b, pb_ln);
     __syncthreads();
-    ln_planes(xr, ln, P.eps, xs);
+    ln_planes(xr, ln, P.eps, xs, ln_plain(ln));
   }
   __syncthreads();
   f32x4 out[kTS / 16];
@@ -559,25 +594,19 @@ __global__ __launch_bounds__(512) void transition_split_kernel(TransitionParams<
   // a 16-channel column tile of a weight as loaded, split a fragment at a time
   // right before its products: splitting and products of the two waves of a
   // SIMD then interleave, and the next tile's loads are in flight meanwhile
-  struct Raw {
-    f32x8 f[4];
-  };
-  auto load_raw = [&](const float* w, int64_t ldw, int64_t k0, Raw& r) {
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) r.f[ks] = load8(w + li * ldw + k0 + 32 * ks + 8 * lg);
-  };
-  Raw ra, rb, ro;
-  load_raw(P.w_a + (int64_t)col * kC, kC, 0, ra);
-  load_raw(P.w_b + (int64_t)col * kC, kC, 0, rb);
+  RawTile ra, rb, ro;
+  load_raw(P.w_a, kC, col + li, 0, ra);
+  load_raw(P.w_b, kC, col + li, 0, rb);
 #pragma unroll 1
   for (int chk = 0; chk < 4; ++chk) {
-    load_raw(P.w_o + (int64_t)col * 4 * kC, 4 * kC, chk * kC, ro);
+    load_raw(P.w_o, 4 * kC, col + li, chk * kC, ro);
+    const bool plain_a = split_plain(ra.f), plain_b = split_plain(rb.f);
     f32x4 av[kTS / 16], bv[kTS / 16];
 #pragma unroll
     for (int rt = 0; rt < kTS / 16; ++rt) av[rt] = bv[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-      const Split8 wa = split8(ra.f[ks]), wb = split8(rb.f[ks]);
+      const Split8 wa = split8(ra.f[ks], plain_a), wb = split8(rb.f[ks], plain_b);
 #pragma unroll
       for (int rt = 0; rt < kTS / 16; ++rt) {
         const Split8 x = xfrag(xs, 16 * rt + li, ks);
@@ -586,8 +615,8 @@ __global__ __launch_bounds__(512) void transition_split_kernel(TransitionParams<
       }
     }
     if (chk < 3) {
-      load_raw(P.w_a + (int64_t)((chk + 1) * kC + col) * kC, kC, 0, ra);
-      load_raw(P.w_b + (int64_t)((chk + 1) * kC + col) * kC, kC, 0, rb);
+      load_raw(P.w_a, kC, (chk + 1) * kC + col + li, 0, ra);
+      load_raw(P.w_b, kC, (chk + 1) * kC + col + li, 0, rb);
     }
 #pragma unroll
     for (int rt = 0; rt < kTS / 16; ++rt) {
@@ -597,9 +626,10 @@ __global__ __launch_bounds__(512) void transition_split_kernel(TransitionParams<
       put_planes4(hs, 16 * rt + li, col + 4 * lg, h);
     }
     __syncthreads();
+    const bool plain_o = split_plain(ro.f);
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-      const Split8 wo = split8(ro.f[ks]);
+      const Split8 wo = split8(ro.f[ks], plain_o);
 #pragma unroll
       for (int rt = 0; rt < kTS / 16; ++rt) mma(out[rt], wo, xfrag(hs, 16 * rt + li, ks));
     }
@@ -636,11 +666,13 @@ __global__ __launch_bounds__(512) void transition_split_kernel(TransitionParams<
   if (!P.pb_out) return;
   // the single attention's pair bias LN_pb(out row) w^T, as pair_bias_epilogue
   WTile wz;
-  load_wtile(P.pb_w, kC, min(li, P.pb_heads - 1), 0, wz);
+  RawTile rz;
+  load_raw(P.pb_w, kC, min(li, P.pb_heads - 1), 0, rz);
+  split_tile(rz, wz);
   __syncthreads();
   Part yr;
   load_part(&ys[p][0], yr);
-  ln_planes(yr, pb_ln, P.pb_eps, xs);
+  ln_planes(yr, pb_ln, P.pb_eps, xs, ln_plain(pb_ln));
   __syncthreads();
   if (wave >= kTS / 16) return;
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
