@@ -1,7 +1,7 @@
 // Flash triangle attention on MFMA with a softmax offset: the fp32 kernel, and
 // the bf16 fallback of the pipelined offset-free pass (fjx_flash_pipe.hip).
 //
-// One wave owns one attention row i of the pair grid and 64 or 128 queries of
+// One wave owns one attention row i of the pair grid and 64 queries of
 // one head; the ROWS waves of a workgroup own ROWS consecutive rows with the same
 // head and query tile, so the [queries x 64] tile of the triangle bias -- shared by
 // every row -- is staged once in LDS per key block (double-buffered, the next
@@ -76,47 +76,24 @@ __device__ __forceinline__ float max_over_groups(float x) {
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
-// all eight elements 1 when `on`, else 0
-template <typename T> __device__ __forceinline__ typename Frag<T>::type ones8(bool on);
-template <> __device__ __forceinline__ bf16x8 ones8<bf16>(bool on) {
-  const bf16 o = static_cast<bf16>(on ? 1.0f : 0.0f);
-  return bf16x8{o, o, o, o, o, o, o, o};
-}
-template <> __device__ __forceinline__ f32x8 ones8<float>(bool on) {
-  const float o = on ? 1.f : 0.f;
-  return f32x8{o, o, o, o, o, o, o, o};
+template <typename T> __device__ __forceinline__ typename Frag<T>::type ones8() {
+  const T o = from_f32<T>(1.0f);
+  return typename Frag<T>::type{o, o, o, o, o, o, o, o};
 }
 
-// NQT query tiles of 16 per wave: 4 (64 queries; Q fragments in LDS, one
-// softmax-sum accumulator per tile) or 8 (128 queries: every K and V load
-// serves twice the queries; Q in registers, and the sums of 4 tiles share an
-// accumulator whose A operand is 1 only in rows 4(qt%4) .. +3, so lane group
-// g holds the sums of tile 4(qt/4) + g -- padded queries have zero scores,
-// so the zero-weighted rows add nothing)
-// vb: the workgroup's index in the launch grid of `total` workgroups (through
-// xcd_remap_f, its tile)
-template <typename T, int ROWS, int NQT>
-__device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t vb, int64_t total) {
+// the workgroup of rows ROWS rg .. of item b and queries q0 .. q0 + 63 of head h
+template <typename T, int ROWS>
+__device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t b, int64_t h, int64_t rg, int64_t q0) {
   typedef typename Frag<T>::type FragT;
+  constexpr int NQT = 4;  // query tiles of 16
   constexpr int QTL = 16 * NQT;
-  constexpr bool kQLds = NQT == 4;
-  constexpr int NLS = kQLds ? 4 : NQT / 4;
   __shared__ __attribute__((aligned(16))) float bias_s[2][QTL][kBiasLd];
-  __shared__ __attribute__((aligned(16))) FragT q_s[kQLds ? ROWS : 1][4][64];  // [wave][qt][lane]: B fragments of Q
+  __shared__ __attribute__((aligned(16))) FragT q_s[ROWS][4][64];  // [wave][qt][lane]: B fragments of Q
   __shared__ __attribute__((aligned(16))) float mb_s[2][ROWS][kKB];  // each row's mask bias, one key block
 
   const int64_t n = P.n;
   const int64_t np = P.np;
   const int64_t H = P.heads;
-  const int64_t QT = (np + QTL - 1) / QTL;
-  const int64_t RG = (P.rows + ROWS - 1) / ROWS;
-  int64_t lid = xcd_remap_f(vb, total);
-  const int64_t qtile = lid % QT;
-  lid /= QT;
-  const int64_t rg = lid % RG;
-  lid /= RG;
-  const int64_t h = lid % H;
-  const int64_t b = lid / H;
 
   const int t = threadIdx.x;
   const int wave = t >> 6;
@@ -126,10 +103,9 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   const int64_t row = rg * ROWS + wave;
   const bool row_ok = row < P.rows;
   const int64_t i = row_ok ? row : P.rows - 1;
-  const int64_t q0 = qtile * QTL;
 
   const int64_t head_off = ((b * P.rows + i) * H + h) * P.qk_rows;  // in rows of length kD
-  const int64_t last = P.qk_rows - 1;  // rows past it (padded queries and keys) repeat it
+  const int last = (int)P.qk_rows - 1;  // keys past it repeat it (their mask bias is -inf); queries are zeros
   const T* Q = P.q + head_off * kD;
   const T* K = P.k + head_off * kD;
   const T* VT = P.vt + ((b * P.rows + i) * H * kD + h * kD) * np;
@@ -140,28 +116,27 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
 
   // Q stays in LDS (in fragment order: conflict-free 16-byte reads) and is
   // re-read per key block, which leaves registers for a second V buffer
-  FragT qreg[kQLds ? 1 : NQT];
 #pragma unroll
   for (int qt = 0; qt < NQT; ++qt) {
-    FragT f = load8(Q + min<int64_t>(q0 + 16 * qt + li, last) * kD + 8 * lg);
+    const int q = (int)q0 + 16 * qt + li;
+    FragT f = load8(Q + min(q, last) * kD + 8 * lg);
+    if (q > last) f = FragT{};
     if (P.q_mul != 1.f) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) f[e] = from_f32<T>(to_f32(f[e]) * P.q_mul);
     }
-    if constexpr (kQLds) q_s[wave][qt][lane] = f;
-    else qreg[qt] = f;
+    q_s[wave][qt][lane] = f;
   }
 
   float m[NQT];
-  f32x4 o[2][NQT], lsum[NLS];
+  f32x4 o[2][NQT], lsum[NQT];  // a query tile has sums of its own: what a NaN score spoils is its query alone
 #pragma unroll
   for (int qt = 0; qt < NQT; ++qt) {
     m[qt] = -1.0e30f;
     o[0][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
     o[1][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    lsum[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-#pragma unroll
-  for (int u = 0; u < NLS; ++u) lsum[u] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // bias tile fill: 8 threads cover one 64-key row (a whole cache line in
   // bf16), 64*ROWS/8 rows per pass
@@ -171,10 +146,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   static_assert(PASSES * RPP == QTL, "bias tile fill");
   const int br = t >> 3;
   const int bc = 8 * (t & 7);
-  // a 128-query tile may end past np (by 64): its missing queries repeat the
-  // last row (of q too, above) and are not stored
-  const T* bsrc = BIAS + bc;
-  auto brow = [&](int c) { return min<int64_t>(q0 + br + RPP * c, np - 1) * np; };
+  const T* bsrc = BIAS + (q0 + br) * np + bc;
   // the next key block's bias tile and mask bias travel in registers and are
   // written to the other LDS buffer at the end of the current block; the
   // mask flag (any non-zero mask bias in this row's block) is wave-uniform
@@ -182,7 +154,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   float mbn;
   auto fetch_tile = [&](int64_t k0) {
 #pragma unroll
-    for (int c = 0; c < PASSES; ++c) breg[c] = load8(bsrc + brow(c) + k0);
+    for (int c = 0; c < PASSES; ++c) breg[c] = load8(bsrc + (int64_t)RPP * c * np + k0);
     mbn = MB[k0 + lane];
   };
   auto put_tile = [&](int buf) {
@@ -200,8 +172,11 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   bool masked_blk = put_tile(0);
 
   FragT kf[4];
+  auto load_k = [&](int64_t k0) {
 #pragma unroll
-  for (int kt = 0; kt < 4; ++kt) kf[kt] = load8(K + min<int64_t>(key_of(kt, li), last) * kD + 8 * lg);
+    for (int kt = 0; kt < 4; ++kt) kf[kt] = load8(K + min((int)k0 + key_of(kt, li), last) * kD + 8 * lg);
+  };
+  load_k(0);
   // V of the current block in vf, the next block's arriving in vn
   FragT vf[2][2], vn[2][2];  // [dt][c]
   auto load_v = [&](FragT (&v)[2][2], int64_t k0) {
@@ -231,9 +206,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
 
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
-      FragT qf;
-      if constexpr (kQLds) qf = q_s[wave][qt][lane];
-      else qf = qreg[qt];
+      const FragT qf = q_s[wave][qt][lane];
       f32x4 s[4];
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt) s[kt] = *reinterpret_cast<const f32x4*>(&bias_s[buf][16 * qt + li][col_of(kt, lg)]);
@@ -250,8 +223,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
       for (int kt = 0; kt < 4; ++kt) mma(s[kt], kf[kt], qf);
       if (qt == NQT - 1) {
         // K of this block is consumed: fetch the next block's into the same registers
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) kf[kt] = load8(K + min<int64_t>(kn + key_of(kt, li), last) * kD + 8 * lg);
+        load_k(kn);
       }
       float pv[4][4];
       // this lane's 16 scores: a max3 tree (5 + 2 + 1)
@@ -273,8 +245,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
         const float alpha = __builtin_amdgcn_exp2f(m[qt] - mnew);
         o[0][qt] *= alpha;
         o[1][qt] *= alpha;
-        if constexpr (kQLds) lsum[qt] *= alpha;
-        else lsum[qt >> 2] *= lg == (qt & 3) ? alpha : 1.0f;
+        lsum[qt] *= alpha;
         m[qt] = mnew;
       }
       const float mnew = m[qt];
@@ -289,8 +260,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
         const FragT pf = pack8<T>(f);
         mma(o[0][qt], vc[0][c], pf);
         mma(o[1][qt], vc[1][c], pf);
-        if constexpr (kQLds) mma(lsum[qt], ones8<T>(true), pf);
-        else mma(lsum[qt >> 2], ones8<T>((li >> 2) == (qt & 3)), pf);
+        mma(lsum[qt], ones8<T>(), pf);
       }
     }
 
@@ -309,10 +279,7 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
   T* OUT = P.out + b * P.o_stride_b + i * P.o_stride_row + h * P.o_stride_head;
 #pragma unroll
   for (int qt = 0; qt < NQT; ++qt) {
-    float ls;
-    if constexpr (kQLds) ls = lsum[qt][0];
-    else ls = __shfl(lsum[qt >> 2][0], 16 * (qt & 3) + li, 64);
-    const float inv = 1.0f / ls;
+    const float inv = 1.0f / lsum[qt][0];
     const int64_t q = q0 + 16 * qt + li;
     if (q >= n) continue;
 #pragma unroll
@@ -328,15 +295,35 @@ __device__ __forceinline__ void flash_tri_body(const FlashParams<T>& P, int64_t 
 
 constexpr int kRows = 4;
 
+// workgroup vb of a grid of `total`, of `queries` queries each
+template <typename T>
+struct FlashTile {
+  int64_t b, h, rg, q0;
+  __device__ __forceinline__ FlashTile(const FlashParams<T>& P, int64_t vb, int64_t total, int queries) {
+    const int64_t QT = (P.np + queries - 1) / queries;
+    const int64_t RG = (P.rows + kRows - 1) / kRows;
+    int64_t lid = xcd_remap_f(vb, total);
+    q0 = lid % QT * queries;
+    lid /= QT;
+    rg = lid % RG;
+    lid /= RG;
+    h = lid % P.heads;
+    b = lid / P.heads;
+  }
+};
+
 // The bf16 fallback of the pipelined offset-free pass (fjx_flash_pipe.hip),
-// over that pass's grid of `total` workgroups of 16 NQT queries: workgroup w
+// over that pass's grid of `total` workgroups of `queries` queries: workgroup w
 // reads the flags of `per` consecutive ones (64 a load) and recomputes the
-// flagged ones with a softmax offset. Launched with no more workgroups than
-// the GPU holds at once, it costs few short workgroups when nothing is flagged
-// and, when everything is, as many rounds of resident workgroups as the full
-// grid would.
-template <int NQT>
-__device__ __forceinline__ void flash_redo_body(const FlashParams<bf16>& P, int64_t total, int64_t per) {
+// flagged ones with a softmax offset, 64 queries at a time (128 would need
+// their sums to share accumulators, through which a NaN of one query reached
+// three others, and spilled). At most four workgroups per resident one: fewer
+// when nothing is flagged, yet flags that lie together still spread. The core
+// on 4 heads, 128 queries and one workgroup per resident one against this, us:
+// nothing flagged 154 / 150 at n = 499, 920 / 916 at 1024; everything 324 / 301
+// and 2100 / 2055; one row in 50 at n = 952 1678 / 1008.
+__global__ __launch_bounds__(64 * kRows) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void flash_tri_redo_kernel_bf16(FlashParams<bf16> P, int queries, int64_t total, int64_t per) {
   const int64_t base = (int64_t)blockIdx.x * per;
   const int lane = threadIdx.x & 63;
   for (int64_t c0 = 0; c0 < per; c0 += 64) {
@@ -346,24 +333,18 @@ __device__ __forceinline__ void flash_redo_body(const FlashParams<bf16>& P, int6
     while (m != 0) {
       const int k = __builtin_ctzll(m);
       m &= m - 1;
-      flash_tri_body<bf16, kRows, NQT>(P, base + c0 + k, total);
-      __syncthreads();  // LDS is reused by the next flagged workgroup
+      const FlashTile<bf16> tl(P, base + c0 + k, total, queries);
+      for (int64_t q0 = tl.q0; q0 < tl.q0 + queries && q0 < P.np; q0 += 64) {
+        flash_tri_body<bf16, kRows>(P, tl.b, tl.h, tl.rg, q0);
+        __syncthreads();  // LDS is reused by the next queries or workgroup
+      }
     }
   }
 }
-// 128 queries per wave: 256 VGPRs, 2 waves per SIMD, 72 KB of LDS
-__global__ __launch_bounds__(64 * kRows) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void flash_tri8_redo_kernel_bf16(FlashParams<bf16> P, int64_t total, int64_t per) {
-  flash_redo_body<8>(P, total, per);
-}
-// 64 queries: 3 waves per SIMD (168 VGPRs) measured faster than 2 without spills
-__global__ __launch_bounds__(64 * kRows) __attribute__((amdgpu_waves_per_eu(3, 3)))
-void flash_tri4_redo_kernel_bf16(FlashParams<bf16> P, int64_t total, int64_t per) {
-  flash_redo_body<4>(P, total, per);
-}
 
 __global__ __launch_bounds__(64 * kRows) void flash_tri_kernel_f32(FlashParams<float> P) {
-  flash_tri_body<float, kRows, 4>(P, blockIdx.x, gridDim.x);
+  const FlashTile<float> tl(P, blockIdx.x, gridDim.x, kQT);
+  flash_tri_body<float, kRows>(P, tl.b, tl.h, tl.rg, tl.q0);
 }
 
 template <typename T>
@@ -386,10 +367,11 @@ void launch_flash(const FlashParams<T>& p, int64_t batch, hipStream_t st) {
     const int queries = groups * ((p.np + 127) / 128) < 320 ? 64 : 128;
     const int64_t total = groups * ((p.np + queries - 1) / queries);
     launch_flash_pipe(p, groups, queries, st);
-    const auto redo = queries == 128 ? flash_tri8_redo_kernel_bf16 : flash_tri4_redo_kernel_bf16;
-    const int64_t cap = tile::resident_blocks(reinterpret_cast<const void*>(redo), 64 * kRows);
-    const int64_t per = (total + cap - 1) / cap;
-    hipLaunchKernelGGL(redo, dim3((unsigned)((total + per - 1) / per)), dim3(64 * kRows), 0, st, p, total, per);
+    const int64_t cap =
+        tile::resident_blocks(reinterpret_cast<const void*>(flash_tri_redo_kernel_bf16), 64 * kRows);
+    const int64_t per = (total + 4 * cap - 1) / (4 * cap);  // flags a workgroup
+    hipLaunchKernelGGL(flash_tri_redo_kernel_bf16, dim3((unsigned)((total + per - 1) / per)), dim3(64 * kRows), 0, st,
+                       p, queries, total, per);
   } else {
     hipLaunchKernelGGL(flash_tri_kernel_f32, dim3((unsigned)(groups * (p.np / kQT))), dim3(64 * kRows), 0, st, p);
   }

@@ -6,7 +6,7 @@
 // softmax sums on MFMA), for the offset-free pass only: p = exp2(s) straight
 // from the log2-unit score. A workgroup whose sums or outputs leave the safe
 // range is flagged for the offset kernel of fjx_flash.hip, which recomputes
-// it (flash_tri8_redo_kernel_bf16 walks the flags); the flags are indexed in
+// it (flash_tri_redo_kernel_bf16 walks the flags); the flags are indexed in
 // that kernel's grid, which this kernel runs exactly (4 rows x 128 or 64
 // queries of one head per workgroup).
 //

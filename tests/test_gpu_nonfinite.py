@@ -3,7 +3,9 @@ output is infinite or NaN where the same call in float64 (converted to the
 call's dtype) is, and only there.
 
 The float32 path multiplies three-plane bf16 splits of its operands, in which
-an infinite or nearly infinite operand needs a form of its own."""
+an infinite or nearly infinite operand needs a form of its own. The attention
+pass sums the softmax of several queries in one accumulator and recomputes
+what leaves the safe range: a query's NaN must stay its own."""
 
 from __future__ import annotations
 
@@ -128,3 +130,32 @@ def test_transition_fp32(field, value, scale):
     h = (a * torch.sigmoid(a)).float() * b.float()  # float32's own overflow
     want = h.double() @ d.w_o.T
     assert_same_kind(got, want, 1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,n", [(5, 40), (9, 100), (81, 430), (81, 500), (1, 70)])
+@pytest.mark.parametrize("where", ["q", "bias"])
+def test_core_nan_of_one_query(where, rows, n, dtype):
+    """64- and 128-query workgroups, padded lengths that are even and odd
+    multiples of 64, the single-row pass and the float32 one."""
+    say(f"core NaN in {where} rows={rows} n={n} {dtype}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    q, k, v = (torch.randn(1, rows, 4, n, 32, generator=g, device="cuda").to(dtype) for _ in range(3))
+    tb = torch.randn(1, 1, 4, n, n, generator=g, device="cuda").to(dtype)
+    clean = kernels.triattn_core(q, k, v, tb, None, scale=32 ** -0.5)
+    row, head, j = rows // 2, 2, n // 2 + 3
+    bad = torch.zeros(1, rows, 4, n, dtype=torch.bool, device="cuda")
+    if where == "q":
+        q[0, row, head, j, 7] = math.nan
+        bad[0, row, head, j] = True
+    else:
+        tb[0, 0, head, j, 5] = math.nan
+        bad[0, :, head, j] = True
+    got = kernels.triattn_core(q, k, v, tb, None, scale=32 ** -0.5)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.isnan(got).all(-1), bad) and torch.equal(torch.isnan(got).any(-1), bad)
+    # the rest: recomputed with another softmax offset at most (bf16: 2^-8 a
+    # rounding of the probabilities and of the output)
+    diff = torch.where(bad[..., None], 0.0, (got - clean).float()).abs().max()
+    assert float(diff) <= (3e-2 if dtype == torch.bfloat16 else 1e-5) * float(clean.float().abs().max())
