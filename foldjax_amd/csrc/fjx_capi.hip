@@ -1,5 +1,6 @@
 // C ABI of the triangle kernels: argument checks, workspace layout, launch
 // sequence, thread-local error strings and optional per-kernel event timing.
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <mutex>
@@ -1079,6 +1080,12 @@ int trimul_check(const fjx_trimul_args* a, const char* fn) {
   return FJX_OK;
 }
 
+// the workspace of a call: with rows padded as the kernels like them, or tight
+size_t trimul_bytes(int64_t batch, int64_t n, int64_t c_z, int64_t c_h, int32_t dtype, bool tight) {
+  return fused_trimul(c_z, c_h) ? trimul_ws(batch, n, c_z, dtype, tight).total
+                                : gen_trimul_ws(batch, n, c_z, c_h, dtype, tight).total;
+}
+
 int trimul_dispatch(const fjx_trimul_args* a, bool tight, hipStream_t st) {
   if (!fused_trimul(a->c_z, a->c_h))
     return a->dtype == FJX_DTYPE_BF16 ? trimul_generic_run<bf16>(a, tight, st)
@@ -1095,18 +1102,19 @@ int fjx_abi_version(void) { return FJX_ABI_VERSION; }
 
 size_t fjx_trimul_workspace_size(int64_t batch, int64_t n, int64_t c_z, int64_t c_h, int32_t dtype) {
   if (batch < 1 || n < 1 || c_z < 1 || c_h < 1 || !dtype_ok(dtype)) return 0;
-  return fused_trimul(c_z, c_h) ? trimul_ws(batch, n, c_z, dtype).total : gen_trimul_ws(batch, n, c_z, c_h, dtype).total;
+  return trimul_bytes(batch, n, c_z, c_h, dtype, false);
 }
 
 
 int fjx_trimul_fwd(const fjx_trimul_args* a, hipStream_t st) {
   g_err.clear();
   if (int rc = trimul_check(a, "fjx_trimul_fwd")) return rc;
-  const size_t need = fjx_trimul_workspace_size(a->batch, a->n, a->c_z, a->c_h, a->dtype);
-  if (!a->workspace || a->workspace_bytes < need)
-    return fail(FJX_ERR_WORKSPACE, "fjx_trimul_fwd: workspace of %zu bytes needed, %zu given", need,
+  const size_t full = trimul_bytes(a->batch, a->n, a->c_z, a->c_h, a->dtype, false);
+  const size_t least = trimul_bytes(a->batch, a->n, a->c_z, a->c_h, a->dtype, true);
+  if (!a->workspace || a->workspace_bytes < std::min(full, least))
+    return fail(FJX_ERR_WORKSPACE, "fjx_trimul_fwd: workspace of %zu bytes needed, %zu given", full,
                 a->workspace_bytes);
-  return trimul_dispatch(a, false, st);
+  return trimul_dispatch(a, a->workspace_bytes < full, st);
 }
 
 
@@ -1360,16 +1368,14 @@ __attribute__((visibility("hidden"))) int trimul_fwd_on_scratch(const fjx_trimul
   // refused by the size of the tight layout (rows of exactly n elements),
   // which is also what runs where the padded one does not fit
   const bool fused = fused_trimul(a->c_z, a->c_h);
-  const size_t need = fused ? trimul_ws(a->batch, a->n, a->c_z, a->dtype, true).total
+  const size_t need = fused ? trimul_bytes(a->batch, a->n, a->c_z, a->c_h, a->dtype, true)
                             : gen_trimul_noalloc_bytes(a->batch, a->n, a->c_z, a->c_h, a->dtype);
   if (need > FJX_NOALLOC_MAX_BYTES)
     return fail(FJX_ERR_WORKSPACE,
                 "%s: this shape needs %zu bytes of scratch, the library's static scratch holds %zu "
                 "(use fjx_trimul_fwd with a workspace)",
                 fn, need, (size_t)FJX_NOALLOC_MAX_BYTES);
-  const size_t padded = fused ? trimul_ws(a->batch, a->n, a->c_z, a->dtype).total
-                              : gen_trimul_ws(a->batch, a->n, a->c_z, a->c_h, a->dtype).total;
-  const bool tight = padded > scratch_bytes;
+  const bool tight = trimul_bytes(a->batch, a->n, a->c_z, a->c_h, a->dtype, false) > scratch_bytes;
   fjx_trimul_args b = *a;
   b.workspace = scratch;
   b.workspace_bytes = scratch_bytes;

@@ -497,7 +497,15 @@ def trimul(
     out = _out_buffer(out, x, xf)
     res = _like(residual, x.dtype)
     ws_bytes = 0 if no_alloc else lib.fjx_trimul_workspace_size(batch, n, c, c_h, code)
-    ws = None if no_alloc else torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
+    try:
+        ws = None if no_alloc else torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
+    except torch.OutOfMemoryError:
+        # a, b and o unpadded and unsplit: slower, but all that a call needs
+        least = 3 * ((batch * n * n * c_h * x.element_size() + 255) // 256 * 256)
+        if c_h != 128 or c not in (32, 64, 96, 128) or least >= ws_bytes:
+            raise
+        ws_bytes = least
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
     a = _lib.TriMulArgs(
         batch=batch, n=n, c_z=c, c_h=c_h,
         direction=_lib.FJX_OUTGOING if direction == "outgoing" else _lib.FJX_INCOMING,

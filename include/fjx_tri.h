@@ -113,6 +113,13 @@ typedef struct fjx_trimul_args {
   const void* out_mask;        /* NULL, or [batch, n, n]: see "Output masks" */
 } fjx_trimul_args;
 
+/* The workspace that the fastest kernels need: a, b and o with their rows padded
+ * to 64 elements and, in float32 with c_z == c_h == 128, a and b as three bf16
+ * planes each (16 bytes an element of a row in place of 12). fjx_trimul_fwd also
+ * takes a smaller one that holds them unpadded and unsplit, each rounded up to
+ * 256 bytes (c_h == 128 and c_z of 32, 64, 96 or 128: 3 * batch * n^2 * 128
+ * elements), and then runs slower kernels on it (float32: on the fp32 matrix
+ * instructions, whose results differ by float32's own rounding). */
 size_t fjx_trimul_workspace_size(int64_t batch, int64_t n, int64_t c_z, int64_t c_h, int32_t dtype);
 int fjx_trimul_fwd(const fjx_trimul_args* args, hipStream_t stream);
 
