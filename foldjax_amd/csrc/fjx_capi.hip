@@ -1375,12 +1375,31 @@ __attribute__((visibility("hidden"))) int trimul_fwd_on_scratch(const fjx_trimul
                 "%s: this shape needs %zu bytes of scratch, the library's static scratch holds %zu "
                 "(use fjx_trimul_fwd with a workspace)",
                 fn, need, (size_t)FJX_NOALLOC_MAX_BYTES);
-  const bool tight = trimul_bytes(a->batch, a->n, a->c_z, a->c_h, a->dtype, false) > scratch_bytes;
   fjx_trimul_args b = *a;
   b.workspace = scratch;
   b.workspace_bytes = scratch_bytes;
+  // float32 planes: as many items at a time as the scratch holds (one at
+  // least, by the limit above), so that the kernels and the bits are
+  // fjx_trimul_fwd's whatever the batch
+  const bool split = trimul_ws(1, a->n, a->c_z, a->dtype).split && fused;
+  const bool tight = !split && trimul_bytes(a->batch, a->n, a->c_z, a->c_h, a->dtype, false) > FJX_NOALLOC_SCRATCH_BYTES;
+  const int64_t items =
+      split ? (int64_t)(scratch_bytes / trimul_bytes(1, a->n, a->c_z, a->c_h, a->dtype, false)) : a->batch;
+  if (items < 1) return fail(FJX_ERR_WORKSPACE, "%s: the static scratch does not hold one item", fn);
+  const int64_t positions = a->n * a->n, es = (int64_t)esize(a->dtype);
+  auto from = [](const void* p, int64_t bytes) { return p ? static_cast<const char*>(p) + bytes : nullptr; };
+  int rc = FJX_OK;
   g_no_events = true;
-  const int rc = trimul_dispatch(&b, tight, st);
+  for (int64_t b0 = 0; b0 < a->batch && rc == FJX_OK; b0 += items) {
+    const int64_t skip = b0 * positions * es;
+    b.batch = std::min(items, a->batch - b0);
+    b.x = from(a->x, skip * a->c_z);
+    b.mask = from(a->mask, skip);
+    b.residual = from(a->residual, skip * a->c_z);
+    b.out = static_cast<char*>(a->out) + skip * a->c_z;
+    b.out_mask = from(a->out_mask, skip);
+    rc = trimul_dispatch(&b, tight, st);
+  }
   g_no_events = false;
   return rc;
 }

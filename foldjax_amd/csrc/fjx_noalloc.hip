@@ -16,7 +16,11 @@
 
 #include "fjx_tri.h"
 
-static __device__ __align__(256) unsigned char scratch[FJX_NOALLOC_SCRATCH_BYTES];
+// the largest of the layouts: float32 at 418 tokens, rows padded to 448, two
+// operands of 6 bytes an element and the output of 4
+constexpr size_t kScratchBytes = (size_t)418 * 448 * 128 * 16;
+static_assert(kScratchBytes >= FJX_NOALLOC_SCRATCH_BYTES, "every other layout");
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace fjx {
 int trimul_fwd_on_scratch(const fjx_trimul_args* a, hipStream_t st, void* scratch_ptr, size_t scratch_bytes,
@@ -65,5 +69,5 @@ extern "C" int fjx_trimul_fwd_noalloc(const fjx_trimul_args* a, hipStream_t stre
   char err[256];
   void* ptr = scratch_on(dev, err, sizeof err);
   if (!ptr) return fjx::set_error(FJX_ERR_HIP, err);
-  return fjx::trimul_fwd_on_scratch(a, stream, ptr, FJX_NOALLOC_SCRATCH_BYTES, "fjx_trimul_fwd_noalloc");
+  return fjx::trimul_fwd_on_scratch(a, stream, ptr, kScratchBytes, "fjx_trimul_fwd_noalloc");
 }

@@ -479,10 +479,11 @@ def trimul(
     ``out_mask != 0`` per position when ``out_mask`` (``[..., N, N]``) is given.
 
     ``no_alloc``: run ``fjx_trimul_fwd_noalloc`` instead, whose workspace is
-    the library's static per-GPU scratch (shapes up to
-    256 MiB of unpadded workspace; calls on one GPU must not overlap). Only the output is allocated here, unless ``out`` is given:
-    the result then goes into that tensor (x's shape, dtype and device,
-    contiguous), which may be ``x`` and/or ``residual`` (in place)."""
+    the library's static per-GPU scratch (shapes up to 256 MiB of unpadded
+    workspace; calls on one GPU must not overlap). Only the output is allocated
+    here, unless ``out`` is given: the result then goes into that tensor (x's
+    shape, dtype and device, contiguous), which may be ``x`` and/or
+    ``residual`` (in place)."""
     if direction not in ("outgoing", "incoming"):
         raise ValueError(f"Unsupported triangle multiplication direction: {direction!r}")
     _same_device(x, residual=residual, out_mask=out_mask)

@@ -130,16 +130,15 @@ int fjx_trimul_fwd(const fjx_trimul_args* args, hipStream_t stream);
  *
  * Same arguments, checks, kernels and results as fjx_trimul_fwd, except that
  * args->workspace and args->workspace_bytes are ignored: the workspace is a
- * static device array of the library, FJX_NOALLOC_SCRATCH_BYTES per GPU,
- * reserved when the library's code is loaded on a GPU and held until the
- * process ends. A shape whose a, b and o (of n-element rows) exceed
- * FJX_NOALLOC_MAX_BYTES is refused with FJX_ERR_WORKSPACE (bf16 with
- * c_z == c_h == 128: batch * n^2 up to 349525, i.e. n <= 591 at batch 1;
- * fp32: n <= 418). The array holds those with their rows padded to 64
- * elements, as fjx_trimul_fwd lays them out, at batch 1; where it does not
- * (some batches), the rows stay unpadded and the contraction runs a slower
- * kernel. The stream must belong to the current device (FJX_ERR_INVALID
- * otherwise).
+ * static device array of the library, 366 MiB per GPU, reserved when the
+ * library's code is loaded on a GPU and held until the process ends. A shape
+ * whose a, b and o (of n-element rows) exceed FJX_NOALLOC_MAX_BYTES is refused
+ * with FJX_ERR_WORKSPACE (bf16 with c_z == c_h == 128: batch * n^2 up to
+ * 349525, i.e. n <= 591 at batch 1; fp32: n <= 418). At batch 1 the array holds
+ * them as fjx_trimul_fwd lays them out. Batches whose padded rows exceed
+ * FJX_NOALLOC_SCRATCH_BYTES run on unpadded rows with a slower contraction, or,
+ * in fp32 with c_z == c_h == 128, as many items at a time as fit. The stream
+ * must belong to the current device (FJX_ERR_INVALID otherwise).
  *
  * Every call on one GPU uses that GPU's single array: calls that overlap on
  * one GPU (other streams, other threads) race and must be serialised by the

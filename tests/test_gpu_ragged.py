@@ -162,18 +162,20 @@ def test_trimul_fp32_corner_of_a_masked_call(n, padded, direction):
     assert torch.equal(got, want)
 
 
-def test_trimul_fp32_without_planes():
-    """The static scratch does not hold the split planes of 400 tokens: the
-    fp32 matrix instructions run instead, within the two paths' fp32 errors
-    (5e-7 of the result's norm each)."""
-    n = 400
-    say(f"trimul fp32 without planes n={n}")
+@pytest.mark.parametrize("n,batch", [(400, 1), (418, 1), (133, 9), (1, 3000), (65, 40)])
+def test_trimul_fp32_noalloc_bits(n, batch):
+    """The static scratch holds the split planes up to its largest float32
+    length, and of larger batches as many items as fit at a time: the bits of
+    the call with a workspace. (65, 40): 22 and 18 items; (1, 3000): 2926."""
+    say(f"trimul fp32 noalloc n={n} batch={batch}")
     w = _weights(torch.float32)
-    z = _pair(n, torch.float32)
-    want = kernels.trimul(z, None, w, "outgoing")
-    got = kernels.trimul(z, None, w, "outgoing", no_alloc=True)
+    z = torch.cat([_pair(n, torch.float32, seed=s % 7) for s in range(batch)])
+    mask = (torch.rand(batch, n, n, device="cuda") > 0.2).float()
+    out_mask = (torch.rand(batch, n, n, device="cuda") > 0.1).float()
+    want = kernels.trimul(z, mask, w, "incoming", residual=z, out_mask=out_mask)
+    got = kernels.trimul(z, mask, w, "incoming", residual=z, out_mask=out_mask, no_alloc=True)
     torch.cuda.synchronize()
-    assert float((got - want).norm() / want.norm()) <= 2e-6
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("n", [1, 5, 8, 33])
