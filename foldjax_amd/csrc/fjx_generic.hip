@@ -142,7 +142,8 @@ template <typename T>
 constexpr int kLnCols = 128 / (int)sizeof(T);
 
 // position-major rows from planes, with the LayerNorm over the channels
-// (w null: none; channels blockIdx.y * 512 .. of more than 512). A workgroup
+// (w null: none; channels blockIdx.y * 512 .. of more than 512; `written` of a
+// row's columns hold values, n at least). A workgroup
 // takes kLnCols columns of one grid row: the planes' 128-byte pieces go to LDS
 // as they are, chunk q (16 bytes) of channel c in slot q ^ (c / 8) % 8, so that
 // 8 lanes reading the same position of channels 8 apart hit different banks; a
@@ -156,7 +157,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void planes_layernorm_kernel(const T* __restrict__ src, int C,
                                                                const T* __restrict__ w, const T* __restrict__ b,
                                                                T* __restrict__ dst, int64_t n, int64_t pitch,
-                                                               bool blocked, bool vec, float eps) {
+                                                               int64_t written, bool blocked, bool vec, float eps) {
   constexpr int PB = kLnCols<T>, E = 16 / (int)sizeof(T);  // columns per tile, elements per chunk
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   T* S = reinterpret_cast<T*>(smem);
@@ -172,8 +173,8 @@ __global__ __launch_bounds__(256) void planes_layernorm_kernel(const T* __restri
     const int64_t p = bb * C + c0 + c;
     const T* g = base + (p >> 7) * gs + (p & 127) * cs + q * E;
     T* d = S + c * PB + (q ^ ((c >> 3) & 7)) * E;
-    if (vec) {
-      if (s0 + q * E < pitch) *reinterpret_cast<u32x4*>(d) = *reinterpret_cast<const u32x4*>(g);
+    if (vec && s0 + q * E + E <= written) {
+      *reinterpret_cast<u32x4*>(d) = *reinterpret_cast<const u32x4*>(g);
     } else {
 #pragma unroll
       for (int k = 0; k < E; ++k) d[k] = s0 + q * E + k < n ? g[k] : from_f32<T>(0.f);
@@ -463,8 +464,11 @@ void launch_planes_layernorm(const T* src, int C, const T* w, const T* b, T* dst
   const bool fused = C <= 512;
   const int64_t blocks = batch * n * ((n + kLnCols<T> - 1) / kLnCols<T>);
   const size_t lds = (size_t)(C < 512 ? C : 512) * 128;
+  // columns of a plane's row that the contraction wrote: the DMA one's all, zeros past n
+  const int64_t written = std::is_same<T, bf16>::value && pitch % 64 == 0 ? pitch : n;
   hipLaunchKernelGGL(planes_layernorm_kernel<T>, dim3((unsigned)blocks, (unsigned)((C + 511) / 512)), dim3(256), lds,
-                     st, src, C, fused ? w : nullptr, b, fused ? dst : tmp, n, pitch, blocked, pitch % 8 == 0 && al16(src), eps);
+                     st, src, C, fused ? w : nullptr, b, fused ? dst : tmp, n, pitch, written, blocked,
+                     pitch % 8 == 0 && al16(src), eps);
   if (!fused) launch_layernorm_rows<T>(tmp, w, b, dst, batch * n * n, C, eps, st);
 }
 template <typename T>

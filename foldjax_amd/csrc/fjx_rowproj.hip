@@ -412,7 +412,7 @@ __global__ __launch_bounds__(256) void trimul_epilogue_kernel(TriMulEpiloguePara
     else load_row_part<T>(p < nvalid ? P.x + (pos0 + p) * kC : nullptr, xr);
     // channel-major: channel ch of the tile at src + ch * n * pitch;
     // tile-blocked: the whole tile is one contiguous [128][ncols] block
-    const int ncols = (int)min<int64_t>(kTE, pitch - tl.s0);  // columns of o that exist
+    const int ncols = P.o_blocked ? (int)min<int64_t>(kTE, pitch - tl.s0) : nvalid;  // columns of o that are written
     const int64_t cstride = P.o_blocked ? ncols : n * pitch;
     const T* src = P.o_blocked ? P.o + (((int64_t)tl.b * n + tl.r) * pitch + tl.s0) * kC
                                : P.o + ((int64_t)tl.b * kC * n + tl.r) * pitch + tl.s0;

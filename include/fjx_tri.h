@@ -114,7 +114,7 @@ typedef struct fjx_trimul_args {
 } fjx_trimul_args;
 
 /* The workspace that the fastest kernels need: a, b and o with their rows padded
- * to 64 elements and, in float32 with c_z == c_h == 128, a and b as three bf16
+ * to 64 elements (float32 at general widths: 8) and, in float32 with c_z == c_h == 128, a and b as three bf16
  * planes each (16 bytes an element of a row in place of 12). fjx_trimul_fwd also
  * takes a smaller one that holds them unpadded and unsplit, each rounded up to
  * 256 bytes (c_h == 128 and c_z of 32, 64, 96 or 128: 3 * batch * n^2 * 128

@@ -72,6 +72,31 @@ def test_trimul_on_an_unpadded_workspace(batch, n, c_z, c_h, dtype, direction):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("c_z,c_h", [(128, 128), (64, 128), (96, 128), (384, 384), (264, 72), (128, 576)])
+@pytest.mark.parametrize("n", [1, 37, 70])
+def test_trimul_leaves_nothing_to_the_workspace(n, c_z, c_h, dtype, monkeypatch):
+    """Every byte that a call reads of its workspace it has written: NaN left
+    there changes nothing."""
+    say(f"trimul workspace contents n={n} {c_z} {c_h} {dtype}")
+    x = torch.randn(1, n, n, c_z, device="cuda").to(dtype)
+    w = P.pack_trimul_torch(P.trimul_to_protenix(syn.trimul_weights(c_z, c_h, seed=5)), dtype, "cuda")
+    empty = torch.empty
+
+    def filled(value):
+        def make(*shape, **kw):
+            t = empty(*shape, **kw)
+            return t.fill_(value) if kw.get("dtype") is torch.uint8 else t
+        return make
+
+    out = []
+    for value in (0, 0xFF):
+        monkeypatch.setattr(torch, "empty", filled(value))
+        out.append(kernels.trimul(x, None, w, "outgoing"))
+        torch.cuda.synchronize()
+    assert torch.isfinite(out[0]).all() and torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_trimul_where_the_full_workspace_does_not_fit(dtype, monkeypatch):
     n = 70
     say(f"trimul out of memory {dtype}")
