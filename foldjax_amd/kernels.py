@@ -65,6 +65,14 @@ def _need_shape(name: str, t: torch.Tensor | None, shape) -> None:
         raise ValueError(f"{name} must have shape {tuple(int(v) for v in shape)}, got {tuple(t.shape)}")
 
 
+def _shaped(*pairs) -> bool:
+    """Every tensor there and of its shape: the usual case, without a message made."""
+    for t, shape in pairs:
+        if t is None or t.shape != shape:
+            return False
+    return True
+
+
 def _rows_of(m: torch.Tensor | None, shape, dtype: torch.dtype, name: str) -> torch.Tensor | None:
     """A per-row (per-position) mask broadcast to ``shape`` in ``dtype``,
     contiguous, as the kernels index it."""
@@ -97,9 +105,9 @@ class TriMulWeights:
         """Shapes against the pair width ``c_z``; returns ``c_h``."""
         c_h = int(self.norm_out_weight.shape[0])
         in_, proj = (c_z,), (2 * c_h, c_z)
-        if (self.norm_in_weight.shape == in_ and self.norm_in_bias.shape == in_ and self.p_in_weight.shape == proj
-                and self.g_in_weight.shape == proj and self.norm_out_bias.shape == (c_h,)
-                and self.p_out_weight.shape == (c_z, c_h) and self.g_out_weight.shape == (c_z, c_z)):
+        if _shaped((self.norm_in_weight, in_), (self.norm_in_bias, in_), (self.p_in_weight, proj),
+                   (self.g_in_weight, proj), (self.norm_out_bias, (c_h,)), (self.p_out_weight, (c_z, c_h)),
+                   (self.g_out_weight, (c_z, c_z))):
             return c_h
         for name, shape in (("norm_in_weight", (c_z,)), ("norm_in_bias", (c_z,)), ("p_in_weight", (2 * c_h, c_z)),
                             ("g_in_weight", (2 * c_h, c_z)), ("norm_out_bias", (c_h,)), ("p_out_weight", (c_z, c_h)),
@@ -134,10 +142,9 @@ class TriAttnWeights:
         if hd % self.heads:
             raise ValueError(f"q projection width {hd} is not divisible by {self.heads} heads")
         in_, proj = (c_z,), (hd, c_z)
-        if (self.norm_weight.shape == in_ and self.norm_bias.shape == in_
-                and self.bias_weight.shape == (self.heads, c_z) and self.q_weight.shape == proj
-                and self.k_weight.shape == proj and self.v_weight.shape == proj
-                and (self.g_weight is None or self.g_weight.shape == proj) and self.o_weight.shape == (c_z, hd)):
+        if _shaped((self.norm_weight, in_), (self.norm_bias, in_), (self.bias_weight, (self.heads, c_z)),
+                   (self.q_weight, proj), (self.k_weight, proj), (self.v_weight, proj), (self.o_weight, (c_z, hd))
+                   ) and (self.g_weight is None or self.g_weight.shape == proj):
             return hd
         for name, shape in (("norm_weight", (c_z,)), ("norm_bias", (c_z,)), ("bias_weight", (self.heads, c_z)),
                             ("q_weight", (hd, c_z)), ("k_weight", (hd, c_z)), ("v_weight", (hd, c_z)),
@@ -164,8 +171,8 @@ class TransitionWeights:
     def check(self, c: int) -> int:
         """Shapes against the width ``c``; returns the hidden width."""
         hidden = int(self.w_a.shape[0])
-        if (self.norm_weight.shape == (c,) and self.norm_bias.shape == (c,) and self.w_a.shape == (hidden, c)
-                and self.w_b.shape == (hidden, c) and self.w_o.shape == (c, hidden)):
+        if _shaped((self.norm_weight, (c,)), (self.norm_bias, (c,)), (self.w_a, (hidden, c)),
+                   (self.w_b, (hidden, c)), (self.w_o, (c, hidden))):
             return hidden
         for name, shape in (("norm_weight", (c,)), ("norm_bias", (c,)), ("w_a", (hidden, c)), ("w_b", (hidden, c)),
                             ("w_o", (c, hidden))):
@@ -213,8 +220,8 @@ class SingleAttentionWeights:
         """Shapes against the single width ``c_s`` and (when z is read) the
         pair width ``c_z``."""
         sq = (c_s, c_s)
-        if not (self.q_weight.shape == sq and self.k_weight.shape == sq and self.v_weight.shape == sq
-                and self.g_weight.shape == sq and self.o_weight.shape == sq):
+        if not _shaped((self.q_weight, sq), (self.k_weight, sq), (self.v_weight, sq), (self.g_weight, sq),
+                       (self.o_weight, sq)):
             for name in ("q_weight", "k_weight", "v_weight", "g_weight", "o_weight"):
                 _need_shape(f"single attention weight {name}", getattr(self, name), sq)
         for name in ("q_bias", "pre_norm_weight", "pre_norm_bias"):

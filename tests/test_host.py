@@ -6,6 +6,8 @@ packing layouts, and the refusal of host tensors."""
 
 from __future__ import annotations
 
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -289,3 +291,23 @@ def test_neutral_triangle_kernel_knob():
     with pytest.raises(RuntimeError, match="JAX backend"):
         protenix.triangle_attention(_z(8), None, P.triattn_to_protenix(syn.triattn_weights()), num_heads=4,
                                     attention_backend=E.triangle_kernel("protenix", "xla"))
+
+
+def test_absent_weights_reach_the_general_checks():
+    """A weight that is None is no shape error (the library names required
+    weights itself); the others' shapes are still checked."""
+    dev = "cpu"
+    tm = P.pack_trimul_torch(P.trimul_to_protenix(syn.trimul_weights()), torch.float32, dev)
+    ta = P.pack_triattn_protenix(P.triattn_to_protenix(syn.triattn_weights()), torch.float32, dev)
+    tr = P.pack_transition_torch(P.transition_to_protenix(syn.transition_weights()), torch.float32, dev)
+    sq = torch.zeros(8, 8)
+    sa = kernels.SingleAttentionWeights(None, None, torch.ones(4), torch.zeros(4), torch.zeros(2, 4), sq, None, sq, sq,
+                                        sq, sq)
+    for w, field, args, want in ((tm, "norm_in_bias", (128,), 128), (ta, "norm_bias", (128,), 128),
+                                 (ta, "g_weight", (128,), 128), (tr, "norm_bias", (128,), 512),
+                                 (sa, "v_weight", (8, 4), None)):
+        absent = dataclasses.replace(w, **{field: None})
+        assert w.check(*args) == want and absent.check(*args) == want
+        other = "z_norm_weight" if w is sa else "w_o" if w is tr else "norm_out_bias" if w is tm else "o_weight"
+        with pytest.raises(ValueError, match=f"{other} must have shape"):
+            dataclasses.replace(absent, **{other: torch.zeros(3)}).check(*args)
