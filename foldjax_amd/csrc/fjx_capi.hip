@@ -309,7 +309,7 @@ int trimul_run(const fjx_trimul_args* a, bool tight, hipStream_t st) {
   bool o_blocked = false;  // the LDS-DMA contraction writes o tile-blocked for the epilogue
   rc = timed(K_TRIMUL_CONTRACT, st, "trimul_contract", [&] {
     if constexpr (std::is_same<T, bf16>::value) {
-      o_blocked = launch_contract(abuf, bbuf, obuf, a->n, ws.pitch, a->batch * 128, st, true);
+      o_blocked = launch_contract(abuf, bbuf, obuf, a->n, ws.pitch, a->batch * 128, st);
     } else if (ws.split) {
       launch_contract_split(at<bf16>(a->workspace, ws.a), at<bf16>(a->workspace, ws.b), obuf, a->n, ws.pitch, ws.plane,
                             a->batch * 128, st);
@@ -670,7 +670,7 @@ int trimul_generic_run(const fjx_trimul_args* a, bool tight, hipStream_t st) {
   bool blocked = false;
   rc = timed(K_TRIMUL_CONTRACT, st, "trimul_contract", [&] {
     if constexpr (std::is_same<T, bf16>::value) {
-      blocked = launch_contract(acm, bcm, ocm, n, pitch, B * ch, st, true);
+      blocked = launch_contract(acm, bcm, ocm, n, pitch, B * ch, st);
     } else {
       GemmParams<T, T> cp = {};
       cp.a = acm;

@@ -179,7 +179,8 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(GemmParams<T, TO> P) {
 
 // ---------------------------------------------------------------------------
 // Triangle contraction, bf16: for every batch c, O[c] = A[c] B[c]^T with all
-// three n x n and k-contiguous (channel-major a and b of the tri-mul).
+// three n x n and k-contiguous (channel-major a and b of the tri-mul), rows
+// `pitch` apart.
 // 256 x 256 output tile per 512-thread workgroup, 2 x 4 waves of 128 x 64;
 // k-tiles of 64 double-buffered in LDS with a register prefetch of the next
 // one. The accumulators are computed transposed (A operand = B rows) so each
@@ -190,7 +191,8 @@ constexpr int kCK = 64;
 constexpr int kCLd = kCK + 8;
 
 __global__ __launch_bounds__(512) void contract_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
-                                                       bf16* __restrict__ O, int64_t n, int64_t batches) {
+                                                       bf16* __restrict__ O, int64_t n, int64_t pitch,
+                                                       int64_t batches) {
   __shared__ __attribute__((aligned(16))) bf16 As[2][kCT][kCLd];
   __shared__ __attribute__((aligned(16))) bf16 Bs[2][kCT][kCLd];
 
@@ -201,8 +203,8 @@ __global__ __launch_bounds__(512) void contract_kernel(const bf16* __restrict__ 
   const int64_t tile = lid % (tpd * tpd);
   const int64_t m0 = (tile / tpd) * kCT;
   const int64_t n0 = (tile % tpd) * kCT;
-  const bf16* Ab = A + bat * n * n;
-  const bf16* Bb = B + bat * n * n;
+  const bf16* Ab = A + bat * n * pitch;
+  const bf16* Bb = B + bat * n * pitch;
 
   const int t = threadIdx.x;
   const int wave = t >> 6;
@@ -211,7 +213,7 @@ __global__ __launch_bounds__(512) void contract_kernel(const bf16* __restrict__ 
   const int lg = lane >> 4;
   const int wm = (wave >> 2) * 128;
   const int wn = (wave & 3) * 64;
-  const bool vec = (n % 8) == 0;
+  const bool vec = (pitch % 8) == 0;
 
   // global -> registers -> LDS: 256 rows x 8 chunks of 8 per operand, 4 chunks per thread
   bf16x8 ra[4], rb[4];
@@ -224,14 +226,14 @@ __global__ __launch_bounds__(512) void contract_kernel(const bf16* __restrict__ 
       const int64_t ga = m0 + row;
       const int64_t gb = n0 + row;
       if (vec && gk + 8 <= n) {
-        ra[it] = ga < n ? load8(Ab + ga * n + gk) : bf16x8{};
-        rb[it] = gb < n ? load8(Bb + gb * n + gk) : bf16x8{};
+        ra[it] = ga < n ? load8(Ab + ga * pitch + gk) : bf16x8{};
+        rb[it] = gb < n ? load8(Bb + gb * pitch + gk) : bf16x8{};
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const bool kin = gk + e < n;
-          ra[it][e] = (kin && ga < n) ? Ab[ga * n + gk + e] : static_cast<bf16>(0.f);
-          rb[it][e] = (kin && gb < n) ? Bb[gb * n + gk + e] : static_cast<bf16>(0.f);
+          ra[it][e] = (kin && ga < n) ? Ab[ga * pitch + gk + e] : static_cast<bf16>(0.f);
+          rb[it][e] = (kin && gb < n) ? Bb[gb * pitch + gk + e] : static_cast<bf16>(0.f);
         }
       }
     }
@@ -274,8 +276,8 @@ __global__ __launch_bounds__(512) void contract_kernel(const bf16* __restrict__ 
     __syncthreads();
   }
 
-  bf16* Ob = O + bat * n * n;
-  const bool vec4 = (n % 4) == 0;
+  bf16* Ob = O + bat * n * pitch;
+  const bool vec4 = (pitch % 4) == 0;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int64_t row = m0 + wm + 16 * i + li;
@@ -284,7 +286,7 @@ __global__ __launch_bounds__(512) void contract_kernel(const bf16* __restrict__ 
     for (int j = 0; j < 4; ++j) {
       const int64_t col = n0 + wn + 16 * j + 4 * lg;
       float v[4] = {acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]};
-      bf16* dst = Ob + row * n + col;
+      bf16* dst = Ob + row * pitch + col;
       if (vec4 && col + 4 <= n) {
         store4f(dst, v);
       } else {
@@ -574,7 +576,8 @@ static void launch_contract_dma(const bf16* a, const bf16* b, bf16* o, int64_t n
 // ---------------------------------------------------------------------------
 // The contraction in fp32 on the bf16 matrix cores: a and b arrive as three
 // bf16 planes each (Split8, written so by the prologue: no conversion here),
-// `plane` elements apart, rows `pitch` apart as above; o is fp32. 128 x 128
+// `plane` elements apart, rows `pitch` apart as above; o is fp32 and
+// tile-blocked. 128 x 128
 // output tiles, 512 threads (2 x 4 waves of 64 x 32), two stages of 32 k with
 // the six planes of the operands in 96 KB; six MFMAs per tile and 32 k.
 // Rows of 64 bytes: chunk c of row r in slot 4 r + (c ^ ((r / 4) % 4)), which
@@ -586,7 +589,7 @@ static void launch_contract_dma(const bf16* a, const bf16* b, bf16* o, int64_t n
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(512) void contract_split_kernel(const bf16* __restrict__ A, const bf16* __restrict__ B,
                                                              float* __restrict__ O, int n, int pitch, int64_t plane,
-                                                             int64_t batches, bool blocked) {
+                                                             int64_t batches) {
   constexpr int BT = 128, DK = 32;
   constexpr int MI = 4, NJ = 2;  // 16-row and 16-column tiles per wave
   constexpr int kStores = MI * NJ;
@@ -695,10 +698,9 @@ __global__ __launch_bounds__(512) void contract_split_kernel(const bf16* __restr
     // transposed accumulators: a lane holds 4 consecutive columns of a row;
     // the wave's 32 columns are all within the pitch or none
     const int c0 = cur.n0 + wn;
-    const int rstride = blocked ? pitch * tile::kC : pitch;
-    const float* Ob = blocked ? O + ((cur.bat >> 7) * n + cur.m0) * (int64_t)rstride + (int64_t)(c0 & ~63) * tile::kC +
-                                    (cur.bat & 127) * 64 + (c0 & 63)
-                              : O + (cur.bat * n + cur.m0) * (int64_t)rstride + c0;
+    const int rstride = pitch * tile::kC;
+    const float* Ob = O + ((cur.bat >> 7) * n + cur.m0) * (int64_t)rstride + (int64_t)(c0 & ~63) * tile::kC +
+                      (cur.bat & 127) * 64 + (c0 & 63);
     const __amdgpu_buffer_rsrc_t ro = crsrc(Ob, c0 < pitch ? ((int64_t)(n - cur.m0 - 1) * rstride + 32) * 4 : 0);
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
@@ -726,13 +728,12 @@ void launch_contract_split(const bf16* a, const bf16* b, float* o, int64_t n, in
   const int64_t cap = std::max<int64_t>(kNumXcd, tile::resident_blocks(k, 512) / kNumXcd * kNumXcd);
   const int64_t grid = std::min<int64_t>(cap, (total + kNumXcd - 1) / kNumXcd * kNumXcd);
   hipLaunchKernelGGL(contract_split_kernel, dim3((unsigned)grid), dim3(512), 0, st, a, b, o, (int)n, (int)pitch, plane,
-                     batches, true);
+                     batches);
 }
 
-bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t pitch, int64_t batches, hipStream_t st,
-                     bool blocked) {
+bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t pitch, int64_t batches, hipStream_t st) {
   if (pitch % 64 == 0) {
-    blocked = blocked && batches % tile::kC == 0;
+    const bool blocked = batches % tile::kC == 0;
     // 128-wide tiles where 256-wide ones would leave CUs without a tile or
     // compute a quarter more padding: whole tri-mul, 128 against 256: 51.8 / 54.5
     // us at n = 256 and 73.5 / 83.3 at 300; 256 elsewhere, its operands being
@@ -744,9 +745,10 @@ bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t p
       launch_contract_dma<256>(a, b, o, n, pitch, batches, st, blocked);
     return blocked;
   }
-  // rows not padded (a fixed scratch that does not hold the padding)
+  // rows not padded (a workspace that does not hold the padding)
   const int64_t tpd = (n + kCT - 1) / kCT;
-  hipLaunchKernelGGL(contract_kernel, dim3((unsigned)(batches * tpd * tpd)), dim3(512), 0, st, a, b, o, n, batches);
+  hipLaunchKernelGGL(contract_kernel, dim3((unsigned)(batches * tpd * tpd)), dim3(512), 0, st, a, b, o, n, pitch,
+                     batches);
   return false;
 }
 

@@ -18,7 +18,7 @@ struct TriMulPrologueParams {
   T* a_cm;          // [B][128][N][pitch] virtual grid; columns N .. pitch-1 are written as zeros
   T* b_cm;
   int64_t n;
-  int64_t pitch;    // elements per row of a and b: N rounded up to 8, or N (tight)
+  int64_t pitch;    // elements per row of a and b: N rounded up to 64, or N (tight)
   float eps;
   int transpose;    // 1 for the incoming direction
   int cw;           // channels of x (and rows of w_p/w_g) when below 128 (a multiple of 32); 0: 128
@@ -63,10 +63,9 @@ struct TriMulEpilogueParams {
   T* out;
   int64_t n;
   float eps;
-  int64_t pitch;      // elements per row of o: N rounded up to 8, or N (tight)
+  int64_t pitch;      // elements per row of o: N rounded up to 64, or N (tight)
   // o tile-blocked (the LDS-DMA contraction's output): a row's columns in
-  // blocks of 64, [B][N rows][pitch / 64 blocks][128 channels][64], the last
-  // block of a row pitch % 64 columns wide when that is not 0
+  // blocks of 64, [B][N rows][pitch / 64 blocks][128 channels][64]
   bool o_blocked;
   int cw;             // channels of x / out (k of w_gout, rows of both weights) when below 128; 0: 128
 };
@@ -200,6 +199,7 @@ struct FlashParams {
 
 template <typename T>
 void launch_trimul_prologue(const TriMulPrologueParams<T>& p, int64_t batch, hipStream_t st);
+// float: below 128 channels (launch_triattn_prologue_split takes 128)
 template <typename T>
 void launch_triattn_prologue(const TriAttnPrologueParams<T>& p, int64_t batch, hipStream_t st);
 template <typename T>
@@ -215,16 +215,17 @@ bool launch_gemm_dma(const GemmParams<bf16, bf16>& p, hipStream_t st);
 bool gemm_dma_ok(const GemmParams<bf16, bf16>& p);
 // triangle contraction, bf16: o[c] = a[c] b[c]^T for c < batches, each n rows
 // of n elements, rows `pitch` apart in a, b and o. A pitch that is a multiple
-// of 8 (with zeros past n in a and b) runs the LDS-DMA kernel; pitch == n any n.
-// blocked: write o tile-blocked (TriMulEpilogueParams::o_blocked; needs
-// batches a multiple of 128), else [batches][n][pitch]; returns whether it
-// wrote the blocked layout
-bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t pitch, int64_t batches, hipStream_t st,
-                     bool blocked = false);
+// of 64 (with zeros past n in a and b) runs the LDS-DMA kernel, which writes
+// whole rows of o, any other the register-staged one, which writes n columns.
+// o comes tile-blocked (TriMulEpilogueParams::o_blocked) from the former where
+// batches is a multiple of 128, else as [batches][n][pitch]; returns whether it
+// is blocked
+bool launch_contract(const bf16* a, const bf16* b, bf16* o, int64_t n, int64_t pitch, int64_t batches, hipStream_t st);
 // the same in fp32 from bf16 planes (Split8) of a and b, `plane` elements
 // apart; pitch a multiple of 64, batches of 128, o tile-blocked
 void launch_contract_split(const bf16* a, const bf16* b, float* o, int64_t n, int64_t pitch, int64_t plane,
                            int64_t batches, hipStream_t st);
+// float: below 128 channels (launch_transition_split takes 128)
 template <typename T>
 void launch_transition(const TransitionParams<T>& p, int c, hipStream_t st);
 // fp32 on the bf16 matrix cores (fjx_rowproj_f32.hip), c_z = 128: a and b of

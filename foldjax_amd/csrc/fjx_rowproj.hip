@@ -54,8 +54,8 @@ namespace {
 //   a_cm/b_cm: [B][128][N][pitch] channel-major in the virtual grid
 //   (contraction operands with the contracted axis contiguous), each
 //   mask * sigmoid(x_ln g_in^T) * (x_ln p_in^T), zero past column N.
-// A pitch that is a multiple of 8 makes every store 16 bytes whatever N is
-// (rows N apart: 2-byte stores when N is odd, 568 against 213 us at N = 1003).
+// A pitch that is a multiple of 8 (it is N rounded up to 64, or N itself where
+// the workspace does not hold that) makes every store 16 bytes whatever N is (rows N apart: 2-byte stores when N is odd, 568 against 213 us at N = 1003).
 // kNarrow: x has P.cw < 128 channels (a multiple of 32); the tile's channels
 // past cw are held at zero (zero LayerNorm affine, zero weight columns). NB:
 // the 32-channel blocks of x worked on (cw / 32 when it is known at compile
@@ -411,9 +411,9 @@ __global__ __launch_bounds__(256) void trimul_epilogue_kernel(TriMulEpiloguePara
     if constexpr (kNarrow) load_row_part_w<T, NB>(p < nvalid ? P.x + (pos0 + p) * cw : nullptr, xr, cw);
     else load_row_part<T>(p < nvalid ? P.x + (pos0 + p) * kC : nullptr, xr);
     // channel-major: channel ch of the tile at src + ch * n * pitch;
-    // tile-blocked: the whole tile is one contiguous [128][ncols] block
-    const int ncols = P.o_blocked ? (int)min<int64_t>(kTE, pitch - tl.s0) : nvalid;  // columns of o that are written
-    const int64_t cstride = P.o_blocked ? ncols : n * pitch;
+    // tile-blocked: the whole tile is one contiguous [128][64] block
+    const int ncols = P.o_blocked ? kTE : nvalid;  // columns of o that are written
+    const int64_t cstride = P.o_blocked ? kTE : n * pitch;
     const T* src = P.o_blocked ? P.o + (((int64_t)tl.b * n + tl.r) * pitch + tl.s0) * kC
                                : P.o + ((int64_t)tl.b * kC * n + tl.r) * pitch + tl.s0;
 #pragma unroll
@@ -698,9 +698,11 @@ void launch_triattn_prologue(const TriAttnPrologueParams<T>& p, int64_t batch, h
       return;
     }
   }
-  launch_persistent(p.cw == 64 ? triattn_prologue_kernel<T, true, 2>
-                    : p.cw ? triattn_prologue_kernel<T, true> : triattn_prologue_kernel<T, false>,
-                    p, 512, ntiles, st);
+  auto kern = p.cw == 64 ? triattn_prologue_kernel<T, true, 2> : triattn_prologue_kernel<T, true>;
+  if constexpr (std::is_same<T, bf16>::value) {
+    if (!p.cw) kern = triattn_prologue_kernel<T, false>;
+  }
+  launch_persistent(kern, p, 512, ntiles, st);
 }
 template <typename T>
 void launch_trimul_epilogue(const TriMulEpilogueParams<T>& p, int64_t batch, hipStream_t st) {

@@ -349,9 +349,9 @@ __device__ __forceinline__ void transition128_body(const TransitionParams<T>& P)
   }
 }
 
-template <typename T, int RT = 8>
-__global__ __launch_bounds__(512) void transition128_kernel(TransitionParams<T> P) {
-  transition128_body<T, false, false, 4, RT>(P);
+template <int RT>
+__global__ __launch_bounds__(512) void transition128_kernel(TransitionParams<bf16> P) {
+  transition128_body<bf16, false, false, 4, RT>(P);
 }
 template <typename T, int NB, int RT = 8>
 __global__ __launch_bounds__(512) void transition_narrow_kernel(TransitionParams<T> P) {
@@ -379,12 +379,9 @@ static void launch_transition_rt(const TransitionParams<T>& p, int c, hipStream_
     return;
   }
   if constexpr (std::is_same<T, bf16>::value) {
-    if (p.pbf_out) {
-      hipLaunchKernelGGL(transition128_pbf32_kernel<RT>, grid, dim3(512), 0, st, p);
-      return;
-    }
+    if (p.pbf_out) hipLaunchKernelGGL(transition128_pbf32_kernel<RT>, grid, dim3(512), 0, st, p);
+    else hipLaunchKernelGGL(transition128_kernel<RT>, grid, dim3(512), 0, st, p);
   }
-  hipLaunchKernelGGL((transition128_kernel<T, RT>), grid, dim3(512), 0, st, p);
 }
 
 template <typename T>
