@@ -4,10 +4,10 @@
 Both run the same kernels on the same inputs, one with a caller workspace and
 one on the library's static per-GPU scratch, so their outputs must be
 bit-identical. Two calls in a row, the second with a smaller input (the
-scratch keeps the first call's contents), cover both contraction kernels
-(n a multiple of 256: the LDS-DMA kernel; otherwise the register-staged one)
-and both dtypes. A shape whose workspace exceeds the scratch is refused on
-the host before anything is launched.
+scratch keeps the first call's contents), in both dtypes, run the LDS-DMA
+contractions on whole and on padded rows; batches that run on unpadded rows
+or in pieces are in test_gpu_ragged.py. A shape whose workspace exceeds the
+scratch is refused on the host before anything is launched.
 """
 
 from __future__ import annotations
@@ -44,7 +44,7 @@ def test_noalloc_matches_workspace_entry(dt):
 
 def test_noalloc_refuses_shapes_beyond_scratch():
     say("noalloc trimul refusal n=600")
-    n = 600  # bf16 workspace 3 * 600^2 * 128 * 2 B = 276 MB > 256 MiB
+    n = 600  # bf16, unpadded: 3 * 600^2 * 128 * 2 B = 276 MB > 256 MiB
     lib = _lib.load()
     assert lib.fjx_trimul_workspace_size(1, n, 128, 128, _lib.FJX_DTYPE_BF16) > _lib.NOALLOC_SCRATCH_BYTES
     z = torch.zeros((n, n, 128), device="cuda", dtype=torch.bfloat16)
