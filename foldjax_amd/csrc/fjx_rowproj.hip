@@ -111,10 +111,15 @@ __global__ __launch_bounds__(512) void trimul_prologue_kernel(TriMulProloguePara
     auto pos_of = [&](int ss) {
       return (int64_t)tl.b * nn + (P.transpose ? (int64_t)ss * n + tl.r : (int64_t)tl.r * n + ss);
     };
-    if constexpr (kNarrow) load_row_part_w<T, NB>(valid ? P.x + pos_of(s) * cw : nullptr, xr, cw);
-    else load_row_part<T>(valid ? P.x + pos_of(s) * kC : nullptr, xr);
+    // columns past n repeat the tile's first one: their products, times 0, are 0
+    // unless that column's own spoil the row already (the products of a zero
+    // row's LayerNorm can be NaN where no column's are: with eps 0, or an
+    // infinite gate weight and a zero LayerNorm bias)
+    const int64_t pos = pos_of(valid ? s : tl.s0);
+    if constexpr (kNarrow) load_row_part_w<T, NB>(p < TP ? P.x + pos * cw : nullptr, xr, cw);
+    else load_row_part<T>(p < TP ? P.x + pos * kC : nullptr, xr);
     mvalid = valid;
-    if (P.mask) mraw = P.mask[pos_of(valid ? s : tl.s0)];
+    if (P.mask) mraw = P.mask[pos];
   };
 
   int64_t tile = blockIdx.x;

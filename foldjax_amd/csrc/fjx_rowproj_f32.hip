@@ -5,8 +5,8 @@
 // the fp32 instances of those kernels (trimul prologue at N = 256: the fp32
 // matrix pipe was busy 64 % of its 87 us) at no larger error (relative to
 // float64, whole tri-mul at N = 256: 4.8e-7 before, 3.8e-7 now). At N = 245:
-// tri-mul prologue 100 -> 54 us, epilogue 70 -> 46; tri-attn prologue 69 -> 51,
-// epilogue 60 -> 48; transition 248 -> 202. What bounds them now is the sum of
+// tri-mul prologue 100 -> 57 us, epilogue 70 -> 47; tri-attn prologue 69 -> 52,
+// epilogue 60 -> 49; transition 248 -> 210. What bounds them now is the sum of
 // MFMA, LDS reads, LayerNorm and splits: one workgroup fits a CU, and its two
 // waves per SIMD mostly run the same phase.
 //
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(512) void trimul_prologue_split_kernel(TriMulProlog
     mvalid = s < n;
     const int ss = mvalid ? s : tl.s0;
     const int64_t pos = tl.b * nn + (P.transpose ? ss * n + tl.r : tl.r * n + ss);
-    load_part(mvalid ? P.x + pos * kC : nullptr, xr);
+    load_part(P.x + pos * kC, xr);  // columns past n repeat the tile's first one (trimul_prologue_kernel)
     if (P.mask) mraw = P.mask[pos];
   };
   bool plain;

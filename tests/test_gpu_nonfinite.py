@@ -159,3 +159,24 @@ def test_core_nan_of_one_query(where, rows, n, dtype):
     # rounding of the probabilities and of the output)
     diff = torch.where(bad[..., None], 0.0, (got - clean).float()).abs().max()
     assert float(diff) <= (3e-2 if dtype == torch.bfloat16 else 1e-5) * float(clean.float().abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("c_z,c_h", [(128, 128), (64, 128), (96, 128), (384, 384), (264, 72)])
+@pytest.mark.parametrize("n", [37, 70, 200])
+def test_trimul_padding_is_zero(n, c_z, c_h, dtype):
+    """The operands' rows are padded past n. The LayerNorm of the padding's zero
+    rows is NaN at eps = 0, and an infinite gate weight times a zero LayerNorm
+    bias is too; neither may reach the contraction."""
+    say(f"trimul padding n={n} {c_z} {c_h} {dtype}")
+    w = P.pack_trimul_torch(P.trimul_to_protenix(syn.trimul_weights(c_z, c_h, seed=3)), dtype, "cuda")
+    x = _x((1, n, n, c_z), 4).cuda().to(dtype)
+    for direction in ("outgoing", "incoming"):
+        got = kernels.trimul(x, None, w, direction, eps=0.0)
+        want = kernels.trimul(x, None, w, direction, eps=1e-30)  # the same LayerNorms on rows that vary
+        torch.cuda.synchronize()
+        assert torch.isfinite(want).all() and torch.equal(got, want)
+    inf = dataclasses.replace(_set(w, "g_in_weight", (5, 17), INF), norm_in_bias=torch.zeros_like(w.norm_in_bias))
+    got = kernels.trimul(x, None, inf, "outgoing")
+    torch.cuda.synchronize()
+    assert torch.isfinite(got).all()
