@@ -132,8 +132,8 @@ __global__ void pad_qk_kernel(const T* __restrict__ src, T* __restrict__ dst, in
   }
 }
 
-// The other operands of the attention core, in one launch of three block
-// ranges of 256 threads:
+// The other operands of the attention core, in one launch of three ranges of
+// 256-thread blocks:
 //   v: [heads_rows][n][32] -> vt [heads_rows][32][np] (zero past n), a 128-key
 //      piece per block through LDS, 16-byte accesses on both sides;
 //   bias: [planes][n][n] -> [planes][np][np] times log2 e (zero past n), a
@@ -150,57 +150,60 @@ __global__ __launch_bounds__(256) void core_prep_kernel(const T* __restrict__ v,
                                                         int64_t n, int64_t np, int64_t vblocks, int64_t bblocks,
                                                         int64_t planes, int64_t mrows) {
   typedef typename Frag<T>::type Frag8;
+  // rows of 128 keys plus a 16-byte pad: a thread holds 8 dims of a pair of
+  // keys and writes them as pairs, 8 rows apart
+  __shared__ __attribute__((aligned(16))) T tile[32][kPrepKeys + 8];
   const int t = threadIdx.x;
-  if (blockIdx.x < vblocks) {
-    // rows of 128 keys plus a 16-byte pad: a thread holds 8 dims of a pair of
-    // keys and writes them as pairs, 8 rows apart
-    __shared__ __attribute__((aligned(16))) T tile[32][kPrepKeys + 8];
-    const int64_t pieces = (np + kPrepKeys - 1) / kPrepKeys;
-    const int64_t hr = blockIdx.x / pieces;
-    const int64_t k0 = (blockIdx.x - hr * pieces) * kPrepKeys;
-    const int pair = t >> 2, d0 = 8 * (t & 3);
-    Frag8 r[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int64_t key = k0 + 2 * pair + u;
-      if (key < n) {
-        r[u] = load8(v + (hr * n + key) * 32 + d0);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) r[u][e] = from_f32<T>(0.f);
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      typedef T T2 __attribute__((ext_vector_type(2)));
-      *reinterpret_cast<T2*>(&tile[d0 + e][2 * pair]) = T2{r[0][e], r[1][e]};
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int d = (t >> 4) + 16 * u, c = 8 * (t & 15);  // 16 lanes: one dim's 128 keys
-      if (k0 + c < np) store8(vt + (hr * 32 + d) * np + k0 + c, load8(&tile[d][c]));
-    }
-    return;
-  }
   const int lane = t & 63;
-  int64_t row = (blockIdx.x - vblocks) * 4 + (t >> 6);
-  if (blockIdx.x < vblocks + bblocks) {
-    if (row >= planes * np) return;
-    const int64_t pl = row / np, q = row - pl * np;
-    const T* src = bias + (pl * n + q) * n;
-    for (int64_t k = 8 * lane; k < np; k += 512) {
-      float f[8];
+  for (int64_t blk = blockIdx.x; blk < vblocks + bblocks + (mrows + 3) / 4; blk += gridDim.x) {
+    if (blk < vblocks) {
+      const int64_t pieces = (np + kPrepKeys - 1) / kPrepKeys;
+      const int64_t hr = blk / pieces;
+      const int64_t k0 = (blk - hr * pieces) * kPrepKeys;
+      const int pair = t >> 2, d0 = 8 * (t & 3);
+      Frag8 r[2];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = q < n && k + e < n ? to_f32(src[k + e]) * kLog2e : 0.f;
-      store8(bias_p + row * np + k, pack8<T>(f));
+      for (int u = 0; u < 2; ++u) {
+        const int64_t key = k0 + 2 * pair + u;
+        if (key < n) {
+          r[u] = load8(v + (hr * n + key) * 32 + d0);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) r[u][e] = from_f32<T>(0.f);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        typedef T T2 __attribute__((ext_vector_type(2)));
+        *reinterpret_cast<T2*>(&tile[d0 + e][2 * pair]) = T2{r[0][e], r[1][e]};
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int d = (t >> 4) + 16 * u, c = 8 * (t & 15);  // 16 lanes: one dim's 128 keys
+        if (k0 + c < np) store8(vt + (hr * 32 + d) * np + k0 + c, load8(&tile[d][c]));
+      }
+      if (blk + gridDim.x < vblocks) __syncthreads();  // the tile is free for the next piece
+      continue;
     }
-    return;
+    int64_t row = (blk - vblocks) * 4 + (t >> 6);
+    if (blk < vblocks + bblocks) {
+      if (row >= planes * np) continue;
+      const int64_t pl = row / np, q = row - pl * np;
+      const T* src = bias + (pl * n + q) * n;
+      for (int64_t k = 8 * lane; k < np; k += 512) {
+        float f[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = q < n && k + e < n ? to_f32(src[k + e]) * kLog2e : 0.f;
+        store8(bias_p + row * np + k, pack8<T>(f));
+      }
+      continue;
+    }
+    row -= 4 * bblocks;
+    if (row >= mrows) continue;
+    for (int64_t k = lane; k < np; k += 64)
+      mask_p[row * np + k] = k < n ? (mask ? mask[row * n + k] * kLog2e : 0.f) : -INFINITY;
   }
-  row -= 4 * bblocks;
-  if (row >= mrows) return;
-  for (int64_t k = lane; k < np; k += 64)
-    mask_p[row * np + k] = k < n ? (mask ? mask[row * n + k] * kLog2e : 0.f) : -INFINITY;
 }
 
 dim3 grid_for(int64_t total) {
@@ -464,7 +467,9 @@ int core_run(const fjx_triattn_core_args* a, hipStream_t st) {
     }
     const int64_t planes = a->batch * a->heads, mrows = a->batch * a->rows;
     const int64_t vblocks = hr * ((np + kPrepKeys - 1) / kPrepKeys), bblocks = (planes * np + 3) / 4;
-    hipLaunchKernelGGL(core_prep_kernel<T>, dim3((unsigned)(vblocks + bblocks + (mrows + 3) / 4)), dim3(256), 0, st,
+    // a launch takes fewer than 2^32 threads; past 2^23 blocks they walk
+    const int64_t blocks = std::min<int64_t>(vblocks + bblocks + (mrows + 3) / 4, (int64_t)1 << 23);
+    hipLaunchKernelGGL(core_prep_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st,
                        static_cast<const T*>(a->v), vt, static_cast<const T*>(a->tri_bias), bias, a->mask_bias, mb, n,
                        np, vblocks, bblocks, planes, mrows);
   });

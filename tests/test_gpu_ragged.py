@@ -236,3 +236,17 @@ def test_transition_rows_do_not_depend_on_the_tile(n, c, bias):
         assert torch.equal(getattr(got_pb, "bias", got_pb)[0], getattr(want_pb, "bias", want_pb)[1])
     assert torch.isfinite(got.float()).all()
     assert torch.equal(got[0], want[1])
+
+
+def test_triattn_core_of_very_many_rows():
+    """65 items of 65535 one-token rows and 4 heads: 17 million head rows, more
+    blocks than one launch takes. One key has probability one: the output is v."""
+    batch, rows = 65, 65535
+    say(f"triattn core batch={batch} rows={rows}")
+    v = torch.randn(batch, rows, 4, 1, 32, device="cuda", dtype=torch.bfloat16)
+    tb = torch.zeros(batch, 1, 4, 1, 1, device="cuda", dtype=torch.bfloat16)
+    got = kernels.triattn_core(v, v, v, tb, None, scale=0.05)
+    torch.cuda.synchronize()
+    assert torch.equal(got, v)
+    del got, v
+    torch.cuda.empty_cache()  # 70 GB of workspace
