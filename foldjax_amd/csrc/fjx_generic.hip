@@ -37,8 +37,8 @@ dim3 stride_grid(int64_t total) {
 template <typename T>
 __global__ __launch_bounds__(256) void ln_grid_kernel(const T* __restrict__ x, const T* __restrict__ w,
                                                       const T* __restrict__ b, T* __restrict__ y, int64_t rows,
-                                                      int64_t n, int c, float eps, int t) {
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+                                                      int64_t n, int c, float eps, int t, int64_t first) {
+  const int64_t row = (first + blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
   const int64_t nn = n * n;
@@ -79,11 +79,11 @@ template <typename T>
 __global__ __launch_bounds__(256) void to_planes_kernel(const T* __restrict__ src, int64_t ld, int C,
                                                         const T* __restrict__ mask, T* __restrict__ A,
                                                         T* __restrict__ B, int64_t n, int64_t pitch, int t, bool vs,
-                                                        bool vd) {
+                                                        bool vd, int64_t first) {
   __shared__ float tile[64][65];
   const int ctiles = (2 * C + 63) / 64;
   const int64_t stiles = (pitch + 63) / 64;
-  int64_t id = blockIdx.x;
+  int64_t id = first + blockIdx.x;
   const int cb = (int)(id % ctiles) * 64;
   id /= ctiles;
   const int64_t s0 = id % stiles * 64;
@@ -157,13 +157,15 @@ template <typename T>
 __global__ __launch_bounds__(256) void planes_layernorm_kernel(const T* __restrict__ src, int C,
                                                                const T* __restrict__ w, const T* __restrict__ b,
                                                                T* __restrict__ dst, int64_t n, int64_t pitch,
-                                                               int64_t written, bool blocked, bool vec, float eps) {
+                                                               int64_t written, bool blocked, bool vec, float eps,
+                                                               int64_t first) {
   constexpr int PB = kLnCols<T>, E = 16 / (int)sizeof(T);  // columns per tile, elements per chunk
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   T* S = reinterpret_cast<T*>(smem);
   const int64_t stiles = (n + PB - 1) / PB;
-  const int64_t s0 = blockIdx.x % stiles * PB;
-  const int64_t br = blockIdx.x / stiles, r = br % n, bb = br / n;
+  const int64_t id = first + blockIdx.x;
+  const int64_t s0 = id % stiles * PB;
+  const int64_t br = id / stiles, r = br % n, bb = br / n;
   const int c0 = blockIdx.y * 512, cn = C - c0 < 512 ? C - c0 : 512;
   // channel c of the item at (p / 128) gs + (p % 128) cs, p = item C + c
   const int64_t cs = blocked ? 64 : n * pitch, gs = 128 * n * pitch;
@@ -294,8 +296,8 @@ __global__ void gate_rows_kernel(T* __restrict__ o, const T* __restrict__ g, int
 template <typename T>
 __global__ __launch_bounds__(256) void ln_grid8_kernel(const T* __restrict__ x, const T* __restrict__ w,
                                                        const T* __restrict__ b, T* __restrict__ y, int64_t rows,
-                                                       int64_t n, int c, float eps, int t) {
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+                                                       int64_t n, int c, float eps, int t, int64_t first) {
+  const int64_t row = (first + blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int64_t nn = n * n;
   const int64_t bb = row / nn;
@@ -441,20 +443,21 @@ template <typename T>
 void launch_ln_grid(const T* x, const T* w, const T* b, T* y, int64_t batch, int64_t n, int c, float eps, int t,
                     hipStream_t st) {
   const int64_t rows = batch * n * n;
-  if (c % 8 == 0 && c <= 512 && al16(x) && al16(w) && al16(b) && al16(y))
-    hipLaunchKernelGGL(ln_grid8_kernel<T>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, x, w, b, y, rows, n, c,
-                       eps, t);
-  else
-    hipLaunchKernelGGL(ln_grid_kernel<T>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, x, w, b, y, rows, n, c,
-                       eps, t);
+  const bool vec = c % 8 == 0 && c <= 512 && al16(x) && al16(w) && al16(b) && al16(y);
+  for_pieces((rows + 3) / 4, [&](int64_t first, unsigned count) {
+    hipLaunchKernelGGL(vec ? ln_grid8_kernel<T> : ln_grid_kernel<T>, dim3(count), dim3(256), 0, st, x, w, b, y, rows, n,
+                       c, eps, t, first);
+  });
 }
 template <typename T>
 void launch_to_planes(const T* src, int64_t ld, int C, const T* mask, T* a, T* b, int64_t batch, int64_t n,
                       int64_t pitch, int t, hipStream_t st) {
   const int64_t blocks = batch * n * ((pitch + 63) / 64) * ((2 * C + 63) / 64);
   const bool vs = C % 8 == 0 && ld % 8 == 0 && al16(src), vd = pitch % 8 == 0 && al16(a) && al16(b);
-  hipLaunchKernelGGL(to_planes_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, st, src, ld, C, mask, a, b, n, pitch,
-                     t, vs, vd);
+  for_pieces(blocks, [&](int64_t first, unsigned count) {
+    hipLaunchKernelGGL(to_planes_kernel<T>, dim3(count), dim3(256), 0, st, src, ld, C, mask, a, b, n, pitch, t, vs, vd,
+                       first);
+  });
 }
 template <typename T>
 void launch_planes_layernorm(const T* src, int C, const T* w, const T* b, T* dst, T* tmp, int64_t batch, int64_t n,
@@ -466,9 +469,11 @@ void launch_planes_layernorm(const T* src, int C, const T* w, const T* b, T* dst
   const size_t lds = (size_t)(C < 512 ? C : 512) * 128;
   // columns of a plane's row that the contraction wrote: the DMA one's all, zeros past n
   const int64_t written = std::is_same<T, bf16>::value && pitch % 64 == 0 ? pitch : n;
-  hipLaunchKernelGGL(planes_layernorm_kernel<T>, dim3((unsigned)blocks, (unsigned)((C + 511) / 512)), dim3(256), lds,
-                     st, src, C, fused ? w : nullptr, b, fused ? dst : tmp, n, pitch, written, blocked,
-                     pitch % 8 == 0 && al16(src), eps);
+  for_pieces(blocks, [&](int64_t first, unsigned count) {
+    hipLaunchKernelGGL(planes_layernorm_kernel<T>, dim3(count, (unsigned)((C + 511) / 512)), dim3(256), lds, st, src, C,
+                       fused ? w : nullptr, b, fused ? dst : tmp, n, pitch, written, blocked,
+                       pitch % 8 == 0 && al16(src), eps, first);
+  });
   if (!fused) launch_layernorm_rows<T>(tmp, w, b, dst, batch * n * n, C, eps, st);
 }
 template <typename T>

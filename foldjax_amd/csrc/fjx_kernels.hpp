@@ -7,6 +7,15 @@
 
 namespace fjx {
 
+// A launch takes fewer than 2^32 threads; past them its block count wraps, with
+// no error. Launches of up to 2^23 blocks of 256 threads, from block `first` on
+template <typename F>
+void for_pieces(int64_t blocks, F launch) {
+  constexpr int64_t kMax = (int64_t)1 << 23;
+  for (int64_t first = 0; first < blocks; first += kMax)
+    launch(first, (unsigned)(blocks - first < kMax ? blocks - first : kMax));
+}
+
 template <typename T>
 struct TriMulPrologueParams {
   const T* x;     // [B][N][N][128]

@@ -245,12 +245,11 @@ dim3 grid_stride(int64_t total) {
 template <typename T>
 void launch_layernorm_rows(const T* x, const T* w, const T* b, T* y, int64_t rows, int c, float eps, hipStream_t st) {
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (c % 8 == 0 && c <= 512 && al16(x) && al16(w) && al16(b) && al16(y))
-    hipLaunchKernelGGL(layernorm_rows8_kernel<T>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, x, w, b, y, rows,
-                       c, eps);
-  else
-    hipLaunchKernelGGL(layernorm_rows_kernel<T>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, x, w, b, y, rows,
-                       c, eps);
+  const bool vec = c % 8 == 0 && c <= 512 && al16(x) && al16(w) && al16(b) && al16(y);
+  for_pieces((rows + 3) / 4, [&](int64_t first, unsigned count) {
+    hipLaunchKernelGGL(vec ? layernorm_rows8_kernel<T> : layernorm_rows_kernel<T>, dim3(count), dim3(256), 0, st,
+                       x + 4 * first * c, w, b, y + 4 * first * c, rows - 4 * first, c, eps);
+  });
 }
 template <typename T>
 void launch_split_heads(const T* qkv, int64_t ld, int64_t batch, int64_t n, int64_t np, int heads, int dh,

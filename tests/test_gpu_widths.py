@@ -379,3 +379,32 @@ def test_transition_wide_256_wide_tiles_bf16(c, rows):
     pick = np.r_[0:300, rows - 300:rows]
     want = O.transition(prep(x[pick], dtype), prep_tree(w, dtype), mask=None)
     assert_parity(to_np(got)[pick], want, dtype, f"transition c={c} rows={rows}")
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp32"])
+@pytest.mark.parametrize("op", ["trimul", "triattn", "transition"])
+def test_wide_very_many_rows(op, dt):
+    """71 million rows of 8 channels, as 65535 equal items: more rows than one
+    launch of the LayerNorms has waves for. Every item's result is the first's,
+    which is the single item's at the kernels' precision (the GEMM tiles may be
+    others)."""
+    batch, n, dtype = 65535, 33, DTYPES[dt]
+    say(f"{op} wide very many rows {dt}")
+    one = torch.from_numpy(syn.pair_input(n, 8, seed=5)).to("cuda", dtype)[None]
+    x = one.expand(batch, -1, -1, -1).contiguous()
+    if op == "trimul":
+        w = P.pack_trimul_torch(P.trimul_to_protenix(syn.trimul_weights(8, 8, seed=3)), dtype, "cuda")
+        call = lambda z: kernels.trimul(z, None, w, "incoming")  # noqa: E731
+    elif op == "triattn":
+        w = P.pack_triattn_protenix(P.triattn_to_protenix(syn.triattn_weights(8, 1, 32, seed=4)), dtype, "cuda")
+        call = lambda z: kernels.triattn(z, None, w, starting=False)  # noqa: E731
+    else:
+        tw = syn.transition_weights(8, 3, seed=23)
+        w = P.pack_transition_torch({k: tw[k] for k in ("layer_norm", "linear_a", "linear_b", "linear_out")}, dtype, "cuda")
+        call = lambda z: kernels.transition(z, w)  # noqa: E731
+    want, got = call(one), call(x)
+    torch.cuda.synchronize()
+    assert torch.equal(got, got[:1].expand_as(got))
+    assert_parity(to_np(got[0]), to_np(want[0]), dtype, "first item")
+    del x, got
+    torch.cuda.empty_cache()
