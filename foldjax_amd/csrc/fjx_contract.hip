@@ -518,9 +518,10 @@ __device__ __forceinline__ void contract_dma_body(const bf16* __restrict__ A, co
     }
 
     // the lane's row and column offsets, opaque here: the store offsets are
-    // then formed after the k-loop instead of being hoisted above it
+    // then formed after the k-loop instead of being hoisted above it (and the
+    // stores stay behind the next tile's DMA, as its wait counts on)
     int lrow = li, lcol = 8 * lg;
-    asm volatile("" : "+v"(lrow), "+v"(lcol));
+    asm volatile("" : "+v"(lrow), "+v"(lcol) : : "memory");
     // this wave's 64 columns start at c0, all of them within the pitch or none
     const int c0 = cur.n0 + wn;
     const int rstride = blocked ? pitch * tile::kC : pitch;  // elements per output row
@@ -694,7 +695,7 @@ __global__ __launch_bounds__(512) void contract_split_kernel(const bf16* __restr
     }
 
     int lrow = li, lcol = 4 * lg;
-    asm volatile("" : "+v"(lrow), "+v"(lcol));
+    asm volatile("" : "+v"(lrow), "+v"(lcol) : : "memory");  // as contract_dma_body
     // transposed accumulators: a lane holds 4 consecutive columns of a row;
     // the wave's 32 columns are all within the pitch or none
     const int c0 = cur.n0 + wn;

@@ -293,9 +293,10 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams<bf16, bf16>& P, c
     }
 
     // lane coordinates, opaque here: the epilogue's offsets are then formed
-    // after the k-loop instead of being hoisted above it
+    // after the k-loop instead of being hoisted above it (and the paired forms'
+    // stores stay behind the next tile's DMA, as its wait counts on)
     int lrow = li, lcol = 8 * lg;
-    asm volatile("" : "+v"(lrow), "+v"(lcol));
+    asm volatile("" : "+v"(lrow), "+v"(lcol) : : "memory");
 
     if constexpr (MODE == kPair) {
       // tiles 0, 1 hold units u0 + lcol .. +7 of a, tiles 2, 3 of b

@@ -83,3 +83,23 @@ def test_no_lds_access_in_flight_at_a_barrier(src):
         assert max(worst) == 0, f"{name}: {worst} LDS or scalar operations in flight at its barriers"
         checked += 1
     assert checked, f"no LDS-DMA kernel found in {src}"
+
+
+def test_a_tiles_stores_follow_the_next_tiles_dma():
+    """A tile's first wait leaves the previous tile's stores in flight, vmcnt(their
+    number): it covers the DMA only if every store was issued after it, none is
+    missing and nothing else was issued since."""
+    checked = set()
+    for src in ("fjx_contract.hip", "fjx_gemm_dma.hip"):
+        for name, code in isa.kernels(src).items():
+            dma = [i for i, c in enumerate(code) if re.match(r"(buffer|global)_load\S*.*\blds\b", c)]
+            waits = [m for m in (re.match(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)", c) for c in code) if m]
+            left = {int(m.group(1)) for m in waits} - {0}
+            if not dma or not left:
+                continue
+            vmem = [i for i, c in enumerate(code) if re.match(r"(buffer|global|scratch|flat)_(load|store|atomic)", c)]
+            after = [i for i in vmem if i > dma[-1]]
+            stores = [i for i in vmem if "_store" in code[i]]
+            assert left == {len(stores)} and after == stores, (name, left, len(stores), len(after))
+            checked.add(re.search(r"contract_dma|contract_split|gemm_dma_pair|gemm_dma_planes", name).group())
+    assert len(checked) == 4, checked
