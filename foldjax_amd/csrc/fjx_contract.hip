@@ -759,6 +759,21 @@ void launch_gemm(const GemmParams<T, TO>& p, hipStream_t st) {
     if (launch_gemm_dma(p, st)) return;
   }
   auto tiles = [&](int64_t bm) { return p.batches * ((p.m + bm - 1) / bm) * ((p.n + bm - 1) / bm); };
+  // a contraction of more tiles than one launch takes blocks for (for_pieces):
+  // some batches at a time
+  constexpr int64_t kMax = (int64_t)1 << 23;
+  if (p.batches > 1 && tiles(128) > kMax && !p.gate && !p.residual && !p.row_gate) {
+    const int64_t some = std::max<int64_t>(1, kMax / (tiles(128) / p.batches));
+    GemmParams<T, TO> q = p;
+    for (int64_t b0 = 0; b0 < p.batches; b0 += some) {
+      q.a = p.a + b0 * p.sa;
+      q.b = p.b + b0 * p.sb;
+      q.c = p.c + b0 * p.sc;
+      q.batches = std::min(some, p.batches - b0);
+      launch_gemm<T, TO>(q, st);
+    }
+    return;
+  }
   // 128-wide tiles unless they would leave most of the 256 CUs idle. fp32
   // problems of fewer than four 64-wide tiles per CU (the single track's
   // projections: 384 tiles at 1024 tokens, so half the SIMDs would run two

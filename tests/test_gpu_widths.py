@@ -408,3 +408,18 @@ def test_wide_very_many_rows(op, dt):
     assert_parity(to_np(got[0]), to_np(want[0]), dtype, "first item")
     del x, got
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("n,c_h", [(1, 264), (9, 136)])
+def test_trimul_wide_fp32_very_many_products(n, c_h):
+    """65535 equal items: 17 million (9 million) n x n contractions, more than one
+    launch of the float32 GEMM has blocks for."""
+    batch, dtype = 65535, DTYPES["fp32"]
+    say(f"trimul wide fp32 very many products n={n} c_h={c_h}")
+    w = P.pack_trimul_torch(P.trimul_to_protenix(syn.trimul_weights(8, c_h, seed=3)), dtype, "cuda")
+    one = torch.from_numpy(syn.pair_input(n, 8, seed=5)).to("cuda", dtype)[None]
+    x = one.expand(batch, -1, -1, -1).contiguous()
+    want, got = kernels.trimul(one, None, w, "outgoing"), kernels.trimul(x, None, w, "outgoing")
+    torch.cuda.synchronize()
+    assert torch.equal(got, got[:1].expand_as(got))
+    assert_parity(to_np(got[0]), to_np(want[0]), dtype, "first item")
