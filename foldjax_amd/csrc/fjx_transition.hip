@@ -386,6 +386,23 @@ static void launch_transition_rt(const TransitionParams<T>& p, int c, hipStream_
 
 template <typename T>
 void launch_transition(const TransitionParams<T>& p, int c, hipStream_t st) {
+  // four threads a row: past 2^30 rows (of 96 channels or fewer: more memory than
+  // there is otherwise) one launch's block count would wrap, with no error
+  constexpr int64_t kMost = (int64_t)1 << 29;
+  if (p.rows > kMost && !p.pb_out && !p.pbf_out) {
+    TransitionParams<T> q = p;
+    auto from = [](auto* ptr, int64_t off) { return ptr ? ptr + off : nullptr; };
+    for (int64_t r0 = 0; r0 < p.rows; r0 += kMost) {
+      q.x = p.x + r0 * c;
+      q.out = p.out + r0 * c;
+      q.residual = from(p.residual, r0 * c);
+      q.row_mask = from(p.row_mask, r0);
+      q.out_mask = from(p.out_mask, r0);
+      q.rows = p.rows - r0 < kMost ? p.rows - r0 : kMost;
+      launch_transition<T>(q, c, st);
+    }
+    return;
+  }
   if constexpr (std::is_same<T, bf16>::value) {
     // 64- and 32-row tiles while they still go one (the narrow forms: two) to a
     // CU: the tile is a serial walk over the hidden chunks, shorter with fewer

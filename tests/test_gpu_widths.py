@@ -423,3 +423,21 @@ def test_trimul_wide_fp32_very_many_products(n, c_h):
     torch.cuda.synchronize()
     assert torch.equal(got, got[:1].expand_as(got))
     assert_parity(to_np(got[0]), to_np(want[0]), dtype, "first item")
+
+
+def test_transition_narrow_very_many_rows():
+    """A thousand million rows of 32 channels, in place (71 GB): more than one
+    launch has threads for."""
+    part, parts, c, dtype = 1 << 20, 1030, 32, DTYPES["bf16"]
+    torch.cuda.empty_cache()
+    say(f"transition narrow rows={part * parts}")
+    w = P.pack_transition_torch(P.transition_to_protenix(syn.transition_weights(c, seed=23)), dtype, "cuda")
+    one = torch.randn(part, c, device="cuda").to(dtype)
+    mask = (torch.rand(part, device="cuda") > 0.5).to(dtype)
+    want = kernels.transition(one, w, row_mask=mask, residual=one)
+    x = one.expand(parts, -1, -1).contiguous()
+    kernels.transition(x, w, row_mask=mask.expand(parts, -1).contiguous(), residual=x, out=x)
+    torch.cuda.synchronize()
+    assert all(torch.equal(x[k], want) for k in range(parts))
+    del x
+    torch.cuda.empty_cache()
